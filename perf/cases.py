@@ -18,8 +18,8 @@ A case is one of six kinds of call:
 Sizes are those of the benchmark, the tests and the instance files in
 tests/golden, and odd ones between them.  Inputs come from the library's own
 seeded generators, as in its benchmark: uniform coordinates in [0, 1000]^2 or
-20 Gaussian clusters in [0, 2000]^2, random permutations, and tours of the
-randomized construction.
+20 Gaussian clusters in [0, 2000]^2, random permutations and tours of the
+randomized construction; and tours along strips of the plane.
 """
 import ctypes
 import math
@@ -58,7 +58,7 @@ def listed():
         {"name": "static_n1000_odc", "kind": "static", "n": 1000, "rowmap": ODC, "tour": "perm"},
         # a long random tour: 2-opt deltas beyond 32 bits
         {"name": "static_n3001", "kind": "static", "n": 3001, "rowmap": ADS, "tour": "perm"},
-        # eight long, nearly greedy tours in one launch (a search in its later stages)
+        # eight long tours of short edges in one launch (a search in its later stages)
         {"name": "evals_8x4001", "kind": "evals", "n": 4001, "count": 8, "rowmap": ADS, "tour": "near"},
         # one round over a population of start tours
         {"name": "round_256x784", "kind": "round", "n": 784, "count": 256, "rounds": 1, "rowmap": ADS},
@@ -130,7 +130,15 @@ def _coords(n, seed, clustered):
 def _tour(how, xs, ys, seed):
     if how == "perm":
         return inputs.perm_tour(seed, len(xs))
-    return inputs.random_tour_fast(xs, ys, 1, seed, 0.02)  # among the nearest 2% of the clients left
+    # up and down strips of the plane, of random width and slightly shuffled:
+    # edges about as short as after a constructive heuristic
+    n = len(xs)
+    rng = np.random.RandomState(seed % 2**31)
+    width = math.sqrt(3e6 / n) * rng.uniform(0.8, 1.25)
+    strip = (xs / width).astype(np.int64)
+    y = ys + rng.normal(0.0, 0.2 * width, n)
+    order = np.lexsort((np.where(strip % 2 == 0, y, -y), strip))
+    return np.concatenate([[0], order[order != 0], [0]]).astype(np.int32)
 
 
 def _jobs(case, seed):
