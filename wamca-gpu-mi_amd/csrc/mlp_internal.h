@@ -33,14 +33,25 @@ enum {
   MLP_INFO_KEPT0 = 8,     // kept-move count of nb (8 + nb)
   MLP_INFO_MG_APPLY = 23, // moves the last many-workgroup merge applied (its rebuild runs if > 0)
   MLP_INFO_PARITY0 = 24,  // row buffer (0/1) holding the last eval of nb (24 + nb)
+  MLP_INFO_PARTIAL = 39,  // 1: the last DVND round kept only improving rows (k_psweep)
   MLP_INFO_WORDS = 40
 };
 
 // info[PATH32] bits: 2-opt / swap and or-opt deltas fit int32; swap and
 // or-opt deltas below 2^26 (keys packed with a 5-bit column iteration);
 // T[N-1] below 2^24 (products of a position and a prefix time are exact in
-// 24-bit multiplies)
-enum { MLP_P32_2OPT = 1, MLP_P32_SWAP_OROPT = 2, MLP_PK_SWAP_OROPT = 4, MLP_T24 = 8 };
+// 24-bit multiplies); 2-opt lower bounds of column blocks fit int32 (the
+// deltas' bound plus the bounds' own slack of 16 T[N-1])
+enum { MLP_P32_2OPT = 1, MLP_P32_SWAP_OROPT = 2, MLP_PK_SWAP_OROPT = 4, MLP_T24 = 8, MLP_LB32_2OPT = 16 };
+
+// Summary of a block of 16 positions [16 b, 16 b + 15], kept during a DVND run
+// whose rounds are pruned: the corners of the bounding box of positions
+// [16 b - 1, 16 b + 16] (packed x << 16 | y), the largest w[p] and the largest
+// w[p] + w[p + 1] of its positions.
+#define MLP_BLK 16
+struct BlkSum {
+  int32_t lo, hi, wmax, wpair;
+};
 
 struct SlotDev {
   int32_t N;      // positions (n + 1)
@@ -59,6 +70,7 @@ struct SlotDev {
   int32_t* h32;   // [N] 2-opt j-side constant Z[p] - (N-p-1) w[p+1]  (mod 2^32)
   int64_t* t64;   // [N]
   int64_t* q64;   // [N]
+  BlkSum* blk;    // [ceil(N / MLP_BLK)]
   int64_t* info;  // [MLP_INFO_WORDS]
   // per-row best keys (delta << 20 | ctx), two buffers of rowcap entries.
   // info[PARITY0 + nb] = p names the buffer holding the last result; the
@@ -170,5 +182,14 @@ struct SlotInitRows {
 struct SlotListInline {
   int32_t id[MLP_SLOTS_INLINE];
 };
+
+// mlp_dvnd_rounds for a caller that never reads rows (the server): rows that
+// do not improve are left out in every round.
+struct mlp_ctx;
+#ifdef __cplusplus
+extern "C"
+#endif
+int mlp_dvnd_rounds_improving(struct mlp_ctx* ctx, const int32_t* slots, int32_t count,
+                              int32_t rowmap, int32_t rounds, int32_t max_rounds);
 
 #endif  // MLP_INTERNAL_H_

@@ -27,6 +27,7 @@
 // square root (mlproblem.cpp:159-162).
 #include <hip/hip_runtime.h>
 
+#include <limits>
 #include <type_traits>
 
 #include "mlp_gpu.h"
@@ -368,6 +369,11 @@ __device__ __forceinline__ int64_t dpp64(int64_t v) {
   return (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
 
+// The value of lane ^ 1 (DPP quad permutation 1, 0, 3, 2).
+__device__ __forceinline__ int swap_pair(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);
+}
+
 // Inclusive wave scan (Hillis-Steele over rows of 16 lanes: shifts 1, 2, 4,
 // 8; then row 0's total into row 1 and row 2's into row 3, then rows 0-1's
 // total into rows 2 and 3), in registers.
@@ -389,6 +395,34 @@ __device__ __forceinline__ int64_t wave_sum64(int64_t v) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
+// The summaries of 16-position blocks from threads holding eight positions
+// each (p0 on: packed coordinates of p0 - 1 .. p0 + 8 and w of p0 .. p0 + 8),
+// joined between neighbouring threads.  Positions clamped into the tour lie
+// inside the last block's range.
+__device__ __forceinline__ void put_summary(const SlotDev& s, int p0, const int (&xy)[kPrepPer + 2],
+                                            const int (&w)[kPrepPer + 1]) {
+  short2v lo = __builtin_bit_cast(short2v, xy[0]), hi = lo;
+  int wm = 0, wp = 0;
+#pragma unroll
+  for (int e = 1; e < kPrepPer + 2; ++e) {
+    const short2v c = __builtin_bit_cast(short2v, xy[e]);
+    lo = __builtin_elementwise_min(lo, c);
+    hi = __builtin_elementwise_max(hi, c);
+  }
+#pragma unroll
+  for (int e = 0; e < kPrepPer; ++e) {
+    wm = max(wm, w[e]);
+    wp = max(wp, w[e] + w[e + 1]);
+  }
+  lo = __builtin_elementwise_min(lo, __builtin_bit_cast(short2v, swap_pair(__builtin_bit_cast(int, lo))));
+  hi = __builtin_elementwise_max(hi, __builtin_bit_cast(short2v, swap_pair(__builtin_bit_cast(int, hi))));
+  wm = max(wm, swap_pair(wm));
+  wp = max(wp, swap_pair(wp));
+  if ((threadIdx.x & 1) == 0 && p0 < s.N)
+    *(int4*)(s.blk + p0 / MLP_BLK) =
+        make_int4(__builtin_bit_cast(int, lo), __builtin_bit_cast(int, hi), wm, wp);
+}
+
 struct PrepLds {
   int64_t wt[kBlock / kWave][2];
   int64_t carry[2];  // T, Q before this segment
@@ -407,7 +441,8 @@ struct PrepLds {
 template <bool WRITE>
 __device__ __forceinline__ void prep_segment(const SlotDev& s, const int32_t* tour, const int32_t* xyc,
                                              int base, int64_t carryT, int64_t carryQ, PrepLds& P,
-                                             int64_t& segT, int64_t& segQ, int64_t& lacc) {
+                                             int64_t& segT, int64_t& segQ, int64_t& lacc,
+                                             bool sum = false) {
   const int N = s.N, tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const float dr = round_dr(s.round);
   const int p0 = base + tid * kPrepPer;
@@ -429,6 +464,7 @@ __device__ __forceinline__ void prep_segment(const SlotDev& s, const int32_t* to
     const int p = p0 + e;
     w[e] = (p >= 1 && p < N) ? dist_xy(xy[e], xy[e + 1], dr) : 0;
   }
+  if (WRITE && sum) put_summary(s, p0, xy, w);
   int64_t lt[kPrepPer], lq[kPrepPer], at = 0, aq = 0;
 #pragma unroll
   for (int e = 0; e < kPrepPer; ++e) {
@@ -528,14 +564,15 @@ __device__ __forceinline__ void prep_flags(const SlotDev& s, int64_t Ttot) {
   s.info[MLP_INFO_PATH32] = (b2 < 2147483647LL ? MLP_P32_2OPT : 0) |
                             (bso < 2147483647LL ? MLP_P32_SWAP_OROPT : 0) |
                             (bso < (1LL << 26) ? MLP_PK_SWAP_OROPT : 0) |
-                            (Ttot < (1LL << 24) ? MLP_T24 : 0);
+                            (Ttot < (1LL << 24) ? MLP_T24 : 0) |
+                            (b2 + 16 * Ttot < 2147483647LL ? MLP_LB32_2OPT : 0);
 }
 
 // The whole tour's prefix arrays and info words by one workgroup (inlined,
 // so that the tour and coordinate arrays keep their address space: LDS in a
 // merge, global memory in k_prep).
 __device__ __forceinline__ void prep_wg(const SlotDev& s, const int32_t* tour, PrepLds& P,
-                                        const int32_t* xyc = nullptr) {
+                                        const int32_t* xyc = nullptr, bool sum = false) {
   const int N = s.N, tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   int64_t lacc = 0;  // this thread's share of L = sum_p T[p]
   if (tid == 0) {
@@ -546,7 +583,7 @@ __device__ __forceinline__ void prep_wg(const SlotDev& s, const int32_t* tour, P
   for (int base = 0; base < N; base += kBlock * kPrepPer) {
     const int64_t cT = P.carry[0], cQ = P.carry[1];
     int64_t segT, segQ;
-    prep_segment<true>(s, tour, xyc, base, cT, cQ, P, segT, segQ, lacc);
+    prep_segment<true>(s, tour, xyc, base, cT, cQ, P, segT, segQ, lacc, sum);
     if (tid == 0) {
       P.carry[0] = cT + segT;
       P.carry[1] = cQ + segQ;
@@ -585,16 +622,28 @@ __global__ __launch_bounds__(kBlock) void k_prep(const SlotDev* __restrict__ tab
   }
 }
 
-// Start of a DVND run: every listed slot becomes active with no rounds.
+// Start of a DVND run: every listed slot becomes active with no rounds; the
+// summaries of its position blocks are written (the run's merges keep them up
+// to date, other rebuilds of a tour leave them).
 __global__ __launch_bounds__(kBlock) void k_dvnd_start(const SlotDev* __restrict__ table,
                                                        SlotListInline list,
-                                                       const int32_t* list_dev, int count) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < count) {
-    const SlotDev& s = table[list_at(list, list_dev, t)];
+                                                       const int32_t* list_dev) {
+  const SlotDev& s = table[list_at(list, list_dev, blockIdx.x)];
+  const int N = s.N;
+  if (threadIdx.x == 0) {
     s.info[MLP_INFO_ACTIVE] = 1;
     s.info[MLP_INFO_ROUNDS] = 0;
     s.info[MLP_INFO_ROUND_MOVES] = 0;
+    s.info[MLP_INFO_PARTIAL] = 0;
+  }
+  for (int base = 0; base < N; base += kBlock * kPrepPer) {
+    const int p0 = base + (int)threadIdx.x * kPrepPer;
+    int xy[kPrepPer + 2], w[kPrepPer + 1];
+#pragma unroll
+    for (int e = 0; e < kPrepPer + 2; ++e) xy[e] = ldg(s.xy + min(max(p0 - 1 + e, 0), N - 1));
+#pragma unroll
+    for (int e = 0; e <= kPrepPer; ++e) w[e] = p0 + e < N ? ldg(s.w + p0 + e) : 0;
+    put_summary(s, p0, xy, w);
   }
 }
 
@@ -1225,7 +1274,7 @@ __device__ __forceinline__ void merge_slot(const SlotDev& s, int nb, int rowmap,
   const int K = sort_greedy<false>(s, nb, rowmap, N, M, keys, lds, ctxL, bits, S, sk);
   // 4. apply the kept moves, rebuild the prefix arrays
   apply_kept(s, nb, K, [&](int q) { return sk[q]; }, told, tnew, S.lng, S.longq, true);
-  prep_wg(s, tnew, S.PL, xyc);
+  prep_wg(s, tnew, S.PL, xyc, (skip_inactive & 2) != 0);
   if (tid == 0) {
     s.info[MLP_INFO_KEPT0 + nb] = K;
     s.info[MLP_INFO_ROUND_MOVES] += K;
@@ -1384,7 +1433,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_sums(const SlotDev* __restrict__ 
 
 __global__ __launch_bounds__(kBlock) void k_mg_rebuild(const SlotDev* __restrict__ table,
                                                        SlotListInline list,
-                                                       const int32_t* list_dev) {
+                                                       const int32_t* list_dev, int sum) {
   __shared__ PrepLds P;
   const SlotDev& s = table[list_at(list, list_dev, blockIdx.y)];
   if (s.info[MLP_INFO_MG_APPLY] == 0) return;
@@ -1403,7 +1452,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_rebuild(const SlotDev* __restrict
     Ttot += t;
   }
   int64_t segT, segQ, lacc = 0;
-  prep_segment<true>(s, a.tnew, a.xyc, base, cT, cQ, P, segT, segQ, lacc);
+  prep_segment<true>(s, a.tnew, a.xyc, base, cT, cQ, P, segT, segQ, lacc, sum != 0);
   for (int p = base + tid; p < min(base + MLP_MG_CHUNK, N); p += kBlock) s.tour[p] = a.tnew[p];
   const int64_t lw = wave_sum64(lacc);
   if (lane == 0) P.lsum[wave] = lw;
@@ -2087,6 +2136,10 @@ __device__ __forceinline__ void reset_other(const SlotDev& s, int nb, int par, i
   }
 }
 
+// Bit of a tile's parity word: it folds into buffers that already hold moves
+// of the same tour and resets nothing.
+constexpr int kNoReset = 1 << 30;
+
 // Value barrier: the compiler sees an opaque value, so a per-column term
 // stays one shared value instead of being distributed into every row's
 // products (which turns two 24-bit multiplies into one quarter-rate 32-bit
@@ -2477,7 +2530,7 @@ __device__ __forceinline__ void sweep_fixed_wide(const SlotDev& s, int rb, int c
   if (ct != 0) return;
 #pragma unroll
   for (int nb = 0; nb < MLP_NB_COUNT; ++nb)
-    if (nb != 1 && ((mask >> nb) & 1))
+    if (nb != 1 && ((mask >> nb) & 1) && !(parity & kNoReset))
       reset_other(s, nb, (parity >> nb) & 1, b0, min(b0 + R, rows_of(nb, RM, N)), rb == 0, RM);
   for (int sg = wave; sg < 4 * R; sg += kBlock / kWave) {
     const int g = sg / R, by = b0 + sg % R;
@@ -2500,7 +2553,7 @@ __device__ __forceinline__ void two_rows_wide(const SlotDev& s, int rb, int ct, 
   const int N = s.N, wave = wave_id(), lane = threadIdx.x % kWave;
   const int rows2 = (N + 1) >> 1, b0 = rb * R;
   const int par = (parity >> 1) & 1;
-  reset_other(s, 1, par, b0, min(b0 + R, rows2), rb == 0);
+  if (!(parity & kNoReset)) reset_other(s, 1, par, b0, min(b0 + R, rows2), rb == 0);
   for (int by = b0 + wave; by < min(b0 + R, rows2); by += kBlock / kWave) {
     if (p32) eval_row<1, true>(s, 1, 0, by, lane, row_buf(s, 1, par) + by);
     else eval_row<1, false>(s, 1, 0, by, lane, row_buf(s, 1, par) + by);
@@ -2559,7 +2612,7 @@ __device__ __forceinline__ void sweep_fixed(const SlotDev& s, int rb, int ct, in
     sweep_fixed_wide<R, RM>(s, rb, ct, mask, parity);
     return;
   }
-  if (ct == 0) {
+  if (ct == 0 && !(parity & kNoReset)) {
 #pragma unroll
     for (int nb = 0; nb < MLP_NB_COUNT; ++nb)
       if (nb != 1 && ((mask >> nb) & 1))
@@ -2684,7 +2737,8 @@ __device__ __forceinline__ void sweep_2opt_wide(const SlotDev& s, int rb, int ct
   const int rows = (s.N + 1) >> 1;
   const int par = (parity >> 1) & 1;
   if (ct != 0) return;
-  reset_other(s, 1, par, rb * MLP_2OPT_ROWS, min(rb * MLP_2OPT_ROWS + MLP_2OPT_ROWS, rows), rb == 0);
+  if (!(parity & kNoReset))
+    reset_other(s, 1, par, rb * MLP_2OPT_ROWS, min(rb * MLP_2OPT_ROWS + MLP_2OPT_ROWS, rows), rb == 0);
   const int by = rb * MLP_2OPT_ROWS + wave;
   if (by < rows) eval_row<1, false>(s, 1, 0, by, lane, row_buf(s, 1, par) + by);
 }
@@ -2761,7 +2815,7 @@ __device__ __forceinline__ void sweep_2opt(const SlotDev& s, int rb, int ct, int
     sweep_2opt_wide(s, rb, ct, parity);
     return;
   }
-  if (ct == 0)
+  if (ct == 0 && !(parity & kNoReset))
     reset_other(s, 1, par, rb * MLP_2OPT_ROWS, min(rb * MLP_2OPT_ROWS + MLP_2OPT_ROWS, rows), rb == 0);
   if constexpr (FLAT) {
     if (net > 0) {
@@ -2957,18 +3011,23 @@ __device__ __forceinline__ SweepSeg find_sweep_dev(const SweepSeg* segs, int nse
 
 template <int R, int C, int X>
 __device__ __forceinline__ void sweep_item(const SlotDev* __restrict__ table, const SweepSeg& sg, int item,
-                           SweepLds<R, C, X>& L, bool dvnd, bool filtered) {
+                           SweepLds<R, C, X>& L, bool dvnd, bool filtered, bool fill = false) {
   const SlotDev& s = table[sg.slot];
-  if (dvnd && s.info[MLP_INFO_ACTIVE] == 0) return;
+  // fill: the rows of a finished DVND run whose last round kept only the
+  // improving ones, completed in place (the tour is the one they were
+  // evaluated on: that round applied no move)
+  if (fill ? s.info[MLP_INFO_PARTIAL] == 0 : dvnd && s.info[MLP_INFO_ACTIVE] == 0) return;
   // bit nb of par: the buffer this sweep writes (the one not holding the last result)
   int par = sg.parity;
   if (dvnd) {
     par = 0;
 #pragma unroll
     for (int nb = 0; nb < MLP_NB_COUNT; ++nb)
-      if ((sg.mask >> nb) & 1) par |= (1 - (int)(s.info[MLP_INFO_PARITY0 + nb] & 1)) << nb;
+      if ((sg.mask >> nb) & 1) par |= (int)((s.info[MLP_INFO_PARITY0 + nb] & 1) ^ (fill ? 0 : 1)) << nb;
+    if (fill) par |= kNoReset;
   }
   const int b = item - sg.blk0;
+  if (dvnd && !fill && b == 0 && threadIdx.x == 0) s.info[MLP_INFO_PARTIAL] = 0;
   const int rb = b / sg.ncols, ct = b % sg.ncols;
   if (!dvnd && b == 0 && threadIdx.x == 0) {
 #pragma unroll
@@ -2995,14 +3054,15 @@ __global__ __launch_bounds__(kBlock, (R * C <= 2048 ? 7 : 1)) void k_sweep(
   // flags bit 0: a DVND launch (inactive slots skipped, parities read from
   // info); bit 1: filtered folds of the diagonal rows (many more tiles than
   // resident workgroups, so most tiles fold after others of their tour);
-  // bits 2, 8..31: equal segments per slot (find_sweep_dev)
+  // bits 2, 8..31: equal segments per slot (find_sweep_dev); bit 3: rows that
+  // a finished DVND run left incomplete (with bit 0)
   __shared__ SweepLds<R, C, X> L;
-  const bool dvnd = (flags & 1) != 0, filtered = (flags & 2) != 0;
+  const bool dvnd = (flags & 1) != 0, filtered = (flags & 2) != 0, fill = (flags & 8) != 0;
   if (!counter) {
     const int item = blockIdx.x;
     const SweepSeg sg = segs_dev ? find_sweep_dev(segs_dev, nsegs, item, flags)
                                   : find_sweep_inline(inl, nsegs, item);
-    sweep_item<R, C, X>(table, sg, item, L, dvnd, filtered);
+    sweep_item<R, C, X>(table, sg, item, L, dvnd, filtered, fill);
     return;
   }
   __shared__ int s_item;
@@ -3014,10 +3074,12 @@ __global__ __launch_bounds__(kBlock, (R * C <= 2048 ? 7 : 1)) void k_sweep(
     if (item >= total) break;
     const SweepSeg sg = segs_dev ? find_sweep_dev(segs_dev, nsegs, item, flags)
                                   : find_sweep_inline(inl, nsegs, item);
-    sweep_item<R, C, X>(table, sg, item, L, dvnd, filtered);
+    sweep_item<R, C, X>(table, sg, item, L, dvnd, filtered, fill);
     __syncthreads();
   }
 }
+
+#include "mlp_prune.h"
 
 // ---------------------------------------------------------------------------
 // DVND rounds as one persistent launch (FusedPlan): each workgroup takes the
@@ -3182,8 +3244,7 @@ hipError_t mlp_launch_prep(hipStream_t st, const SlotDev* table, const SlotListI
 
 hipError_t mlp_launch_dvnd_start(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
                                  const int32_t* list_dev, int count) {
-  hipLaunchKernelGGL(k_dvnd_start, dim3((count + kBlock - 1) / kBlock), dim3(kBlock), 0, st,
-                     table, inl, list_dev, count);
+  hipLaunchKernelGGL(k_dvnd_start, dim3(count), dim3(kBlock), 0, st, table, inl, list_dev);
   return hipGetLastError();
 }
 
@@ -3245,6 +3306,27 @@ hipError_t mlp_launch_sweep(hipStream_t st, int tile, const SlotDev* table,
       else if (odc) MLP_SWEEP_LAUNCH(8, 512, kOdc);
       else MLP_SWEEP_LAUNCH(16, 1024, kPlain);
       break;
+  }
+  return hipGetLastError();
+}
+
+int mlp_prune_rows() { return kPWg; }
+// A row near the start that can save much survives against most columns, so
+// a wave's columns bound its time: or-opt, whose columns lie on both sides,
+// gets fewer (n = 9001, or-opt-3 in the late rounds: 75 us at 4096 columns)
+int mlp_prune_max_w(int nb) { return nb >= 2 ? kPMaxW / 2 : kPMaxW; }
+
+hipError_t mlp_launch_psweep(hipStream_t st, const SlotDev* table, const SweepSegsInline& inl,
+                             const SweepSeg* segs_dev, int nsegs, int total, int nb, int W) {
+#define MLP_PSWEEP(NB, LDS)                                                                   \
+  hipLaunchKernelGGL(k_psweep<NB>, dim3(total), dim3(kBlock), LDS, st, table, inl, segs_dev, \
+                     nsegs, W)
+  switch (nb) {
+    case 0: MLP_PSWEEP(0, 0); break;
+    case 1: MLP_PSWEEP(1, sizeof(int64_t) * (size_t)(4 + W + kPWg)); break;
+    case 2: MLP_PSWEEP(2, 0); break;
+    case 3: MLP_PSWEEP(3, 0); break;
+    default: MLP_PSWEEP(4, 0); break;
   }
   return hipGetLastError();
 }
@@ -3321,7 +3403,8 @@ hipError_t mlp_launch_merge_gmem(hipStream_t st, const SlotDev* table, const Slo
   hipLaunchKernelGGL(k_mg_select, dim3(count), dim3(kBlock), kGmemMergeLds, st, table, inl,
                      list_dev, nb, rowmap, skip_inactive, tail);
   hipLaunchKernelGGL(k_mg_sums, seg, dim3(kBlock), 0, st, table, inl, list_dev);
-  hipLaunchKernelGGL(k_mg_rebuild, seg, dim3(kBlock), 0, st, table, inl, list_dev);
+  hipLaunchKernelGGL(k_mg_rebuild, seg, dim3(kBlock), 0, st, table, inl, list_dev,
+                     skip_inactive & 2);
   return hipGetLastError();
 }
 

@@ -23,10 +23,18 @@ hipError_t mlp_launch_eval(hipStream_t st, const SlotDev* table, const EvalSegsI
 // flags bit 0: DVND launch (inactive slots skipped); bit 1: filtered folds
 // of the diagonal rows (launches with many more tiles than resident
 // workgroups); bits 8..31 (with bit 2: two segments per slot): the items per
-// slot when every slot of a device segment list has the same segments
+// slot when every slot of a device segment list has the same segments; bit 3
+// (with bit 0): complete the rows a finished DVND run left partial
 hipError_t mlp_launch_sweep(hipStream_t st, int tile, const SlotDev* table,
                             const SweepSegsInline& inl, const SweepSeg* segs_dev, int nsegs,
                             int total, int* counter, int grid, int flags);
+// A DVND round's evaluation of one neighborhood (ids 0..4, ADS row map): only
+// improving moves (mlp_prune.h).  Items of W columns (a multiple of 64, at
+// most mlp_prune_max_w(nb)) x mlp_prune_rows() rows.
+hipError_t mlp_launch_psweep(hipStream_t st, const SlotDev* table, const SweepSegsInline& inl,
+                             const SweepSeg* segs_dev, int nsegs, int total, int nb, int W);
+int mlp_prune_rows();
+int mlp_prune_max_w(int nb);
 void mlp_tile_shape(int tile, int* rows, int* cols);
 size_t mlp_merge_lds_bytes(int pcap, int ncap);
 hipError_t mlp_merge_setup(size_t max_dyn_lds);

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -107,7 +108,7 @@ size_t merge_gmem_bytes(int N) {
 
 // Byte layout of one slot's device block.
 struct SlotLayout {
-  size_t tour, xy, w, t32, q32, g32, h32, t64, q64, info, rows[MLP_NB_MAX], kc[MLP_NB_MAX],
+  size_t tour, xy, w, t32, q32, g32, h32, t64, q64, blk, info, rows[MLP_NB_MAX], kc[MLP_NB_MAX],
       kij[MLP_NB_MAX], ms, total;
 };
 
@@ -128,6 +129,7 @@ SlotLayout slot_layout(int N, int nbs) {
   L.h32 = take(4 * (size_t)N);
   L.t64 = take(8 * (size_t)N);
   L.q64 = take(8 * (size_t)N);
+  L.blk = take(sizeof(BlkSum) * (size_t)((N + MLP_BLK - 1) / MLP_BLK));
   L.info = take(8 * MLP_INFO_WORDS);
   for (int nb = 0; nb < nbs; ++nb) {
     const size_t r = (size_t)row_cap(N);
@@ -803,6 +805,7 @@ int mlp_slot_create(mlp_ctx* ctx, int32_t inst, int32_t* slot) {
   d.h32 = (int32_t*)(b + L.h32);
   d.t64 = (int64_t*)(b + L.t64);
   d.q64 = (int64_t*)(b + L.q64);
+  d.blk = (BlkSum*)(b + L.blk);
   d.info = (int64_t*)(b + L.info);
   d.nbs = ctx->nbs;
   for (int nb = 0; nb < d.nbs; ++nb) {
@@ -1031,6 +1034,10 @@ int auto_tile_moves(const mlp_ctx* ctx, int64_t moves, int count, uint32_t mask)
 int auto_tile(const mlp_ctx* ctx, const int32_t* slots, int count, uint32_t mask) {
   return auto_tile_moves(ctx, launch_moves(ctx, slots, count, mask), count, mask);
 }
+
+// Waves of a pruned evaluation's launch (prune_impl).
+constexpr int64_t kPruneWaves = 2048;
+constexpr int kPruneMinN = 256;
 
 // Forget the cached DVND chunk graph (its launches embed the neighborhood
 // set, tile choices and merge mode of the moment it was captured).
@@ -1580,8 +1587,8 @@ int mlp_get_moves64(mlp_ctx* ctx, int32_t slot, int32_t nb, uint64_t* moves, int
   return MLP_OK;
 }
 
-// tail > 0: the last merge of a DVND round, which also ends the round
-// (max_rounds = tail - 1).
+// skip: inside a DVND round (bit 1: block summaries are kept).  tail > 0: the
+// last merge of a DVND round, which also ends the round (max_rounds = tail - 1).
 static int merge_impl(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t nb, int skip,
                       int tail = 0) {
   if (count == 0) return MLP_OK;
@@ -1801,10 +1808,66 @@ int mlp_merge_total(mlp_ctx* ctx, const int32_t* slots, int32_t count) {
 
 namespace {
 
+// The pruned evaluation of a DVND round applies: ADS row map and the context's
+// own tile choice, one launch per neighborhood, a tour of kPruneMinN positions
+// among the slots (below that every block survives and the launch is as long
+// as its latency: n = 100, 5.3 us a neighborhood against 4.6 tiled).
+bool prune_ok(const mlp_ctx* ctx, const int32_t* slots, int count, int rowmap) {
+  if (rowmap != 0 || ctx->tile_override >= 0 || ctx->dvnd_persistent || ctx->dvnd_fused) return false;
+  int maxn = 0;
+  for (int q = 0; q < count; ++q) maxn = std::max(maxn, ctx->slots[slots[q]].N);
+  return maxn >= kPruneMinN;
+}
+
+// One pruned evaluation of nb (0..4) over the slots inside a DVND round.
+int prune_impl(mlp_ctx* ctx, const int32_t* slots, int count, int nb) {
+  const int R = mlp_prune_rows();
+  // columns of a wave: 128 in a launch of at most kPruneWaves waves (spread
+  // over the GPU), more in a longer one (the rows' set-up serves more
+  // blocks), up to mlp_prune_max_w(nb)
+  int W = 128;
+  for (; W < mlp_prune_max_w(nb); W *= 2) {
+    int64_t total = 0;
+    for (int q = 0; q < count; ++q) {
+      const int N = ctx->slots[slots[q]].N;
+      total += (int64_t)((N + 7) / 8) * ((N + W - 1) / W);
+    }
+    if (total <= kPruneWaves) break;
+  }
+  std::vector<SweepSeg> segs((size_t)count);
+  int total = 0;
+  for (int q = 0; q < count; ++q) {
+    Slot& s = ctx->slots[slots[q]];
+    s.parity_stale = true;
+    s.eval_rowmap[nb] = 0;
+    s.merged[nb] = false;
+    // 2-opt rows i = 1 .. N-3
+    const int rows = nb == 1 ? s.N - 3 : rows_of(nb, 0, s.N);
+    const int ncols = (s.N + W - 1) / W;
+    segs[(size_t)q] = SweepSeg{slots[q], 0, 1 << nb, total, ncols, 0};
+    if (rows > 0) total += (rows + R - 1) / R * ncols;
+  }
+  if (total == 0) return MLP_OK;
+  SweepSegsInline inl{};
+  const SweepSeg* dev = nullptr;
+  if (count <= MLP_SEGS_INLINE) {
+    for (int q = 0; q < count; ++q) inl.s[q] = segs[(size_t)q];
+  } else {
+    const int st = device_list(ctx, (const int32_t*)segs.data(), count * MLP_SWEEPSEG_INTS,
+                               (const int32_t**)&dev);
+    if (st) return st;
+  }
+  HCK(mlp_launch_psweep(ctx->stream, ctx->d_table, inl, dev, count, total, nb, W));
+  return MLP_OK;
+}
+
 // One DVND round over `slots`: round begin, {eval, merge + apply} for each
 // neighborhood in order, round end.  Slots that stopped are skipped by every
 // kernel, so the same launches serve all rounds of a chunk.
-int enqueue_round(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max_rounds) {
+// prune: its evaluations may leave out rows that do not improve; keep: its
+// merges keep the block summaries that a pruned round reads.
+int enqueue_round(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max_rounds,
+                  bool prune, bool keep) {
   SlotListInline inl;
   const int32_t* dev = nullptr;
   int st = slot_list(ctx, slots, count, inl, &dev);
@@ -1823,11 +1886,13 @@ int enqueue_round(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int
     for (int q = 0; q < count && !any; ++q)
       if (rows_of(nb, rowmap, ctx->slots[slots[q]].N) > 0) any = true;
     if (!any) continue;
-    st = eval_impl(ctx, slots, count, 1u << nb, rowmap, ctx->dvnd_persistent, 1,
-                   ctx->d_counter + 1 + nb);
+    st = prune && nb < MLP_NB_COUNT
+             ? prune_impl(ctx, slots, count, nb)
+             : eval_impl(ctx, slots, count, 1u << nb, rowmap, ctx->dvnd_persistent, 1,
+                         ctx->d_counter + 1 + nb);
     if (st) return st;
     // the round's last merge also ends the round for each slot
-    st = merge_impl(ctx, slots, count, nb, 1, nb == last ? max_rounds + 1 : 0);
+    st = merge_impl(ctx, slots, count, nb, keep ? 3 : 1, nb == last ? max_rounds + 1 : 0);
     if (st) return st;
   }
   if (last < 0) HCK(mlp_launch_round_end(ctx->stream, ctx->d_table, inl, dev, count, max_rounds));
@@ -1927,27 +1992,34 @@ int enqueue_fused(mlp_ctx* ctx, const int32_t* slots, int count, int max_rounds,
 // `rounds` DVND rounds over `slots`, as one captured graph when enabled.  A
 // chunk is captured the second time the same (slots, settings) is seen, so
 // every device list it needs already exists (no copies inside a capture).
+// The first `pruned` rounds may leave out rows that do not improve; the block
+// summaries are kept if they are pruned, or if another call on some of the
+// slots may be (keep).
 int enqueue_rounds(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max_rounds,
-                   int rounds) {
+                   int rounds, int pruned, bool keep) {
   int pcap = 0, ncap = 0;
   const bool fused = fused_ok(ctx, slots, count, rowmap, &pcap, &ncap);
+  if (!prune_ok(ctx, slots, count, rowmap)) pruned = 0;
   for (int r = 0; r < rounds; ++r) {
     const int st = fused ? enqueue_fused(ctx, slots, count, max_rounds, 1, pcap, ncap)
-                         : enqueue_round(ctx, slots, count, rowmap, max_rounds);
+                         : enqueue_round(ctx, slots, count, rowmap, max_rounds, r < pruned,
+                                         keep || r < pruned);
     if (st) return st;
   }
   return MLP_OK;
 }
 
 int run_chunk(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max_rounds,
-              int rounds, int gc = 0) {
+              int rounds, int pruned, bool keep = false, int gc = 0) {
+  pruned = std::max(0, std::min(pruned, rounds));
   if (!ctx->dvnd_graph || ctx->user_capture)
-    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds);
+    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
   int tile = ctx->tile_override;  // (the per-neighborhood shapes follow from the slots)
   // the captured launches embed the slot table address, every slot's id and
   // size (segment tables, merge capacities) and the settings
-  const int32_t hdr[9] = {rowmap, max_rounds, rounds, ctx->dvnd_persistent, tile, count,
-                          ctx->dvnd_nbs, ctx->merge_force_global ? 1 : 0, ctx->dvnd_fused};
+  const int32_t hdr[11] = {rowmap, max_rounds, rounds, ctx->dvnd_persistent, tile, count,
+                           ctx->dvnd_nbs, ctx->merge_force_global ? 1 : 0, ctx->dvnd_fused,
+                           pruned, keep ? 1 : 0};
   std::string key((const char*)hdr, sizeof hdr);
   key.append((const char*)&ctx->d_table, sizeof ctx->d_table);
   key.append((const char*)slots, 4 * (size_t)count);
@@ -1974,18 +2046,18 @@ int run_chunk(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max
       ctx->graph_exec[gc] = nullptr;
     }
     ctx->graph_key[gc] = key;
-    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds);
+    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
   }
   hipGraph_t g = nullptr;
   HCK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeRelaxed));
   ctx->capturing = true;
-  int st = enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds);
+  int st = enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
   ctx->capturing = false;
   const hipError_t ec = hipStreamEndCapture(ctx->stream, &g);
   if (st || ec != hipSuccess) {  // nothing captured ran: run the chunk eagerly instead
     if (g) hipGraphDestroy(g);
     ctx->graph_key[gc].clear();
-    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds);
+    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
   }
   const hipError_t ei = hipGraphInstantiate(&ctx->graph_exec[gc], g, nullptr, nullptr, 0);
   hipGraphDestroy(g);
@@ -2060,10 +2132,10 @@ int group_streams(mlp_ctx* ctx, int groups) {
 // capture).  Work queued after the call on the context stream follows every
 // group.
 int run_grouped(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max_rounds,
-                int rounds) {
+                int rounds, int pruned, bool keep = false) {
   const int groups = std::min(ctx->dvnd_groups, count);
   if (groups < 2 || ctx->dvnd_fused || ctx->dvnd_persistent || ctx->user_capture)
-    return run_chunk(ctx, slots, count, rowmap, max_rounds, rounds);
+    return run_chunk(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
   int st = group_streams(ctx, groups);
   if (st) return st;
   std::vector<int32_t> active(slots, slots + count), part[MLP_DVND_GROUPS];
@@ -2074,7 +2146,7 @@ int run_grouped(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int m
   for (int g = 1; g < groups; ++g) HCK(hipStreamWaitEvent(ctx->stream_grp[g], ctx->ev_fork, 0));
   for (int g = 0; g < groups && !st; ++g) {
     ctx->stream = g ? ctx->stream_grp[g] : ctx->stream_main;
-    st = run_chunk(ctx, part[g].data(), (int)part[g].size(), rowmap, max_rounds, rounds, g);
+    st = run_chunk(ctx, part[g].data(), (int)part[g].size(), rowmap, max_rounds, rounds, pruned, keep, g);
   }
   ctx->stream = ctx->stream_main;
   // joined also after a failed enqueue, so later work still follows it
@@ -2082,6 +2154,24 @@ int run_grouped(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int m
     HCK(hipEventRecord(ctx->ev_join[g], ctx->stream_grp[g]));
     HCK(hipStreamWaitEvent(ctx->stream_main, ctx->ev_join[g], 0));
   }
+  return st;
+}
+
+// Rounds after `done` ones of an mlp_dvnd call that may leave out rows that
+// do not improve: all but the one that max_rounds makes the last, whose rows
+// the caller can read (those of a round that applied nothing are completed
+// after it, complete_rows).
+int prunable(int max_rounds, int done) {
+  return max_rounds > 0 ? max_rounds - 1 - done : INT_MAX;
+}
+
+// The rows of slots whose DVND run ended in a pruned round, completed in
+// place: that round applied no move, so the tour is the one they belong to.
+int complete_rows(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap) {
+  const int nbs = std::min(ctx->dvnd_nbs, MLP_NB_COUNT);
+  const int st = eval_impl(ctx, slots, count, (1u << nbs) - 1u, rowmap, 0, 1 | 8, nullptr);
+  for (int q = 0; q < count; ++q)
+    for (int nb = 0; nb < nbs; ++nb) ctx->slots[slots[q]].merged[nb] = true;
   return st;
 }
 
@@ -2102,12 +2192,14 @@ int dvnd_independent(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap,
   HCK(hipEventRecord(ctx->ev_fork, ctx->stream_main));
   for (int g = 1; g < groups; ++g) HCK(hipStreamWaitEvent(ctx->stream_grp[g], ctx->ev_fork, 0));
   bool pending[MLP_DVND_GROUPS] = {};
+  int done[MLP_DVND_GROUPS] = {};  // rounds queued
   for (;;) {
     for (int g = 0; g < groups && !st; ++g)
       if (!pending[g] && !part[g].empty()) {
         ctx->stream = g ? ctx->stream_grp[g] : ctx->stream_main;
         st = run_chunk(ctx, part[g].data(), (int)part[g].size(), rowmap, max_rounds,
-                       ctx->dvnd_chunk, g);
+                       ctx->dvnd_chunk, prunable(max_rounds, done[g]), false, g);
+        done[g] += ctx->dvnd_chunk;
         if (!st && hipEventRecord(ctx->ev_chunk[g], ctx->stream) != hipSuccess)
           st = fail(ctx, MLP_EDEVICE, "DVND chunk event");
         pending[g] = !st;
@@ -2171,8 +2263,8 @@ int mlp_dvnd_start(mlp_ctx* ctx, const int32_t* slots, int32_t count) {
   return MLP_OK;
 }
 
-int mlp_dvnd_rounds(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
-                    int32_t rounds, int32_t max_rounds) {
+static int dvnd_rounds_impl(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
+                            int32_t rounds, int32_t max_rounds, bool improving) {
   int st = check_slots(ctx, slots, count);
   if (st) return st;
   st = check_mask(ctx, slots, count, (1u << ctx->dvnd_nbs) - 1u);
@@ -2180,7 +2272,18 @@ int mlp_dvnd_rounds(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t r
   if (rowmap != 0 && rowmap != 1) return fail(ctx, MLP_EINVAL, "rowmap must be 0 or 1");
   if (rounds < 0) return fail(ctx, MLP_EINVAL, "rounds must be >= 0");
   if (count == 0 || rounds == 0) return MLP_OK;
-  return run_grouped(ctx, slots, count, rowmap, max_rounds, rounds);
+  return run_grouped(ctx, slots, count, rowmap, max_rounds, rounds, improving ? INT_MAX : 0, improving);
+}
+
+int mlp_dvnd_rounds(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
+                    int32_t rounds, int32_t max_rounds) {
+  // the rows of the last round can be read: no round leaves any out
+  return dvnd_rounds_impl(ctx, slots, count, rowmap, rounds, max_rounds, false);
+}
+
+int mlp_dvnd_rounds_improving(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
+                              int32_t rounds, int32_t max_rounds) {
+  return dvnd_rounds_impl(ctx, slots, count, rowmap, rounds, max_rounds, true);
 }
 
 int mlp_dvnd_status(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t* active,
@@ -2237,9 +2340,12 @@ int mlp_dvnd(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
     if (st) return st;
     active.clear();
   }
+  int done = 0;
   while (!active.empty()) {
     const int c = (int)active.size();
-    st = run_grouped(ctx, active.data(), c, rowmap, max_rounds, ctx->dvnd_chunk);
+    st = run_grouped(ctx, active.data(), c, rowmap, max_rounds, ctx->dvnd_chunk,
+                     prunable(max_rounds, done));
+    done += ctx->dvnd_chunk;
     if (st) return st;
     st = mlp_dvnd_status(ctx, active.data(), c, flag.data(), nullptr);
     if (st) return st;
@@ -2248,6 +2354,10 @@ int mlp_dvnd(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
       if (flag[(size_t)q]) next.push_back(active[(size_t)q]);
     active.swap(next);
   }
+  // (a round is pruned for its active slots only if it is for all of them)
+  if (prunable(max_rounds, 0) > 0 && prune_ok(ctx, slots, count, rowmap))
+    st = complete_rows(ctx, slots, count, rowmap);
+  if (st) return st;
   if (rounds_out) return mlp_dvnd_status(ctx, slots, count, nullptr, rounds_out);
   return MLP_OK;
 }
@@ -2429,6 +2539,7 @@ int mlp_eval_static(mlp_ctx* ctx, int32_t inst, const int32_t* tour, uint32_t nb
   d.h32 = (int32_t*)(b + L.h32);
   d.t64 = (int64_t*)(b + L.t64);
   d.q64 = (int64_t*)(b + L.q64);
+  d.blk = (BlkSum*)(b + L.blk);
   d.info = (int64_t*)(b + L.info);
   d.nbs = MLP_NB_COUNT;
   SlotInitRows rows{};

@@ -17,6 +17,8 @@
 #include <new>
 #include <vector>
 
+#include "mlp_internal.h"
+
 namespace {
 
 struct Job {
@@ -302,8 +304,9 @@ int mlp_server_step(mlp_server* s, int32_t* active_out, int32_t* queued_out) {
     if (!ready[L] || l.active.empty()) continue;
     std::vector<int32_t> slots;
     for (Job* j : l.active) slots.push_back(j->slot);
-    st = mlp_dvnd_rounds(l.ctx, slots.data(), (int32_t)slots.size(), s->cfg.rowmap,
-                         s->cfg.rounds_per_step, s->cfg.max_rounds);
+    // the jobs' rows are never read
+    st = mlp_dvnd_rounds_improving(l.ctx, slots.data(), (int32_t)slots.size(), s->cfg.rowmap,
+                                   s->cfg.rounds_per_step, s->cfg.max_rounds);
     if (st) return st;
     l.chunk_pending = true;
   }
