@@ -369,11 +369,6 @@ __device__ __forceinline__ int64_t dpp64(int64_t v) {
   return (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
 
-// The value of lane ^ 1 (DPP quad permutation 1, 0, 3, 2).
-__device__ __forceinline__ int swap_pair(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);
-}
-
 // Inclusive wave scan (Hillis-Steele over rows of 16 lanes: shifts 1, 2, 4,
 // 8; then row 0's total into row 1 and row 2's into row 3, then rows 0-1's
 // total into rows 2 and 3), in registers.
@@ -395,33 +390,9 @@ __device__ __forceinline__ int64_t wave_sum64(int64_t v) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-// The summaries of 16-position blocks from threads holding eight positions
-// each (p0 on: packed coordinates of p0 - 1 .. p0 + 8 and w of p0 .. p0 + 8),
-// joined between neighbouring threads.  Positions clamped into the tour lie
-// inside the last block's range.
-__device__ __forceinline__ void put_summary(const SlotDev& s, int p0, const int (&xy)[kPrepPer + 2],
-                                            const int (&w)[kPrepPer + 1]) {
-  short2v lo = __builtin_bit_cast(short2v, xy[0]), hi = lo;
-  int wm = 0, wp = 0;
-#pragma unroll
-  for (int e = 1; e < kPrepPer + 2; ++e) {
-    const short2v c = __builtin_bit_cast(short2v, xy[e]);
-    lo = __builtin_elementwise_min(lo, c);
-    hi = __builtin_elementwise_max(hi, c);
-  }
-#pragma unroll
-  for (int e = 0; e < kPrepPer; ++e) {
-    wm = max(wm, w[e]);
-    wp = max(wp, w[e] + w[e + 1]);
-  }
-  lo = __builtin_elementwise_min(lo, __builtin_bit_cast(short2v, swap_pair(__builtin_bit_cast(int, lo))));
-  hi = __builtin_elementwise_max(hi, __builtin_bit_cast(short2v, swap_pair(__builtin_bit_cast(int, hi))));
-  wm = max(wm, swap_pair(wm));
-  wp = max(wp, swap_pair(wp));
-  if ((threadIdx.x & 1) == 0 && p0 < s.N)
-    *(int4*)(s.blk + p0 / MLP_BLK) =
-        make_int4(__builtin_bit_cast(int, lo), __builtin_bit_cast(int, hi), wm, wp);
-}
+template <int PER>
+__device__ __forceinline__ void put_summary(const SlotDev& s, int p0, const int (&xy)[PER + 2],
+                                            const int (&w)[PER + 1]);
 
 struct PrepLds {
   int64_t wt[kBlock / kWave][2];
@@ -464,7 +435,7 @@ __device__ __forceinline__ void prep_segment(const SlotDev& s, const int32_t* to
     const int p = p0 + e;
     w[e] = (p >= 1 && p < N) ? dist_xy(xy[e], xy[e + 1], dr) : 0;
   }
-  if (WRITE && sum) put_summary(s, p0, xy, w);
+  if (WRITE && sum) put_summary<kPrepPer>(s, p0, xy, w);
   int64_t lt[kPrepPer], lq[kPrepPer], at = 0, aq = 0;
 #pragma unroll
   for (int e = 0; e < kPrepPer; ++e) {
@@ -568,38 +539,243 @@ __device__ __forceinline__ void prep_flags(const SlotDev& s, int64_t Ttot) {
                             (b2 + 16 * Ttot < 2147483647LL ? MLP_LB32_2OPT : 0);
 }
 
-// The whole tour's prefix arrays and info words by one workgroup (inlined,
-// so that the tour and coordinate arrays keep their address space: LDS in a
-// merge, global memory in k_prep).
-__device__ __forceinline__ void prep_wg(const SlotDev& s, const int32_t* tour, PrepLds& P,
-                                        const int32_t* xyc = nullptr, bool sum = false) {
-  const int N = s.N, tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-  int64_t lacc = 0;  // this thread's share of L = sum_p T[p]
-  if (tid == 0) {
-    P.carry[0] = 0;
-    P.carry[1] = 0;
+// The wave sums of a prefix build (two sets, used in turn by its segments).
+template <int TB>
+struct PrepWaves {
+  int64_t q[2][TB / kWave];
+  int32_t t[2][TB / kWave];
+};
+
+// Inclusive scan of an int32 over the wave (DPP, as wave_scan_incl).
+__device__ __forceinline__ int wave_scan_i32(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+
+__device__ __forceinline__ int64_t readlane64(int64_t v, int l) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(uint64_t)v, l);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)v >> 32), l);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// The minimum (maximum) of packed 16-bit pairs over G neighbouring lanes.
+template <int G, bool MIN>
+__device__ __forceinline__ int group_pk(int v) {
+#define MLP_PK_STEP(CTRL)                                                                       \
+  {                                                                                             \
+    const int o = __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);                      \
+    const short2v a = __builtin_bit_cast(short2v, v), b = __builtin_bit_cast(short2v, o);       \
+    v = __builtin_bit_cast(int, MIN ? __builtin_elementwise_min(a, b) : __builtin_elementwise_max(a, b)); \
   }
-  __syncthreads();
-  for (int base = 0; base < N; base += kBlock * kPrepPer) {
-    const int64_t cT = P.carry[0], cQ = P.carry[1];
-    int64_t segT, segQ;
-    prep_segment<true>(s, tour, xyc, base, cT, cQ, P, segT, segQ, lacc, sum);
-    if (tid == 0) {
-      P.carry[0] = cT + segT;
-      P.carry[1] = cQ + segQ;
+  if constexpr (G >= 2) MLP_PK_STEP(0xb1)    // lane ^ 1
+  if constexpr (G >= 4) MLP_PK_STEP(0x4e)    // lane ^ 2
+  if constexpr (G >= 8) MLP_PK_STEP(0x141)   // 7 - lane within eight
+  if constexpr (G >= 16) MLP_PK_STEP(0x140)  // 15 - lane within sixteen
+#undef MLP_PK_STEP
+  return v;
+}
+template <int G>
+__device__ __forceinline__ int group_max(int v) {
+  if constexpr (G >= 2) v = max(v, __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true));
+  if constexpr (G >= 4) v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true));
+  if constexpr (G >= 8) v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true));
+  if constexpr (G >= 16) v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true));
+  return v;
+}
+
+// The summaries of 16-position blocks from threads holding PER positions
+// each (p0 on: packed coordinates of p0 - 1 .. p0 + PER and w of p0 .. p0 + PER),
+// joined between neighbouring lanes.  Positions clamped into the tour lie
+// inside the last block's range.
+template <int PER>
+__device__ __forceinline__ void put_summary(const SlotDev& s, int p0, const int (&xy)[PER + 2],
+                                            const int (&w)[PER + 1]) {
+  constexpr int G = MLP_BLK / PER;
+  short2v lo = __builtin_bit_cast(short2v, xy[0]), hi = lo;
+  int wm = 0, wp = 0;
+#pragma unroll
+  for (int e = 1; e < PER + 2; ++e) {
+    const short2v c = __builtin_bit_cast(short2v, xy[e]);
+    lo = __builtin_elementwise_min(lo, c);
+    hi = __builtin_elementwise_max(hi, c);
+  }
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    wm = max(wm, w[e]);
+    wp = max(wp, w[e] + w[e + 1]);
+  }
+  const int a = group_pk<G, true>(__builtin_bit_cast(int, lo));
+  const int b = group_pk<G, false>(__builtin_bit_cast(int, hi));
+  wm = group_max<G>(wm);
+  wp = group_max<G>(wp);
+  if (threadIdx.x % G == 0 && p0 < s.N) *(int4*)(s.blk + p0 / MLP_BLK) = make_int4(a, b, wm, wp);
+}
+
+// n consecutive words of a thread as the widest stores they allow.
+template <int PER>
+__device__ __forceinline__ void put_words(int32_t* d, const int32_t (&v)[PER]) {
+  if constexpr (PER >= 4) {
+#pragma unroll
+    for (int h = 0; h < PER; h += 4) *(int4*)(d + h) = make_int4(v[h], v[h + 1], v[h + 2], v[h + 3]);
+  } else if constexpr (PER == 2) {
+    *(int2*)d = make_int2(v[0], v[1]);
+  } else {
+    d[0] = v[0];
+  }
+}
+template <int PER>
+__device__ __forceinline__ void put_words(int64_t* d, const int64_t (&v)[PER]) {
+  if constexpr (PER >= 2) {
+#pragma unroll
+    for (int h = 0; h < PER; h += 2)
+      *(longlong2*)(d + h) = make_longlong2((long long)v[h], (long long)v[h + 1]);
+  } else {
+    d[0] = v[0];
+  }
+}
+
+// The whole tour's prefix arrays and info words by one workgroup of TB
+// threads, PER consecutive positions each, in segments of TB x PER positions
+// (inlined, so that the tour and coordinate arrays keep their address space:
+// LDS in a merge, global memory in k_prep).  One barrier a segment: the wave
+// sums go through LDS and every wave scans them; the latency needs no scan of
+// its own, sum_p T[p] = sum_p (N - p) w[p] = N T[N-1] - Q[N-1].
+// xyc: packed coordinates indexed by client (the merge's copy of the old
+// tour's xy, so the new tour needs no gather from the instance arrays), or
+// nullptr to read the instance arrays.  tour_out: where the tour is copied to
+// (nullptr: nowhere).  sum: block summaries too.
+template <int TB, int PER>
+__device__ __forceinline__ void prep_tour(const SlotDev& s, const int32_t* tour, PrepWaves<TB>& P,
+                                          const int32_t* xyc, int32_t* tour_out, bool sum) {
+  constexpr int NW = TB / kWave;
+  const int N = s.N, tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const float dr = round_dr(s.round);
+  int carryT = 0;  // T[N-1] < 2^31 (every instance: N maxd < 2^30)
+  int64_t carryQ = 0;
+  int buf = 0;
+  for (int base = 0; base < N; base += TB * PER, buf ^= 1) {
+    const int p0 = base + tid * PER;
+    // positions p0 - 1 .. p0 + PER (clamped into the tour): every client id is
+    // loaded before the first coordinate gather
+    int cl[PER + 2], xy[PER + 2];
+#pragma unroll
+    for (int e = 0; e < PER + 2; ++e) cl[e] = tour[min(max(p0 - 1 + e, 0), N - 1)];
+#pragma unroll
+    for (int e = 0; e < PER + 2; ++e) {
+      // client ids clamped into the instance: a tour read from caller memory
+      // never indexes outside the coordinate arrays
+      const int c = min(max(cl[e], 0), s.n - 1);
+      xy[e] = xyc ? xyc[c] : (ldg(s.xs + c) << 16) | ldg(s.ys + c);
     }
-    __syncthreads();
+    int w[PER + 1];  // w[e]: edge into position p0 + e
+#pragma unroll
+    for (int e = 0; e <= PER; ++e) {
+      const int p = p0 + e;
+      const int d = dist_xy(xy[e], xy[e + 1], dr);
+      w[e] = (p >= 1 && p < N) ? d : 0;
+    }
+    if (sum) put_summary<PER>(s, p0, xy, w);
+    int lt[PER], at = 0;
+    int64_t lq[PER], aq = 0;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      at += w[e];
+      aq += (int64_t)(p0 + e) * w[e];
+      lt[e] = at;
+      lq[e] = aq;
+    }
+    const int it = wave_scan_i32(at);
+    const int64_t iq = wave_scan_incl(aq, lane);
+    int offT = carryT + it - at;
+    int64_t offQ = carryQ + iq - aq;
+    if constexpr (NW > 1) {
+      if (lane == kWave - 1) {
+        P.t[buf][wave] = it;
+        P.q[buf][wave] = iq;
+      }
+      __syncthreads();
+      // inclusive scan of the wave sums over the first NW (at most 16) lanes
+      int tv = P.t[buf][lane % NW];
+      int64_t qv = P.q[buf][lane % NW];
+      tv += __builtin_amdgcn_update_dpp(0, tv, 0x111, 0xf, 0xf, false);
+      qv += dpp64<0x111, 0xf>(qv);
+      tv += __builtin_amdgcn_update_dpp(0, tv, 0x112, 0xf, 0xf, false);
+      qv += dpp64<0x112, 0xf>(qv);
+      if constexpr (NW > 4) {
+        tv += __builtin_amdgcn_update_dpp(0, tv, 0x114, 0xf, 0xf, false);
+        qv += dpp64<0x114, 0xf>(qv);
+      }
+      if constexpr (NW > 8) {
+        tv += __builtin_amdgcn_update_dpp(0, tv, 0x118, 0xf, 0xf, false);
+        qv += dpp64<0x118, 0xf>(qv);
+      }
+      if (wave > 0) {
+        offT += __builtin_amdgcn_readlane(tv, wave - 1);
+        offQ += readlane64(qv, wave - 1);
+      }
+      carryT += __builtin_amdgcn_readlane(tv, NW - 1);
+      carryQ += readlane64(qv, NW - 1);
+    } else {
+      carryT += __builtin_amdgcn_readlane(it, kWave - 1);
+      carryQ += readlane64(iq, kWave - 1);
+    }
+    int32_t vx[PER], vw[PER], vt[PER], vq[PER], vg[PER], vh[PER], vc[PER];
+    int64_t T8[PER], Q8[PER];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const int p = p0 + e;
+      const int T = offT + lt[e];
+      const int64_t Q = offQ + lq[e];
+      T8[e] = T;
+      Q8[e] = Q;
+      vc[e] = cl[e + 1];
+      vx[e] = xy[e + 1];
+      vw[e] = w[e];
+      vt[e] = T;
+      vq[e] = (int32_t)(uint32_t)(uint64_t)Q;
+      const uint32_t Z = 2u * (uint32_t)(uint64_t)Q - (uint32_t)(2 * p + 1) * (uint32_t)T;
+      vg[e] = (int32_t)(0u - (uint32_t)(N - p) * (uint32_t)w[e] - Z);
+      vh[e] = (int32_t)(Z - (uint32_t)(N - p - 1) * (uint32_t)w[e + 1]);
+    }
+    if (p0 + PER <= N) {
+      // p0 is a multiple of PER and every array 256-byte aligned
+      put_words<PER>(s.xy + p0, vx);
+      put_words<PER>(s.w + p0, vw);
+      put_words<PER>(s.t32 + p0, vt);
+      put_words<PER>(s.q32 + p0, vq);
+      put_words<PER>(s.g32 + p0, vg);
+      put_words<PER>(s.h32 + p0, vh);
+      put_words<PER>(s.t64 + p0, T8);
+      put_words<PER>(s.q64 + p0, Q8);
+      if (tour_out) put_words<PER>(tour_out + p0, vc);
+    } else {
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        const int p = p0 + e;
+        if (p < N) {
+          s.xy[p] = vx[e];
+          s.w[p] = vw[e];
+          s.t32[p] = vt[e];
+          s.q32[p] = vq[e];
+          s.g32[p] = vg[e];
+          s.h32[p] = vh[e];
+          s.t64[p] = T8[e];
+          s.q64[p] = Q8[e];
+          if (tour_out) tour_out[p] = vc[e];
+        }
+      }
+    }
   }
-  const int64_t lw = wave_sum64(lacc);
-  if (lane == 0) P.lsum[wave] = lw;
-  __syncthreads();
-  if (tid == 0) {
-    int64_t L = 0;
-    for (int q = 0; q < kBlock / kWave; ++q) L += P.lsum[q];
-    s.info[MLP_INFO_LATENCY] = L;
-    prep_flags(s, P.carry[0]);  // T[N-1]: positions past N-1 add nothing
+  if (tid == 0) {  // positions past N-1 add nothing to the carries
+    s.info[MLP_INFO_LATENCY] = (int64_t)N * carryT - carryQ;
+    prep_flags(s, carryT);
   }
-  __syncthreads();
 }
 
 }  // namespace
@@ -608,12 +784,16 @@ __device__ __forceinline__ void prep_wg(const SlotDev& s, const int32_t* tour, P
 // kernels
 // ===========================================================================
 
-__global__ __launch_bounds__(kBlock) void k_prep(const SlotDev* __restrict__ table,
-                                                 SlotListInline list, const int32_t* list_dev) {
-  __shared__ PrepLds P;
+// One workgroup per slot.  Its time is the latency of one chain (client ids,
+// coordinates, scans, stores), so a tour up to PER x 1024 positions takes one
+// segment with as few positions a thread as its size allows.
+template <int TB, int PER>
+__global__ __launch_bounds__(TB) void k_prep(const SlotDev* __restrict__ table,
+                                             SlotListInline list, const int32_t* list_dev) {
+  __shared__ PrepWaves<TB> P;
   const int id = list_at(list, list_dev, blockIdx.x);
   const SlotDev& s = table[id];
-  prep_wg(s, s.tour, P);
+  prep_tour<TB, PER>(s, s.tour, P, nullptr, nullptr, false);
   if (threadIdx.x == 0) {
     s.info[MLP_INFO_ROUND_MOVES] = 0;
     s.info[MLP_INFO_TOTAL_MOVES] = 0;
@@ -643,7 +823,7 @@ __global__ __launch_bounds__(kBlock) void k_dvnd_start(const SlotDev* __restrict
     for (int e = 0; e < kPrepPer + 2; ++e) xy[e] = ldg(s.xy + min(max(p0 - 1 + e, 0), N - 1));
 #pragma unroll
     for (int e = 0; e <= kPrepPer; ++e) w[e] = p0 + e < N ? ldg(s.w + p0 + e) : 0;
-    put_summary(s, p0, xy, w);
+    put_summary<kPrepPer>(s, p0, xy, w);
   }
 }
 
@@ -853,45 +1033,47 @@ __device__ __forceinline__ int greedy_wave(const SlotDev& s, int nb, int N, int 
 }
 
 
-// Applies K kept moves (disjoint regions) to s.tour through a position ->
-// source map: a move with a short region is applied by one thread, the few
-// long ones (regions are disjoint, so at most N / kShortMove) by all threads.
-// ij(q) gives the q-th kept move as (i << 32 | j); tnew ends as the new tour.
-// loaded: told and tnew already hold the tour (copied at the kernel's start,
-// its load overlapping the row-key loads).
-template <typename IJ>
+// Applies K kept moves (disjoint regions) to tnew, a copy of the tour told,
+// through a position -> source map: 16 lanes to a move whose region is short,
+// a wave to each of the few long ones (regions are disjoint, so at most
+// N / kShortMove), or the workgroup if there are fewer of those than waves.
+// ij(q) gives the q-th kept move as (i << 32 | j); tnew ends as the new tour
+// (after the caller's next barrier).  loaded: told and tnew already hold the
+// tour (copied at the kernel's start, its load overlapping the row-key loads).
+template <int TB, typename IJ>
 __device__ __forceinline__ void apply_kept(const SlotDev& s, int nb, int K, IJ ij, int32_t* told,
                                            int32_t* tnew, int& s_long, int* s_longq,
-                                           bool loaded = false, bool copy_back = true) {
+                                           bool loaded = false) {
   const int N = s.N, tid = threadIdx.x, k = nb_k(nb);
   int32_t* const tour = s.tour;  // in a register across the loops' stores
   if (!loaded)
-    for (int p = tid; p < N; p += kBlock) {
+    for (int p = tid; p < N; p += TB) {
       const int c = tour[p];
       told[p] = c;
       tnew[p] = c;
     }
   if (tid == 0) s_long = 0;
   __syncthreads();
-  for (int q = tid; q < K; q += kBlock) {
+  constexpr int G = 16;
+  for (int q = tid / G; q < K; q += TB / G) {
     const int64_t v = ij(q);
     const int i = (int)(v >> 32), j = (int)(uint32_t)v;
     if (move_span(nb, k, i, j) <= kShortMove) {
-      apply_span(nb, k, i, j, told, tnew, 0, 1);
-    } else {
+      apply_span(nb, k, i, j, told, tnew, tid % G, G);
+    } else if (tid % G == 0) {
       const int at = atomicAdd(&s_long, 1);
       if (at < kLongMoves) s_longq[at] = q;
     }
   }
   __syncthreads();
   const int nl = min(s_long, kLongMoves);
-  for (int t = 0; t < nl; ++t) {
+  const bool all = nl * (2 * kWave) < TB;  // fewer than half a move a wave
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  for (int t = all ? 0 : wave; t < nl; t += all ? 1 : TB / kWave) {
     const int64_t v = ij(s_longq[t]);
-    apply_span(nb, k, (int)(v >> 32), (int)(uint32_t)v, told, tnew, tid, kBlock);
+    if (all) apply_span(nb, k, (int)(v >> 32), (int)(uint32_t)v, told, tnew, tid, TB);
+    else apply_span(nb, k, (int)(v >> 32), (int)(uint32_t)v, told, tnew, tid % kWave, kWave);
   }
-  __syncthreads();
-  if (copy_back)
-    for (int p = tid; p < N; p += kBlock) tour[p] = tnew[p];
 }
 
 }  // namespace
@@ -900,7 +1082,7 @@ __device__ __forceinline__ void apply_kept(const SlotDev& s, int nb, int K, IJ i
 // merges blocks of kk keys, element i ascending when (i & kk) == 0 (the
 // whole array flipped for a descending sort); its phase jj compares i with
 // i + jj for (i & jj) == 0.  The array is cut into segments of 64 E keys
-// (E = 2, 4 or 8: every wave of the workgroup holds at least one), held in
+// (E = 2, 4 or 8: at least four waves of the workgroup hold one), held in
 // the registers of one wave, key base + 64 e + lane in v[e] of that lane:
 // phases with jj of 64 .. 32 E pair keys inside a lane, jj of 1..32 pair
 // lanes (lane ^ jj); phases with jj >= 64 E go pair by pair through memory
@@ -973,11 +1155,11 @@ __device__ __forceinline__ void seg_phases(int64_t (&v)[E], int base, int lane, 
 
 // Stages kk0 .. kk1 (powers of two) on every segment of k[0..P), phases
 // below 64 E only (those of a larger stage follow its memory phases).
-template <int E>
+template <int E, int TB>
 __device__ __forceinline__ void seg_pass(int64_t* k, int P, int kk0, int kk1, bool desc) {
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // uniform segment bases
-  for (int base = wave * kWave * E; base < P; base += kBlock * E) {
+  for (int base = wave * kWave * E; base < P; base += TB * E) {
     int64_t v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = k[base + kWave * e + lane];
@@ -989,14 +1171,15 @@ __device__ __forceinline__ void seg_pass(int64_t* k, int P, int kk0, int kk1, bo
 
 // Phase jj (>= 64 E) of stage kk through memory: P/2 compare-swaps, up to
 // four pairs per thread loaded before any is compared.
+template <int TB>
 __device__ __forceinline__ void pair_phase(int64_t* k, int P, int kk, int jj, bool desc) {
   const int half = P >> 1, lj = 31 - __clz(jj);
-  for (int p0 = threadIdx.x; p0 < half; p0 += 4 * kBlock) {
+  for (int p0 = threadIdx.x; p0 < half; p0 += 4 * TB) {
     int lo[4];
     int64_t va[4], vb[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int pr = min(p0 + u * kBlock, half - 1);
+      const int pr = min(p0 + u * TB, half - 1);
       lo[u] = ((pr >> lj) << (lj + 1)) | (pr & (jj - 1));
       va[u] = k[lo[u]];
       vb[u] = k[lo[u] + jj];
@@ -1004,7 +1187,7 @@ __device__ __forceinline__ void pair_phase(int64_t* k, int P, int kk, int jj, bo
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const bool sw = (va[u] > vb[u]) == (((lo[u] & kk) == 0) != desc);
-      if (p0 + u * kBlock < half) {
+      if (p0 + u * TB < half) {
         k[lo[u]] = sw ? vb[u] : va[u];
         k[lo[u] + jj] = sw ? va[u] : vb[u];
       }
@@ -1013,43 +1196,45 @@ __device__ __forceinline__ void pair_phase(int64_t* k, int P, int kk, int jj, bo
 }
 
 // Sort of k[0..P), P a power of two >= 256 E, ascending or descending.
-template <int E>
+template <int E, int TB>
 __device__ __forceinline__ void sort_block(int64_t* k, int P, bool desc) {
   constexpr int SEG = kWave * E;
-  seg_pass<E>(k, P, 2, min(P, SEG), desc);
+  seg_pass<E, TB>(k, P, 2, min(P, SEG), desc);
   __syncthreads();
   for (int kk = 2 * SEG; kk <= P; kk <<= 1) {
     for (int jj = kk >> 1; jj >= SEG; jj >>= 1) {
-      pair_phase(k, P, kk, jj, desc);
+      pair_phase<TB>(k, P, kk, jj, desc);
       __syncthreads();
     }
-    seg_pass<E>(k, P, kk, kk, desc);
+    seg_pass<E, TB>(k, P, kk, kk, desc);
     __syncthreads();
   }
 }
 
 // Ascending sort of a bitonic sequence k[0..P) (the last stage of a sort),
 // P >= 2048.
+template <int TB>
 __device__ __forceinline__ void merge_block(int64_t* k, int P) {
   for (int jj = P >> 1; jj >= kSortSeg; jj >>= 1) {
-    pair_phase(k, P, 2 * P, jj, false);
+    pair_phase<TB>(k, P, 2 * P, jj, false);
     __syncthreads();
   }
-  seg_pass<8>(k, P, 2 * P, 2 * P, false);
+  seg_pass<8, TB>(k, P, 2 * P, 2 * P, false);
   __syncthreads();
 }
 
 // Ascending sort of keys[0..M) (keys[M..P) padded with KEY_NONE, P the
 // power of two at or above max(M, 512)), in segments of 128, 256 or 512
-// keys so that each of the four waves holds one.
+// keys so that four waves hold one each.
+template <int TB>
 __device__ __forceinline__ void bitonic_keys(int64_t* keys, int M) {
-  int P = 2 * kBlock;
+  int P = 512;
   while (P < M) P <<= 1;
-  for (int t = M + threadIdx.x; t < P; t += kBlock) keys[t] = MLP_KEY_NONE;
+  for (int t = M + threadIdx.x; t < P; t += TB) keys[t] = MLP_KEY_NONE;
   __syncthreads();
-  if (P <= 2 * kBlock) sort_block<2>(keys, P, false);
-  else if (P <= 4 * kBlock) sort_block<4>(keys, P, false);
-  else sort_block<8>(keys, P, false);
+  if (P <= 512) sort_block<2, TB>(keys, P, false);
+  else if (P <= 1024) sort_block<4, TB>(keys, P, false);
+  else sort_block<8, TB>(keys, P, false);
 }
 
 template <typename T>
@@ -1059,22 +1244,24 @@ __device__ __forceinline__ void stg(T* p, T v) {
 
 // n keys from global memory into LDS, eight loads in flight per thread;
 // those from index `valid` on read as KEY_NONE.
+template <int TB>
 __device__ __forceinline__ void keys_to_lds(int64_t* sb, const int64_t* g, int n, int valid) {
-  for (int t0 = threadIdx.x; t0 < n; t0 += 8 * kBlock) {
+  for (int t0 = threadIdx.x; t0 < n; t0 += 8 * TB) {
     int64_t v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int t = t0 + u * kBlock;
+      const int t = t0 + u * TB;
       v[u] = (t < n && t < valid) ? ldg(g + t) : MLP_KEY_NONE;
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
-      if (t0 + u * kBlock < n) sb[t0 + u * kBlock] = v[u];
+      if (t0 + u * TB < n) sb[t0 + u * TB] = v[u];
   }
 }
 
+template <int TB>
 __device__ __forceinline__ void keys_to_global(int64_t* g, const int64_t* sb, int n) {
-  for (int t = threadIdx.x; t < n; t += kBlock) stg(g + t, sb[t]);
+  for (int t = threadIdx.x; t < n; t += TB) stg(g + t, sb[t]);
 }
 
 // A merge whose working arrays are in global memory still sorts up to
@@ -1084,20 +1271,21 @@ constexpr int kGmemSortCap = 16384;
 
 // The merge's small shared variables (counts, the long-move queue, the
 // prefix rebuild's scan carries).
+template <int TB>
 struct MergeShared {
   int m, kept, lng;
   int longq[kLongMoves];
-  PrepLds PL;
+  PrepWaves<TB> PL;
 };
 
 // 2.-3. of a merge: sort of the M improving (cost, row) keys == stable sort
 // by cost of the row list, then the greedy filter on wave 0.  Returns the
 // kept count; sk points at the sorted keys, whose first entries then hold the
 // kept moves as (i << 32 | j).
-template <bool GMEM>
+template <bool GMEM, int TB>
 __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap, int N, int M,
                                            int64_t* keys, int64_t* lds, const uint16_t* ctxL,
-                                           uint32_t* bits, MergeShared& S, int64_t*& sk) {
+                                           uint32_t* bits, MergeShared<TB>& S, int64_t*& sk) {
   const int tid = threadIdx.x;
   const int64_t* gtail = nullptr;  // sorted keys beyond the LDS buffer
   int tail = INT32_MAX;
@@ -1114,7 +1302,7 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
       if (tid < M) keys[rank] = my;
       __builtin_amdgcn_wave_barrier();
     }
-  } else if (!GMEM && M <= kBlock) {
+  } else if (!GMEM && M <= 256) {
     // one key per thread: the same rank sort over the workgroup (M reads of
     // LDS broadcasts per thread against the 36 barrier phases of a bitonic
     // sort of 256)
@@ -1130,8 +1318,8 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
     // fit the LDS sort buffer: sort them there, and let the greedy and the
     // apply read them from LDS
     int64_t* sb = lds;
-    keys_to_lds(sb, keys, M, M);
-    bitonic_keys(sb, M);
+    keys_to_lds<TB>(sb, keys, M, M);
+    bitonic_keys<TB>(sb, M);
     sk = sb;
   } else if (GMEM && M <= 2 * kGmemSortCap) {
     // twice the LDS buffer (keys[M..2 cap) in the slot's memory are padded):
@@ -1142,32 +1330,32 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
     int64_t* sb = lds;
     constexpr int H = kGmemSortCap;
     for (int h = 0; h < 2; ++h) {
-      keys_to_lds(sb, keys + h * H, H, M - h * H);
+      keys_to_lds<TB>(sb, keys + h * H, H, M - h * H);
       __syncthreads();
-      sort_block<8>(sb, H, h == 1);
-      keys_to_global(keys + h * H, sb, H);
+      sort_block<8, TB>(sb, H, h == 1);
+      keys_to_global<TB>(keys + h * H, sb, H);
       __syncthreads();
     }
-    for (int t0 = tid; t0 < H; t0 += 4 * kBlock) {
+    for (int t0 = tid; t0 < H; t0 += 4 * TB) {
       int64_t a[4], b[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        a[u] = ldg(keys + t0 + u * kBlock);
-        b[u] = ldg(keys + t0 + u * kBlock + H);
+        a[u] = ldg(keys + t0 + u * TB);
+        b[u] = ldg(keys + t0 + u * TB + H);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        stg(keys + t0 + u * kBlock, min(a[u], b[u]));
-        stg(keys + t0 + u * kBlock + H, max(a[u], b[u]));
+        stg(keys + t0 + u * TB, min(a[u], b[u]));
+        stg(keys + t0 + u * TB + H, max(a[u], b[u]));
       }
     }
     __syncthreads();
     for (int h = 1; h >= 0; --h) {
-      keys_to_lds(sb, keys + h * H, H, H);
+      keys_to_lds<TB>(sb, keys + h * H, H, H);
       __syncthreads();
-      merge_block(sb, H);
+      merge_block<TB>(sb, H);
       if (h == 1) {
-        keys_to_global(keys + H, sb, H);
+        keys_to_global<TB>(keys + H, sb, H);
         __syncthreads();
       }
     }
@@ -1175,7 +1363,7 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
     gtail = keys;
     tail = H;
   } else {
-    bitonic_keys(keys, M);
+    bitonic_keys<TB>(keys, M);
   }
   // 3. greedy filter on wave 0
   if (tid < kWave) {
@@ -1191,52 +1379,57 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
 
 // Rows [q0, q1) of a merge: the tour and its coordinates by client copied
 // (told, tnew, xyc), and each improving row's (cost, row) key handed to
-// put(key) with its ctx recorded.  Each thread issues the loads of eight
-// rows (strided by kBlock) before it uses the first.
-template <typename Put>
-__device__ __forceinline__ void merge_rows(const SlotDev& s, const int64_t* rk, int R, int q0,
+// put(key) with its ctx recorded.  Each thread issues the loads of P rows
+// (strided by TB) before it uses the first.  rows(q) loads row q's key from
+// either buffer; the choice, which waits for the slot's info words, comes
+// when the keys are used: pick(a, b).
+template <int TB, int P, typename Rows, typename Pick, typename Put>
+__device__ __forceinline__ void merge_rows(const SlotDev& s, Rows rows, Pick pick, int R, int q0,
                                            int q1, int32_t* told, int32_t* tnew, int32_t* xyc,
                                            uint16_t* ctxL, Put put) {
-  constexpr int P = 8;
   const int N = s.N, tid = threadIdx.x;
   const int32_t* const tour = s.tour;  // in registers across the loop's stores
   const int32_t* const xy = s.xy;
   const int rend = min(R, q1), nend = min(N, q1);
-  for (int base = q0; base < q1; base += kBlock * P) {
-    int64_t key[P];
+  for (int base = q0; base < q1; base += TB * P) {
+    int64_t ka[P], kb[P];
     int c[P], xq[P];
 #pragma unroll
     for (int e = 0; e < P; ++e) {
-      const int q = base + e * kBlock + tid;
-      key[e] = q < rend ? rk[q] : MLP_KEY_NONE;
+      const int q = base + e * TB + tid;
+      ka[e] = kb[e] = MLP_KEY_NONE;
+      if (q < rend) rows(q, ka[e], kb[e]);
       c[e] = q < nend ? tour[q] : 0;
       xq[e] = q < nend ? xy[q] : 0;
     }
 #pragma unroll
     for (int e = 0; e < P; ++e) {
-      const int q = base + e * kBlock + tid;
+      const int q = base + e * TB + tid;
       if (q < nend) {
         told[q] = c[e];
         tnew[q] = c[e];
         xyc[c[e]] = xq[e];
       }
-      if (key[e] != MLP_KEY_NONE && (key[e] >> MLP_KEY_SHIFT) < 0) {
-        put((key[e] >> MLP_KEY_SHIFT) * (int64_t)(1 << MLP_KEY_SHIFT) + q);
-        ctxL[q] = (uint16_t)(key[e] & MLP_KEY_MASK);
+      const int64_t key = pick(ka[e], kb[e]);  // KEY_NONE is positive
+      if (key < 0) {
+        put((key >> MLP_KEY_SHIFT) * (int64_t)(1 << MLP_KEY_SHIFT) + q);
+        ctxL[q] = (uint16_t)(key & MLP_KEY_MASK);
       }
     }
   }
 }
 
 // Merge + apply of one slot by one workgroup; lds holds the working arrays
-// (mlp_merge_lds_bytes(pcap_l, ncap_l)).
+// (mlp_merge_lds_bytes(pcap_l, ncap_l)).  flags bit 0: inside a DVND round;
+// bit 1: block summaries of the new tour are kept.
+template <int TB, int PER>
 __device__ __forceinline__ void merge_slot(const SlotDev& s, int nb, int rowmap, int pcap_l,
-                                           int ncap_l, int skip_inactive, int tail, int64_t* lds,
-                                           MergeShared& S) {
-  if (skip_inactive && s.info[MLP_INFO_ACTIVE] == 0) return;
+                                           int ncap_l, int flags, int tail, int64_t* lds,
+                                           MergeShared<TB>& S) {
   const int N = s.N, tid = threadIdx.x;
   const int R = rows_of(nb, rowmap, N);
   const int pcap = pcap_l, ncap = ncap_l;  // capacities of the launch
+  const bool dvnd = flags != 0;
   int64_t* keys = lds;
   int32_t* told = (int32_t*)(keys + pcap);
   int32_t* tnew = told + ncap;
@@ -1245,24 +1438,33 @@ __device__ __forceinline__ void merge_slot(const SlotDev& s, int nb, int rowmap,
   uint32_t* bits = (uint32_t*)(xyc + ncap);
   uint16_t* ctxL = (uint16_t*)((uint32_t*)(xyc + ncap) + claim_words(ncap));  // ctx of each improving row
   int64_t* sk = keys;  // the sorted keys (greedy, apply)
+  const int64_t active = ldg(s.info + MLP_INFO_ACTIVE);
+  const int64_t parity = ldg(s.info + MLP_INFO_PARITY0 + nb);
 
   if (tid == 0) S.m = 0;
-  for (int w = tid; w < nwords; w += kBlock) bits[w] = 0;
+  for (int w = tid; w < nwords; w += TB) bits[w] = 0;
+  if (dvnd && active == 0) return;
   __syncthreads();
   // 1. improving rows -> (cost, row) keys.  Inside a DVND round the eval
   // wrote the buffer opposite info[PARITY0 + nb]; this merge commits it.
   // The tour (for the apply step) and its coordinates (for the prefix
   // rebuild, by client) are copied in the same loop, so their loads go out
-  // with the row keys'.
-  const int par = (int)(s.info[MLP_INFO_PARITY0 + nb] & 1) ^ (skip_inactive ? 1 : 0);
-  const int64_t* rk = s.rows[nb] + (par ? s.rowcap : 0);
-  if (skip_inactive) {
-    __syncthreads();  // every thread has read the old parity
-    if (tid == 0) s.info[MLP_INFO_PARITY0 + nb] = par;
-  }
-  merge_rows(s, rk, R, 0, max(R, N), told, tnew, xyc, ctxL,
-             [&](int64_t k) { keys[atomicAdd(&S.m, 1)] = k; });
+  // with the row keys'; both buffers' keys are loaded, so that the loads do
+  // not wait for the parity.
+  const int par = (int)(parity & 1) ^ (dvnd ? 1 : 0);
+  const int64_t* const rk = s.rows[nb];
+  const int cap = s.rowcap;
+  merge_rows<TB, PER>(
+      s,
+      [&](int q, int64_t& a, int64_t& b) {
+        a = ldg(rk + q);
+        b = ldg(rk + cap + q);
+      },
+      [&](int64_t a, int64_t b) { return par ? b : a; }, R, 0, max(R, N), told, tnew, xyc, ctxL,
+      [&](int64_t k) { keys[atomicAdd(&S.m, 1)] = k; });
   __syncthreads();
+  // every thread has read the old parity
+  if (dvnd && tid == 0) s.info[MLP_INFO_PARITY0 + nb] = par;
   const int M = S.m;
   if (M == 0) {
     if (tid == 0) {
@@ -1271,10 +1473,11 @@ __device__ __forceinline__ void merge_slot(const SlotDev& s, int nb, int rowmap,
     }
     return;
   }
-  const int K = sort_greedy<false>(s, nb, rowmap, N, M, keys, lds, ctxL, bits, S, sk);
+  const int K = sort_greedy<false, TB>(s, nb, rowmap, N, M, keys, lds, ctxL, bits, S, sk);
   // 4. apply the kept moves, rebuild the prefix arrays
-  apply_kept(s, nb, K, [&](int q) { return sk[q]; }, told, tnew, S.lng, S.longq, true);
-  prep_wg(s, tnew, S.PL, xyc, (skip_inactive & 2) != 0);
+  apply_kept<TB>(s, nb, K, [&](int q) { return sk[q]; }, told, tnew, S.lng, S.longq, true);
+  __syncthreads();
+  prep_tour<TB, PER>(s, tnew, S.PL, xyc, s.tour, (flags & 2) != 0);
   if (tid == 0) {
     s.info[MLP_INFO_KEPT0 + nb] = K;
     s.info[MLP_INFO_ROUND_MOVES] += K;
@@ -1285,16 +1488,18 @@ __device__ __forceinline__ void merge_slot(const SlotDev& s, int nb, int rowmap,
 
 // One workgroup per slot.  Dynamic LDS: keys[P] int64 | told[N] | tnew[N] | bits | ctx[P].
 // tail != 0: this is the last merge of a DVND round, and it also ends the
-// round for each active slot (round_tail, max_rounds = tail - 1).
-__global__ __launch_bounds__(kBlock) void k_merge_apply(const SlotDev* __restrict__ table,
-                                                        SlotListInline list,
-                                                        const int32_t* list_dev, int nb,
-                                                        int rowmap, int pcap_l, int ncap_l,
-                                                        int skip_inactive, int tail) {
+// round for each active slot (round_tail, max_rounds = tail - 1).  TB x PER is
+// at least the largest N of the launch, with PER 1 while a workgroup has
+// threads enough (merge_launch).
+template <int TB, int PER>
+__global__ __launch_bounds__(TB) void k_merge_apply(const SlotDev* __restrict__ table,
+                                                    SlotListInline list, const int32_t* list_dev,
+                                                    int nb, int rowmap, int pcap_l, int ncap_l,
+                                                    int flags, int tail) {
   extern __shared__ int64_t lds[];
-  __shared__ MergeShared S;
+  __shared__ MergeShared<TB> S;
   const int id = list_at(list, list_dev, blockIdx.x);
-  merge_slot(table[id], nb, rowmap, pcap_l, ncap_l, skip_inactive, tail, lds, S);
+  merge_slot<TB, PER>(table[id], nb, rowmap, pcap_l, ncap_l, flags, tail, lds, S);
 }
 
 // ---------------------------------------------------------------------------
@@ -1358,8 +1563,10 @@ __global__ __launch_bounds__(kBlock) void k_mg_compact(const SlotDev* __restrict
   const int64_t* rk = s.rows[nb] + (par ? s.rowcap : 0);
   if (tid == 0) lm = 0;
   __syncthreads();
-  merge_rows(s, rk, R, q0, q1, a.told, a.tnew, a.xyc, a.ctxL,
-             [&](int64_t k) { lk[atomicAdd(&lm, 1)] = k; });
+  merge_rows<kBlock, 8>(
+      s, [&](int q, int64_t& ka, int64_t& kb) { ka = kb = ldg(rk + q); },
+      [&](int64_t ka, int64_t) { return ka; }, R, q0, q1, a.told, a.tnew, a.xyc, a.ctxL,
+      [&](int64_t k) { lk[atomicAdd(&lm, 1)] = k; });
   __syncthreads();
   const int m = lm;
   if (m == 0) return;
@@ -1369,12 +1576,14 @@ __global__ __launch_bounds__(kBlock) void k_mg_compact(const SlotDev* __restrict
   for (int t = tid; t < m; t += kBlock) a.keys[lbase + t] = lk[t];
 }
 
-__global__ __launch_bounds__(kBlock) void k_mg_select(const SlotDev* __restrict__ table,
+constexpr int kSelBlock = 1024;  // threads of k_mg_select
+
+__global__ __launch_bounds__(kSelBlock) void k_mg_select(const SlotDev* __restrict__ table,
                                                       SlotListInline list, const int32_t* list_dev,
                                                       int nb, int rowmap, int skip_inactive,
                                                       int tail) {
   extern __shared__ int64_t lds[];
-  __shared__ MergeShared S;
+  __shared__ MergeShared<kSelBlock> S;
   const SlotDev& s = table[list_at(list, list_dev, blockIdx.x)];
   const int tid = threadIdx.x;
   if (skip_inactive && s.info[MLP_INFO_ACTIVE] == 0) {
@@ -1387,7 +1596,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_select(const SlotDev* __restrict_
   const int par = (int)(s.info[MLP_INFO_PARITY0 + nb] & 1) ^ (skip_inactive ? 1 : 0);
   uint32_t* bits = (uint32_t*)(lds + kGmemSortCap);
   const int nwords = claim_words(N);
-  for (int w = tid; w < nwords; w += kBlock) bits[w] = 0;
+  for (int w = tid; w < nwords; w += kSelBlock) bits[w] = 0;
   __syncthreads();  // every thread has read the count and the parity
   if (tid == 0) {
     s.info[MLP_INFO_MCOUNT] = 0;
@@ -1402,9 +1611,9 @@ __global__ __launch_bounds__(kBlock) void k_mg_select(const SlotDev* __restrict_
     return;
   }
   int64_t* sk = a.keys;
-  const int K = sort_greedy<true>(s, nb, rowmap, N, M, a.keys, lds, a.ctxL, bits, S, sk);
+  const int K = sort_greedy<true, kSelBlock>(s, nb, rowmap, N, M, a.keys, lds, a.ctxL, bits, S, sk);
   // tnew becomes the new tour; k_mg_rebuild copies it back
-  apply_kept(s, nb, K, [&](int q) { return sk[q]; }, a.told, a.tnew, S.lng, S.longq, true, false);
+  apply_kept<kSelBlock>(s, nb, K, [&](int q) { return sk[q]; }, a.told, a.tnew, S.lng, S.longq, true);
   if (tid == 0) {
     s.info[MLP_INFO_KEPT0 + nb] = K;
     s.info[MLP_INFO_ROUND_MOVES] += K;
@@ -1636,7 +1845,7 @@ __global__ __launch_bounds__(kBlock) void k_total_merge(const SlotDev* __restric
                                                         const int32_t* __restrict__ ve) {
   extern __shared__ int64_t lds[];
   __shared__ TotalLds T;
-  __shared__ PrepLds PL;
+  __shared__ PrepWaves<kBlock> PL;
   const SlotDev& s = table[id];
   const int N = s.N, tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const int k = nb_k(nb);
@@ -1733,11 +1942,12 @@ __global__ __launch_bounds__(kBlock) void k_total_merge(const SlotDev* __restric
   }
   const int K = T.kept;
   const int32_t* kij = s.kept_ij[nb];
-  apply_kept(
+  apply_kept<kBlock>(
       s, nb, K,
       [&](int q) { return ((int64_t)kij[3 * q] << 32) | (uint32_t)kij[3 * q + 1]; }, told, tnew,
       T.nlong, T.longq);
-  prep_wg(s, tnew, PL);
+  __syncthreads();
+  prep_tour<kBlock, 8>(s, tnew, PL, nullptr, s.tour, false);
   if (tid == 0) {
     s.info[MLP_INFO_KEPT0 + nb] = K;
     s.info[MLP_INFO_ROUND_MOVES] += K;
@@ -3137,7 +3347,7 @@ template <int R, int C>
 __global__ __launch_bounds__(kBlock) void k_dvnd_fused(const SlotDev* __restrict__ table,
                                                        FusedPlan P) {
   extern __shared__ int64_t dyn[];
-  __shared__ MergeShared MS;
+  __shared__ MergeShared<kBlock> MS;
   __shared__ int s_item;
   SweepLds<R, C, kPlain>& L = *reinterpret_cast<SweepLds<R, C, kPlain>*>(dyn);
   int32_t* work = P.sync;
@@ -3166,7 +3376,7 @@ __global__ __launch_bounds__(kBlock) void k_dvnd_fused(const SlotDev* __restrict
       }
       wait_at_least(merged + q, rr * MLP_NB_COUNT + nb, timeout);
       wait_at_least(done + q, rr * all + upto, timeout);
-      merge_slot(table[P.slots[q]], nb, 0, P.pcap, P.ncap, 1,
+      merge_slot<kBlock, 8>(table[P.slots[q]], nb, 0, P.pcap, P.ncap, 1,
                         nb == MLP_NB_COUNT - 1 ? P.tail : 0, dyn, MS);
       signal_done(merged + q);
     } else {  // up to P.group tiles of the evaluation of nb for slot q
@@ -3237,8 +3447,14 @@ MLP_SWEEP_INST(4, 512, kOdc)
 #include "mlp_launch.h"
 
 hipError_t mlp_launch_prep(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
-                           const int32_t* list_dev, int count) {
-  hipLaunchKernelGGL(k_prep, dim3(count), dim3(kBlock), 0, st, table, inl, list_dev);
+                           const int32_t* list_dev, int count, int max_n) {
+#define MLP_PREP(TB, PER)                                                                     \
+  hipLaunchKernelGGL((k_prep<TB, PER>), dim3(count), dim3(TB), 0, st, table, inl, list_dev)
+  if (max_n <= 256) MLP_PREP(256, 1);
+  else if (max_n <= 1024) MLP_PREP(1024, 1);
+  else if (max_n <= 2048) MLP_PREP(1024, 2);
+  else MLP_PREP(1024, 4);
+#undef MLP_PREP
   return hipGetLastError();
 }
 
@@ -3359,9 +3575,24 @@ size_t mlp_merge_lds_bytes(int pcap, int ncap) {
 // sort buffer and the conflict bitmap of the largest N.
 constexpr size_t kGmemMergeLds = kGmemSortCap * 8 + claim_words(MLP_MAX_N) * 4;
 
+// The merge's workgroup for tours of up to n positions: as few positions a
+// thread as 1024 threads allow (its steps over the tour are one batch each).
+#define MLP_MERGE_FOR(n, F)          \
+  do {                               \
+    if ((n) <= 256) F(256, 1);       \
+    else if ((n) <= 512) F(512, 1);  \
+    else if ((n) <= 1024) F(1024, 1); \
+    else if ((n) <= 2048) F(1024, 2); \
+    else if ((n) <= 4096) F(1024, 4); \
+    else F(1024, 8);                 \
+  } while (0)
+
 hipError_t mlp_merge_setup(size_t max_dyn_lds) {
-  hipError_t e = hipFuncSetAttribute((const void*)k_merge_apply,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_dyn_lds);
+  hipError_t e = hipSuccess;
+#define MLP_MERGE_ATTR(TB, PER)                                                              \
+  e = hipFuncSetAttribute((const void*)k_merge_apply<TB, PER>,                               \
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_dyn_lds)
+  for (int n = 256; n <= 8192 && e == hipSuccess; n *= 2) MLP_MERGE_FOR(n, MLP_MERGE_ATTR);
   if (e == hipSuccess)
     e = hipFuncSetAttribute((const void*)k_mg_select, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)kGmemMergeLds);
@@ -3389,8 +3620,11 @@ hipError_t mlp_launch_fused(hipStream_t st, const SlotDev* table, const FusedPla
 hipError_t mlp_launch_merge_apply(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
                                   const int32_t* list_dev, int count, int nb, int rowmap,
                                   int pcap, int ncap, int skip_inactive, int tail) {
-  hipLaunchKernelGGL(k_merge_apply, dim3(count), dim3(kBlock), mlp_merge_lds_bytes(pcap, ncap), st,
-                     table, inl, list_dev, nb, rowmap, pcap, ncap, skip_inactive, tail);
+#define MLP_MERGE_LAUNCH(TB, PER)                                                             \
+  hipLaunchKernelGGL((k_merge_apply<TB, PER>), dim3(count), dim3(TB),                          \
+                     mlp_merge_lds_bytes(pcap, ncap), st, table, inl, list_dev, nb, rowmap, pcap, \
+                     ncap, skip_inactive, tail)
+  MLP_MERGE_FOR(ncap, MLP_MERGE_LAUNCH);
   return hipGetLastError();
 }
 
@@ -3400,7 +3634,7 @@ hipError_t mlp_launch_merge_gmem(hipStream_t st, const SlotDev* table, const Slo
   const dim3 seg((max_n + MLP_MG_CHUNK - 1) / MLP_MG_CHUNK, count);
   hipLaunchKernelGGL(k_mg_compact, seg, dim3(kBlock), 0, st, table, inl, list_dev, nb, rowmap,
                      skip_inactive);
-  hipLaunchKernelGGL(k_mg_select, dim3(count), dim3(kBlock), kGmemMergeLds, st, table, inl,
+  hipLaunchKernelGGL(k_mg_select, dim3(count), dim3(kSelBlock), kGmemMergeLds, st, table, inl,
                      list_dev, nb, rowmap, skip_inactive, tail);
   hipLaunchKernelGGL(k_mg_sums, seg, dim3(kBlock), 0, st, table, inl, list_dev);
   hipLaunchKernelGGL(k_mg_rebuild, seg, dim3(kBlock), 0, st, table, inl, list_dev,
@@ -3415,7 +3649,7 @@ size_t mlp_total_merge_lds_bytes(int N) {
 // The merge kernel's own static LDS (chunk arrays, prefix scratch) is below
 // kTotalStaticLds; its dynamic part may use the rest.
 constexpr size_t kTotalStaticLds = 48 * 1024;
-static_assert(sizeof(TotalLds) + sizeof(PrepLds) <= kTotalStaticLds, "static LDS estimate");
+static_assert(sizeof(TotalLds) + sizeof(PrepWaves<kBlock>) <= kTotalStaticLds, "static LDS estimate");
 
 size_t mlp_total_static_lds() { return kTotalStaticLds; }
 

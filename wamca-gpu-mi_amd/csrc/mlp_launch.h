@@ -8,8 +8,9 @@
 
 #include "mlp_internal.h"
 
+// max_n: the largest N among the slots.
 hipError_t mlp_launch_prep(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
-                           const int32_t* list_dev, int count);
+                           const int32_t* list_dev, int count, int max_n);
 hipError_t mlp_launch_dvnd_start(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
                                  const int32_t* list_dev, int count);
 hipError_t mlp_launch_round_begin(hipStream_t st, const SlotDev* table, const SlotListInline& inl,

@@ -895,7 +895,9 @@ int mlp_set_tours(mlp_ctx* ctx, const int32_t* slots, int32_t count, const int32
     const int32_t* dev = nullptr;
     st = slot_list(ctx, slots + q0, c, inl, &dev);
     if (st) return st;
-    HCK(mlp_launch_prep(ctx->stream, ctx->d_table, inl, dev, c));
+    int max_n = 0;
+    for (int q = q0; q < q0 + c; ++q) max_n = std::max(max_n, ctx->slots[slots[q]].N);
+    HCK(mlp_launch_prep(ctx->stream, ctx->d_table, inl, dev, c, max_n));
   }
   return MLP_OK;
 }
@@ -2557,7 +2559,7 @@ int mlp_eval_static(mlp_ctx* ctx, int32_t inst, const int32_t* tour, uint32_t nb
   HCK(mlp_launch_slot_init(ctx->stream, table, 0, d, (int64_t*)b, (int64_t)(L.ms / 8), rows));
   SlotListInline one{};
   one.id[0] = 0;
-  HCK(mlp_launch_prep(ctx->stream, table, one, nullptr, 1));
+  HCK(mlp_launch_prep(ctx->stream, table, one, nullptr, 1, N));
   // every neighborhood writes buffer 1 (the first tile records it)
   int total_rows = 0;
   for (int nb = 0; nb < MLP_NB_COUNT; ++nb)
