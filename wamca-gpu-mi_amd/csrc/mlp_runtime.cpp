@@ -2159,6 +2159,13 @@ int run_grouped(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int m
   return st;
 }
 
+// Rounds of an mlp_dvnd call's next chunk after `done` ones: none beyond
+// max_rounds, which would be launches over slots that have all stopped (256
+// tours n = 784, one round: 30 of 40 launches, 1.82 ms against 1.62).
+int chunk_rounds(const mlp_ctx* ctx, int max_rounds, int done) {
+  return max_rounds > 0 ? std::max(1, std::min(ctx->dvnd_chunk, max_rounds - done)) : ctx->dvnd_chunk;
+}
+
 // Rounds after `done` ones of an mlp_dvnd call that may leave out rows that
 // do not improve: all but the one that max_rounds makes the last, whose rows
 // the caller can read (those of a round that applied nothing are completed
@@ -2199,9 +2206,10 @@ int dvnd_independent(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap,
     for (int g = 0; g < groups && !st; ++g)
       if (!pending[g] && !part[g].empty()) {
         ctx->stream = g ? ctx->stream_grp[g] : ctx->stream_main;
-        st = run_chunk(ctx, part[g].data(), (int)part[g].size(), rowmap, max_rounds,
-                       ctx->dvnd_chunk, prunable(max_rounds, done[g]), false, g);
-        done[g] += ctx->dvnd_chunk;
+        const int rounds = chunk_rounds(ctx, max_rounds, done[g]);
+        st = run_chunk(ctx, part[g].data(), (int)part[g].size(), rowmap, max_rounds, rounds,
+                       prunable(max_rounds, done[g]), false, g);
+        done[g] += rounds;
         if (!st && hipEventRecord(ctx->ev_chunk[g], ctx->stream) != hipSuccess)
           st = fail(ctx, MLP_EDEVICE, "DVND chunk event");
         pending[g] = !st;
@@ -2345,9 +2353,9 @@ int mlp_dvnd(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
   int done = 0;
   while (!active.empty()) {
     const int c = (int)active.size();
-    st = run_grouped(ctx, active.data(), c, rowmap, max_rounds, ctx->dvnd_chunk,
-                     prunable(max_rounds, done));
-    done += ctx->dvnd_chunk;
+    const int rounds = chunk_rounds(ctx, max_rounds, done);
+    st = run_grouped(ctx, active.data(), c, rowmap, max_rounds, rounds, prunable(max_rounds, done));
+    done += rounds;
     if (st) return st;
     st = mlp_dvnd_status(ctx, active.data(), c, flag.data(), nullptr);
     if (st) return st;
