@@ -53,11 +53,16 @@ struct BlkSum {
   int32_t lo, hi, wmax, wpair;
 };
 
+// maxd - 1 bounds the real distances (mlp_runtime.cpp check_instance): up to
+// this maxd every dx^2 + dy^2 <= 1448^2 < 2^21.
+#define MLP_SMALL_MAXD 1449
+
 struct SlotDev {
   int32_t N;      // positions (n + 1)
   int32_t n;      // clients
   int32_t round;  // 0 trunc, 1 nint
   int32_t maxd;   // upper bound of any distance in the instance
+  int32_t small;  // every squared distance is below 2^21 (short distance form)
   int32_t rowcap; // entries per row buffer (rows[nb] holds two buffers)
   const int32_t* xs;  // instance coordinates (client indexed)
   const int32_t* ys;

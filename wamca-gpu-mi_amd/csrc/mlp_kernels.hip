@@ -79,6 +79,37 @@ __device__ __forceinline__ int dist_xy(int a, int b, float dr) {
   return dist_s(__builtin_amdgcn_sdot2(d, d, 0, false), dr);
 }
 
+// The same distance for s < 2^21 (instances up to MLP_SMALL_MAXD): there float(s) is exact and the reference's rounded expression
+// equals isqrt(s) (truncated) and the integer nearest sqrt(s) (rounded: for
+// m < 2048 the float below m + 0.5 nearest sqrt(m^2 + m) is not m + 0.5).
+// sqrt(s + 1/2) and sqrt(s - 1/4) + 1/2 keep a distance of at least 1 / (4 m)
+// > 2^-13 from every integer between two results, more than the hardware
+// estimate's one ulp (2^-13 up to m = 1448), so no correction is needed: 7
+// instructions instead of 14.  |s - 1/4 + 2^-10| stands for s = 0 (0.2490:
+// distance 0).  mlp_sqrt_selfcheck compares every s < 2^21 in both modes.
+// Side by side: DVND n = 1000 7.48 -> 7.12 ms, one tour n = 1000 (with its
+// prefix build and row output) 17.9 -> 17.5 us, 8 tours n = 4001 512 -> 500 us.
+constexpr int kSmallS = 1 << 21;
+struct FastDist {
+  float c0, c1;
+  __device__ __forceinline__ int operator()(int s) const {
+    return (int)(__builtin_amdgcn_sqrtf(__builtin_fabsf((float)(uint32_t)s + c0)) + c1);
+  }
+};
+__device__ __forceinline__ FastDist fast_dist(int round) {
+  return round ? FastDist{-0.2490234375F, 0.5F} : FastDist{0.5F, 0.0F};
+}
+// Distances of a tile: Dist is FastDist or the general form.
+struct FullDist {
+  float dr;
+  __device__ __forceinline__ int operator()(int s) const { return dist_s(s, dr); }
+};
+template <typename Dist>
+__device__ __forceinline__ int dist_by(int a, int b, const Dist& D) {
+  const short2v d = __builtin_bit_cast(short2v, a) - __builtin_bit_cast(short2v, b);
+  return D(__builtin_amdgcn_sdot2(d, d, 0, false));
+}
+
 // ---------------------------------------------------------------------------
 // row maps (the reference's launch grids and thread -> move maps, tour = 1)
 // ---------------------------------------------------------------------------
@@ -2079,6 +2110,11 @@ __global__ void k_sqrt_selfcheck(uint32_t s0, uint32_t count, unsigned long long
   for (uint32_t q = base; q < count; q += stride) {
     const float f = (float)(s0 + q);
     nb += (__float_as_uint(sqrt_rn_int(f)) != __float_as_uint(__builtin_sqrtf(f))) ? 1ull : 0ull;
+    // the short distance where it is used, in both rounding modes
+    const int si = (int)(s0 + q);
+    if (s0 + q < (uint32_t)kSmallS)
+      nb += (fast_dist(0)(si) != dist_s(si, 0.0F) ? 1ull : 0ull) +
+            (fast_dist(1)(si) != dist_s(si, 0.5F) ? 1ull : 0ull);
   }
   if (nb) atomicAdd(bad, nb);
 }
@@ -2831,17 +2867,21 @@ __device__ __forceinline__ void sweep_fixed(const SlotDev& s, int rb, int ct, in
   }
   // swap alone covers j >= i + 2 only: a tile left of that diagonal is empty
   if (mask == 1 && q1 <= b0 + 3) return;
+  auto fill = [&](const auto& dist) {
 #pragma unroll
-  for (int it = 0; it < FI; ++it) {
-    const int c = cfill + tid + it * kBlock;
-    if (c < cend) {
+    for (int it = 0; it < FI; ++it) {
+      const int c = cfill + tid + it * kBlock;
+      if (c < cend) {
 #pragma unroll
-      for (int va = 0; va < R + 4; ++va) L.v[va][c - cbase] = (uint16_t)dist_xy(xa[va], xc[it], dr);
-      L.w[c - cbase] = (uint16_t)wv[it];
-      L.t[c - cbase] = tv[it];
-      if constexpr (TWO) F.two.h[c - cbase] = hv[it];
+        for (int va = 0; va < R + 4; ++va) L.v[va][c - cbase] = (uint16_t)dist_by(xa[va], xc[it], dist);
+        L.w[c - cbase] = (uint16_t)wv[it];
+        L.t[c - cbase] = tv[it];
+        if constexpr (TWO) F.two.h[c - cbase] = hv[it];
+      }
     }
-  }
+  };
+  if (s.small) fill(fast_dist(s.round));
+  else fill(FullDist{dr});
   if (tid < R + 8) {
     L.rw[tid] = rwv;
     L.rt[tid] = rtv;
@@ -3027,31 +3067,35 @@ __device__ __forceinline__ void sweep_2opt(const SlotDev& s, int rb, int ct, int
   }
   if (ct == 0 && !(parity & kNoReset))
     reset_other(s, 1, par, rb * MLP_2OPT_ROWS, min(rb * MLP_2OPT_ROWS + MLP_2OPT_ROWS, rows), rb == 0);
-  if constexpr (FLAT) {
-    if (net > 0) {
-#pragma unroll
-      for (int it = 0; it < FI; ++it) {
-        const int x = lane + it * kWave;
-        if (x < net) {
-          const bool p1 = x >= ne0;
-          L.e[wave][p1 ? 1 : 0][p1 ? x - ne0 : x] = (uint16_t)dist_xy(pa[0][it], pb[0][it], dr);
-        }
-      }
-    }
-  } else {
-#pragma unroll
-    for (int part = 0; part < FP; ++part) {
-      const int ne = part ? ne1 : ne0;
-      uint16_t* e = L.e[wave][part];
-      if (ne >= 2) {
+  auto fill = [&](const auto& dist) {
+    if constexpr (FLAT) {
+      if (net > 0) {
 #pragma unroll
         for (int it = 0; it < FI; ++it) {
           const int x = lane + it * kWave;
-          if (x < ne) e[x] = (uint16_t)dist_xy(pa[part][it], pb[part][it], dr);
+          if (x < net) {
+            const bool p1 = x >= ne0;
+            L.e[wave][p1 ? 1 : 0][p1 ? x - ne0 : x] = (uint16_t)dist_by(pa[0][it], pb[0][it], dist);
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int part = 0; part < FP; ++part) {
+        const int ne = part ? ne1 : ne0;
+        uint16_t* e = L.e[wave][part];
+        if (ne >= 2) {
+#pragma unroll
+          for (int it = 0; it < FI; ++it) {
+            const int x = lane + it * kWave;
+            if (x < ne) e[x] = (uint16_t)dist_by(pa[part][it], pb[part][it], dist);
+          }
         }
       }
     }
-  }
+  };
+  if (s.small) fill(fast_dist(s.round));
+  else fill(FullDist{dr});
   __syncthreads();
   // A tour above the int32 bound can still have rows whose moves all stay
   // below 2^31: reversing positions i..j moves each reversed node's arrival

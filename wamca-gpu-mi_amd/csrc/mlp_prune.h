@@ -333,12 +333,19 @@ __device__ __forceinline__ void prune_wave(const SlotDev& s, int b0, int ct, int
     if (g + 1 < groups) nx = load(g + 1);
     const int c = o.c;
     const uint32_t nc = (uint32_t)(N - c);
-    int own[NA];
+    // own[a]: distance of row position a to the lane's column; hl, hr: of row
+    // position lane % 16 to the columns beyond the block's edges
+    int own[NA], hl, hr = 0;
+    auto dists = [&](const auto& dist) {
 #pragma unroll
-    for (int a = A0; a < NA; ++a) own[a] = dist_xy(xa[a], o.xy, dr);
+      for (int a = A0; a < NA; ++a) own[a] = dist_by(xa[a], o.xy, dist);
+      hl = dist_by(rxy, o.xl, dist);
+      if constexpr (NB == 0) hr = dist_by(rxy, o.xr, dist);
+    };
+    if (s.small) dists(fast_dist(s.round));
+    else dists(FullDist{dr});
     // left[a]: distance of row position a to the column on the left; the
     // block's first lane takes it from lane a, which computed row a's
-    const int hl = dist_xy(rxy, o.xl, dr);
     int left[NA];
 #define MLP_LEFT(A)                                                                          \
   if constexpr ((A) >= A0 && (A) < NA)                                                       \
@@ -348,7 +355,6 @@ __device__ __forceinline__ void prune_wave(const SlotDev& s, int b0, int ct, int
 #undef MLP_LEFT
     int right[kPR + 1];
     if constexpr (NB == 0) {
-      const int hr = dist_xy(rxy, o.xr, dr);
 #define MLP_RIGHT(A)                                                                         \
   right[A] = __builtin_amdgcn_update_dpp(row_shr<15 - (A)>(hr), own[A], 0x101, 0xf, 0xf, false);
       MLP_RIGHT(1) MLP_RIGHT(2) MLP_RIGHT(3) MLP_RIGHT(4) MLP_RIGHT(5) MLP_RIGHT(6) MLP_RIGHT(7)

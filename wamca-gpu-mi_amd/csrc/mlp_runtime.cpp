@@ -793,6 +793,7 @@ int mlp_slot_create(mlp_ctx* ctx, int32_t inst, int32_t* slot) {
   d.n = in.n;
   d.round = in.round;
   d.maxd = in.maxd;
+  d.small = in.maxd <= MLP_SMALL_MAXD;
   d.rowcap = row_cap(N);
   d.xs = in.xs;
   d.ys = in.ys;
@@ -2537,6 +2538,7 @@ int mlp_eval_static(mlp_ctx* ctx, int32_t inst, const int32_t* tour, uint32_t nb
   d.n = in.n;
   d.round = in.round;
   d.maxd = in.maxd;
+  d.small = in.maxd <= MLP_SMALL_MAXD;
   d.rowcap = row_cap(N);
   d.xs = in.xs;
   d.ys = in.ys;
