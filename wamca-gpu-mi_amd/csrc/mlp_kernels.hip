@@ -984,21 +984,22 @@ __device__ __forceinline__ bool conflicts_kind(int k, int i1, int j1, int i2, in
   return ((int)(max(i1, j1) + k < min(i2, j2)) | (int)(min(i1, j1) > max(i2, j2) + k)) == 0;
 }
 
-// Greedy over the M candidates sorted by (cost, row), on one wave, 64 at a
-// time.  The bitmap of positions claimed by kept moves is an exact conflict
-// test against every move kept so far (swap: positions i-1..i+1, j-1..j+1;
-// 2-opt: [i, j+1]; or-opt: [min(i,j), max(i,j)+k]); within a batch the
-// candidates that pass it are decided in order by a scalar loop over the
-// kept ones.  Kept moves go to keys[q]
-// as (i << 32 | j) and to the slot's kept arrays.  Returns their count.
+// Greedy over the M candidates keys[0..M) sorted by (cost, row), on one wave,
+// 64 at a time.  The bitmap of positions claimed by kept moves is an exact
+// conflict test against every move kept so far (swap: positions i-1..i+1,
+// j-1..j+1; 2-opt: [i, j+1]; or-opt: [min(i,j), max(i,j)+k]); within a batch
+// the candidates that pass it are decided in order by a scalar loop over the
+// kept ones.  The kept moves follow the kept0 ones of earlier calls: to
+// out[q] as (i << 32 | j) (out may be keys: kept moves overwrite only keys of
+// decided batches) and to the slot's kept arrays.  Returns their count.
 // Candidates from index `tail` on are read from gtail (a sort whose keys
-// exceed the LDS buffer); kept moves are written below `tail`.  The next
-// batch's keys and ctx and the key after it are read while a batch is
-// decided (kept moves overwrite only keys of decided batches).
+// exceed the LDS buffer).  The next batch's keys and ctx and the key after it
+// are read while a batch is decided.
 template <int KIND>
 __device__ __forceinline__ int greedy_wave(const SlotDev& s, int nb, int N, int rowmap, int M,
-                                           int64_t* keys, const uint16_t* ctxL, uint32_t* bits,
-                                           int lane, const int64_t* gtail, int tail) {
+                                           const int64_t* keys, int64_t* out, int kept0,
+                                           const uint16_t* ctxL, uint32_t* bits, int lane,
+                                           const int64_t* gtail, int tail) {
   const int K = KIND == 2 ? nb - 1 : 0;
   auto key_at = [&](int t) -> int64_t {
     return t < M ? (t < tail ? keys[t] : ldg(gtail + t)) : MLP_KEY_NONE;
@@ -1013,7 +1014,7 @@ __device__ __forceinline__ int greedy_wave(const SlotDev& s, int nb, int N, int 
   int64_t skc = key_at(lane);
   int ctxc = ctx_at(lane, skc);
   int64_t skn = key_at(kWave + lane);
-  int kept_total = 0;
+  int kept_total = kept0;
   for (int base = 0; base < M; base += kWave) {
     const int t = base + lane;
     const bool valid = t < M;
@@ -1049,7 +1050,7 @@ __device__ __forceinline__ int greedy_wave(const SlotDev& s, int nb, int N, int 
         claims_set(bits, N, a, b);
       }
       const int q = kept_total + __popcll(kept & ((1ull << lane) - 1ull));
-      keys[q] = ((int64_t)i << 32) | (uint32_t)j;  // q <= t: already consumed
+      out[q] = ((int64_t)i << 32) | (uint32_t)j;
       kcost[q] = cost;
       kij[3 * q + 0] = i;
       kij[3 * q + 1] = j;
@@ -1296,34 +1297,322 @@ __device__ __forceinline__ void keys_to_global(int64_t* g, const int64_t* sb, in
 }
 
 // A merge whose working arrays are in global memory still sorts up to
-// kGmemSortCap improving rows in LDS; the rest of its dynamic LDS holds the
-// conflict bitmap.
+// kGmemSortCap improving rows in LDS and selects in kGmemBuf entries; the rest
+// of its dynamic LDS holds the conflict bitmap.
 constexpr int kGmemSortCap = 16384;
+constexpr int kGmemBuf = 18432;
 
 // The merge's small shared variables (counts, the long-move queue, the
 // prefix rebuild's scan carries).
+constexpr int kSelCap = 256;      // candidates of one greedy pass
+constexpr int kSelClasses = 512;  // cost classes of select_spans
 template <int TB>
 struct MergeShared {
   int m, kept, lng;
+  int cnt, top, cut, left;  // selection
   int longq[kLongMoves];
+  int hist[kSelClasses];    // candidates per class; ranks
+  int64_t list[kSelCap];
   PrepWaves<TB> PL;
 };
+static_assert(sizeof(MergeShared<1024>) <= 8192, "static LDS left beside the merge's dynamic part");
+
+// Sort of list[0..n), n <= 256, distinct keys: a key's rank is the number of
+// smaller keys, counted by TB / 256 threads a key (M reads of LDS broadcasts
+// against the 36 barrier phases of a bitonic sort of 256).
+template <int TB>
+__device__ __forceinline__ void rank_sort(int64_t* list, int n, int* rank) {
+  constexpr int G = TB / 256;
+  const int tid = threadIdx.x, e = tid & 255, g = tid >> 8;
+  const int64_t my = e < n ? list[e] : 0;
+  int r = 0;
+  if constexpr (G > 1) {
+    if (tid < 256) rank[tid] = 0;
+    __syncthreads();
+  }
+  if (e < n) {
+    const int per = (n + G - 1) / G, u1 = min(n, per * (g + 1));
+    for (int u = per * g; u < u1; ++u) r += list[u] < my ? 1 : 0;
+    if constexpr (G > 1) atomicAdd(&rank[e], r);
+  }
+  __syncthreads();
+  if (g == 0 && e < n) list[G > 1 ? rank[e] : r] = my;
+  __syncthreads();
+}
+
+// Selection of the greedy subset without a sort of all M candidates: thread
+// tid looks after candidates t = tid + u TB (u < 32, a bit of `alive` each);
+// key(t) is t's (cost, row) key and move(t, key) its move (i << 16 | j), both
+// unchanged until the selection ends.
+//
+// select_spans, for the interval moves (2-opt, or-opt).  The best moves are
+// long and conflict with most others, so the candidates are taken in slices
+// of the best 256 or fewer (by classes of the cost's magnitude, 32 an octave,
+// counted in LDS): sort the slice, greedy on wave 0, then every thread drops
+// those of its candidates that now conflict.  A slice ends between classes,
+// so equal costs stay together and the order is that of the whole sort.
+// Returns -1 (no claims left) when one class exceeds a slice.  out: the kept
+// moves, at most N / 2 (a span claims at least two positions).
+template <int KIND, int TB, typename Key, typename Move>
+__device__ __forceinline__ int select_spans(const SlotDev& s, int nb, int N, int rowmap, int M, Key key,
+                                            Move move, int64_t* out, const uint16_t* ctxL,
+                                            uint32_t* bits, MergeShared<TB>& S) {
+  const int tid = threadIdx.x, lane = tid % kWave, K = KIND == 2 ? nb - 1 : 0;
+  // class of a key: the float bits of -cost down to 5 of the mantissa
+  auto cls = [](int64_t v) { return __float_as_int((float)(-(v >> MLP_KEY_SHIFT))) >> 18; };
+  uint32_t alive = 0;
+  int mx = 0;
+#pragma unroll 1
+  for (int u = 0; tid + u * TB < M; ++u) {
+    alive |= 1u << u;
+    mx = max(mx, cls(key(tid + u * TB)));
+  }
+  if (tid == 0) S.top = S.cnt = 0;
+  __syncthreads();
+  mx = wave_max_i32(mx);
+  if (lane == 0) atomicMax(&S.top, mx);
+  int left = M, kept = 0;
+  for (;;) {
+    int top = 0, cut = 0;
+    if (left > kSelCap) {
+      for (int b = tid; b < kSelClasses; b += TB) S.hist[b] = 0;
+      __syncthreads();
+      top = S.top;
+#pragma unroll 1
+      for (uint32_t m = alive; m; m &= m - 1) {
+        const int64_t k = key(tid + __builtin_ctz(m) * TB);
+        atomicAdd(&S.hist[min(top - cls(k), kSelClasses - 1)], 1);
+      }
+      __syncthreads();
+      if (tid < kWave) {  // the classes whose cumulative count fits a slice
+        constexpr int PB = kSelClasses / kWave;
+        int c[PB], sum = 0, in = 0;
+#pragma unroll
+        for (int b = 0; b < PB; ++b) {
+          sum += S.hist[lane * PB + b];
+          c[b] = sum;
+        }
+        const int before = wave_scan_i32(sum) - sum;
+#pragma unroll
+        for (int b = 0; b < PB; ++b) in += before + c[b] <= kSelCap ? 1 : 0;
+        in = wave_scan_i32(in);
+        if (lane == kWave - 1) S.cut = in - 1;
+      }
+      __syncthreads();
+      cut = S.cut;
+      if (cut < 0) {
+        for (int w = tid; w < claim_words(N); w += TB) bits[w] = 0;
+        __syncthreads();
+        return -1;
+      }
+    }
+#pragma unroll 1
+    for (uint32_t m = alive; m; m &= m - 1) {
+      const int u = __builtin_ctz(m);
+      const int64_t k = key(tid + u * TB);
+      if (left <= kSelCap || min(top - cls(k), kSelClasses - 1) <= cut) {
+        S.list[atomicAdd(&S.cnt, 1)] = k;
+        alive &= ~(1u << u);
+      }
+    }
+    __syncthreads();
+    const int n = S.cnt;
+    rank_sort<TB>(S.list, n, S.hist);
+    if (tid < kWave) {
+      const int kk = greedy_wave<KIND>(s, nb, N, rowmap, n, S.list, out, kept, ctxL, bits, lane,
+                                       nullptr, INT32_MAX);
+      if (lane == 0) {
+        S.kept = kk;
+        S.cnt = S.top = S.left = 0;
+      }
+    }
+    __syncthreads();
+    kept = S.kept;
+    left -= n;
+    if (left == 0) break;
+    mx = 0;
+#pragma unroll 1
+    for (uint32_t m = alive; m; m &= m - 1) {
+      const int u = __builtin_ctz(m);
+      const int64_t k = key(tid + u * TB);
+      const int ij = move(tid + u * TB, k), i = ij >> 16, j = ij & 0xffff;
+      if (claims_any(bits, N, KIND == 1 ? i : min(i, j), KIND == 1 ? j + 1 : max(i, j) + K))
+        alive &= ~(1u << u);
+      else mx = max(mx, cls(k));
+    }
+    const int c = wave_scan_i32(__popc(alive));  // lane 63: the wave's
+    mx = wave_max_i32(mx);
+    if (lane == kWave - 1 && c) {
+      atomicMax(&S.top, mx);
+      atomicAdd(&S.left, c);
+    }
+    __syncthreads();
+    left = S.left;
+    if (left == 0) break;
+  }
+  return kept;
+}
+
+// select_swaps: a swap conflicts only with swaps that have an end within one
+// position of one of its ends, so the candidates decide among themselves, many
+// at a time: the best key at each position (pm, an LDS minimum), then a
+// candidate that is the best at its ends' six positions is kept (nothing
+// before it in the order can conflict), its positions are claimed and the
+// others that touch them leave.  This keeps exactly what the greedy in order
+// keeps; the kept ones are sorted at the end for the list.  Returns -1 as
+// select_spans does when kSwapRounds rounds leave candidates (a chain of
+// conflicts in the order of the costs).  pm: max(N, 512) entries; the kept
+// moves end there.
+constexpr int kSwapRounds = 24;
+template <int TB, typename Key, typename Move>
+__device__ __forceinline__ int select_swaps(const SlotDev& s, int N, int rowmap, int M, Key key,
+                                            Move move, int64_t* pm, const uint16_t* ctxL,
+                                            uint32_t* bits, MergeShared<TB>& S) {
+  const int tid = threadIdx.x;
+  uint32_t alive = 0, keep = 0;
+  for (int u = 0; tid + u * TB < M; ++u) alive |= 1u << u;
+  if (tid == 0) S.cnt = 0;
+  for (int p = tid; p < N; p += TB) pm[p] = MLP_KEY_NONE;
+  __syncthreads();
+  bool more = true;
+  for (int round = 0; round < kSwapRounds && more; ++round) {
+#pragma unroll 1
+    for (uint32_t m = alive; m; m &= m - 1) {
+      const int t = tid + __builtin_ctz(m) * TB;
+      const int64_t k = key(t);
+      const int ij = move(t, k);
+      atomicMin((long long*)&pm[ij >> 16], (long long)k);
+      atomicMin((long long*)&pm[ij & 0xffff], (long long)k);
+    }
+    __syncthreads();
+    uint32_t win = 0;
+#pragma unroll 1
+    for (uint32_t m = alive; m; m &= m - 1) {
+      const int u = __builtin_ctz(m), t = tid + u * TB;
+      const int64_t k = key(t);
+      const int ij = move(t, k), i = ij >> 16, j = ij & 0xffff;  // 1 <= i, j <= N - 2
+      const int64_t a = min(min(pm[i - 1], pm[i]), pm[i + 1]);
+      const int64_t b = min(min(pm[j - 1], pm[j]), pm[j + 1]);
+      if (min(a, b) == k) win |= 1u << u;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (uint32_t m = alive; m; m &= m - 1) {
+      const int u = __builtin_ctz(m), t = tid + u * TB;
+      const int ij = move(t, key(t)), i = ij >> 16, j = ij & 0xffff;
+      pm[i] = pm[j] = MLP_KEY_NONE;
+      if ((win >> u) & 1u) {
+        claims_set(bits, N, i - 1, i + 1);
+        claims_set(bits, N, j - 1, j + 1);
+      }
+    }
+    keep |= win;
+    alive &= ~win;
+    __syncthreads();
+#pragma unroll 1
+    for (uint32_t m = alive; m; m &= m - 1) {
+      const int u = __builtin_ctz(m), t = tid + u * TB;
+      const int ij = move(t, key(t));
+      if ((int)claimed(bits, N, ij >> 16) | (int)claimed(bits, N, ij & 0xffff)) alive &= ~(1u << u);
+    }
+    more = __syncthreads_or(alive != 0) != 0;
+  }
+  if (more) {
+    for (int w = tid; w < claim_words(N); w += TB) bits[w] = 0;
+    __syncthreads();
+    return -1;
+  }
+#pragma unroll 1
+  for (uint32_t m = keep; m; m &= m - 1) pm[atomicAdd(&S.cnt, 1)] = key(tid + __builtin_ctz(m) * TB);
+  __syncthreads();
+  const int n = S.cnt;
+  if (n <= kSelCap) rank_sort<TB>(pm, n, S.hist);
+  else bitonic_keys<TB>(pm, n);
+  int64_t* const kcost = s.kept_cost[0];
+  int32_t* const kij = s.kept_ij[0];
+#pragma unroll 1
+  for (int q = tid; q < n; q += TB) {
+    const int64_t k = pm[q];
+    const int row = (int)(k & MLP_KEY_MASK);
+    int i, j;
+    move_ij(0, rowmap, N, row, (int)ctxL[row], i, j);
+    pm[q] = ((int64_t)i << 32) | (uint32_t)j;
+    kcost[q] = k >> MLP_KEY_SHIFT;
+    kij[3 * q + 0] = i;
+    kij[3 * q + 1] = j;
+    kij[3 * q + 2] = row;
+  }
+  __syncthreads();
+  return n;
+}
 
 // 2.-3. of a merge: sort of the M improving (cost, row) keys == stable sort
-// by cost of the row list, then the greedy filter on wave 0.  Returns the
-// kept count; sk points at the sorted keys, whose first entries then hold the
-// kept moves as (i << 32 | j).
+// by cost of the row list, then the greedy filter on wave 0; or the same
+// subset from a selection.  Returns the kept count; sk points at LDS or the
+// keys, whose first entries then hold the kept moves as (i << 32 | j).
+// cap: entries of the LDS buffer (the keys' own, or at lds when GMEM); a
+// selection runs where it holds what the selection needs.
+// Swaps are selected from 65 candidates on, spans from 257 on (a slice).
+// First merges of a solve, whole sort and serial greedy before and now:
+// n = 9001 swap 320 -> 108 us, 2-opt 116 -> 35; n up to 2000 swap 63 -> 42,
+// or-opt 50 -> 25; n = 1000 swap 30 -> 27, or-opt 24 -> 19.
 template <bool GMEM, int TB>
 __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap, int N, int M,
-                                           int64_t* keys, int64_t* lds, const uint16_t* ctxL,
+                                           int64_t* keys, int64_t* lds, int cap, const uint16_t* ctxL,
                                            uint32_t* bits, MergeShared<TB>& S, int64_t*& sk) {
   const int tid = threadIdx.x;
   const int64_t* gtail = nullptr;  // sorted keys beyond the LDS buffer
   int tail = INT32_MAX;
+  const int64_t* in = keys;
+  if constexpr (TB >= 512) {
+    int kept = -1;
+    auto decode = [&](int64_t key) {
+      const int row = (int)(key & MLP_KEY_MASK);
+      int i, j;
+      move_ij(nb, rowmap, N, row, (int)ctxL[row], i, j);
+      return (i << 16) | j;
+    };
+    if constexpr (GMEM) {
+      // the moves (and the spans' keys) in LDS, so that no pass gathers
+      // them from global memory again
+      const bool swaps = nb == 0 && M > kWave && 2 * N + M <= 2 * kGmemBuf;
+      const bool spans = nb > 0 && M > kSelCap && 3 * M + N + 2 <= 2 * kGmemBuf;
+      if (swaps || spans) {
+        int32_t* const lij = (int32_t*)(lds + (swaps ? N : M + (N + 1) / 2));
+        for (int t = tid; t < M; t += TB) {
+          const int64_t key = ldg(keys + t);
+          if (spans) lds[t] = key;
+          lij[t] = decode(key);
+        }
+        __syncthreads();
+        auto move = [&](int t, int64_t) { return lij[t]; };
+        auto lkey = [&](int t) { return lds[t]; };
+        sk = swaps ? lds : lds + M;
+        if (swaps)
+          kept = select_swaps<TB>(s, N, rowmap, M, [&](int t) { return ldg(keys + t); }, move, sk,
+                                  ctxL, bits, S);
+        else if (nb == 1)
+          kept = select_spans<1, TB>(s, nb, N, rowmap, M, lkey, move, sk, ctxL, bits, S);
+        else kept = select_spans<2, TB>(s, nb, N, rowmap, M, lkey, move, sk, ctxL, bits, S);
+      }
+    } else {
+      auto move = [&](int, int64_t key) { return decode(key); };
+      auto lkey = [&](int t) { return keys[t]; };
+      sk = keys + M;
+      if (nb == 0 && M > kWave && M + max(N, kSortSeg) <= cap)
+        kept = select_swaps<TB>(s, N, rowmap, M, lkey, move, sk, ctxL, bits, S);
+      else if (nb == 1 && M > kSelCap && M + N / 2 <= cap)
+        kept = select_spans<1, TB>(s, nb, N, rowmap, M, lkey, move, sk, ctxL, bits, S);
+      else if (nb > 1 && M > kSelCap && M + N / 2 <= cap)
+        kept = select_spans<2, TB>(s, nb, N, rowmap, M, lkey, move, sk, ctxL, bits, S);
+    }
+    if (kept >= 0) return kept;
+  }
+  sk = GMEM && M <= cap ? lds : keys;
   // Up to one key per lane of a wave, keys in LDS: rank sort on wave 0, which
   // also runs the greedy next (the keys are distinct; a key's rank is the
   // number of smaller keys; every lane reads all keys before any lane
-  // writes).  Otherwise a bitonic sort over the workgroup.
+  // writes).  Up to 256 the same over the workgroup, else a bitonic sort.
   if (!GMEM && M <= kWave) {
     if (tid < kWave) {
       const int64_t my = tid < M ? keys[tid] : 0;
@@ -1333,17 +1622,11 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
       if (tid < M) keys[rank] = my;
       __builtin_amdgcn_wave_barrier();
     }
-  } else if (!GMEM && M <= 256) {
-    // one key per thread: the same rank sort over the workgroup (M reads of
-    // LDS broadcasts per thread against the 36 barrier phases of a bitonic
-    // sort of 256)
-    const int64_t my = tid < M ? keys[tid] : 0;
-    int rank = 0;
-    if (tid < M)
-      for (int u = 0; u < M; ++u) rank += keys[u] < my ? 1 : 0;
+  } else if (M <= kSelCap) {
+    if (tid < M) S.list[tid] = keys[tid];
     __syncthreads();
-    if (tid < M) keys[rank] = my;
-    __syncthreads();
+    rank_sort<TB>(S.list, M, S.hist);
+    in = S.list;
   } else if (GMEM && M <= kGmemSortCap) {
     // the slot's working arrays are in global memory, but its improving rows
     // fit the LDS sort buffer: sort them there, and let the greedy and the
@@ -1351,7 +1634,7 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
     int64_t* sb = lds;
     keys_to_lds<TB>(sb, keys, M, M);
     bitonic_keys<TB>(sb, M);
-    sk = sb;
+    in = sb;
   } else if (GMEM && M <= 2 * kGmemSortCap) {
     // twice the LDS buffer (keys[M..2 cap) in the slot's memory are padded):
     // the lower half sorted ascending and the upper half descending in LDS,
@@ -1390,7 +1673,7 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
         __syncthreads();
       }
     }
-    sk = sb;
+    in = sk = sb;
     gtail = keys;
     tail = H;
   } else {
@@ -1399,9 +1682,9 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
   // 3. greedy filter on wave 0
   if (tid < kWave) {
     int kept = 0;
-    if (nb == 0) kept = greedy_wave<0>(s, nb, N, rowmap, M, sk, ctxL, bits, tid, gtail, tail);
-    else if (nb == 1) kept = greedy_wave<1>(s, nb, N, rowmap, M, sk, ctxL, bits, tid, gtail, tail);
-    else if (nb < MLP_NB_MAX) kept = greedy_wave<2>(s, nb, N, rowmap, M, sk, ctxL, bits, tid, gtail, tail);
+    if (nb == 0) kept = greedy_wave<0>(s, nb, N, rowmap, M, in, sk, 0, ctxL, bits, tid, gtail, tail);
+    else if (nb == 1) kept = greedy_wave<1>(s, nb, N, rowmap, M, in, sk, 0, ctxL, bits, tid, gtail, tail);
+    else if (nb < MLP_NB_MAX) kept = greedy_wave<2>(s, nb, N, rowmap, M, in, sk, 0, ctxL, bits, tid, gtail, tail);
     if (tid == 0) S.kept = kept;
   }
   __syncthreads();
@@ -1504,7 +1787,7 @@ __device__ __forceinline__ void merge_slot(const SlotDev& s, int nb, int rowmap,
     }
     return;
   }
-  const int K = sort_greedy<false, TB>(s, nb, rowmap, N, M, keys, lds, ctxL, bits, S, sk);
+  const int K = sort_greedy<false, TB>(s, nb, rowmap, N, M, keys, lds, pcap, ctxL, bits, S, sk);
   // 4. apply the kept moves, rebuild the prefix arrays
   apply_kept<TB>(s, nb, K, [&](int q) { return sk[q]; }, told, tnew, S.lng, S.longq, true);
   __syncthreads();
@@ -1625,7 +1908,7 @@ __global__ __launch_bounds__(kSelBlock) void k_mg_select(const SlotDev* __restri
   const MgArrays a = mg_arrays(s);
   const int M = (int)s.info[MLP_INFO_MCOUNT];
   const int par = (int)(s.info[MLP_INFO_PARITY0 + nb] & 1) ^ (skip_inactive ? 1 : 0);
-  uint32_t* bits = (uint32_t*)(lds + kGmemSortCap);
+  uint32_t* bits = (uint32_t*)(lds + kGmemBuf);
   const int nwords = claim_words(N);
   for (int w = tid; w < nwords; w += kSelBlock) bits[w] = 0;
   __syncthreads();  // every thread has read the count and the parity
@@ -1642,7 +1925,8 @@ __global__ __launch_bounds__(kSelBlock) void k_mg_select(const SlotDev* __restri
     return;
   }
   int64_t* sk = a.keys;
-  const int K = sort_greedy<true, kSelBlock>(s, nb, rowmap, N, M, a.keys, lds, a.ctxL, bits, S, sk);
+  const int K = sort_greedy<true, kSelBlock>(s, nb, rowmap, N, M, a.keys, lds, kGmemSortCap, a.ctxL, bits, S,
+                                             sk);
   // tnew becomes the new tour; k_mg_rebuild copies it back
   apply_kept<kSelBlock>(s, nb, K, [&](int q) { return sk[q]; }, a.told, a.tnew, S.lng, S.longq, true);
   if (tid == 0) {
@@ -3617,7 +3901,8 @@ size_t mlp_merge_lds_bytes(int pcap, int ncap) {
 
 // Dynamic LDS of a merge whose working arrays are in global memory: the
 // sort buffer and the conflict bitmap of the largest N.
-constexpr size_t kGmemMergeLds = kGmemSortCap * 8 + claim_words(MLP_MAX_N) * 4;
+constexpr size_t kGmemMergeLds = kGmemBuf * 8 + claim_words(MLP_MAX_N) * 4;
+static_assert(kGmemMergeLds + sizeof(MergeShared<kSelBlock>) <= 160 * 1024, "LDS of a CU");
 
 // The merge's workgroup for tours of up to n positions: as few positions a
 // thread as 1024 threads allow (its steps over the tour are one batch each).

@@ -1621,6 +1621,13 @@ static int merge_impl(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t
     in_gmem.insert(in_gmem.end(), in_lds.begin(), in_lds.end());
     in_lds.clear();
   }
+  // room beside the keys for the selections of merges with many improving
+  // rows (a position array for swaps, the kept spans), where LDS has it
+  if (ncap > 256) {
+    int roomy = pcap;
+    while (roomy < ncap + std::max(ncap, 512)) roomy <<= 1;
+    if (mlp_merge_lds_bytes(roomy, ncap) <= ctx->max_merge_lds) pcap = roomy;
+  }
   for (int q = 0; q < count; ++q) ctx->slots[slots[q]].merged[nb] = true;
   if (ctx->user_capture)
     for (int q = 0; q < count; ++q) ctx->capture_ops.push_back({slots[q], 1, (uint32_t)nb, rowmap});
