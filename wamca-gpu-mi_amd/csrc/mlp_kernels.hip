@@ -66,14 +66,65 @@ __device__ __forceinline__ int dist_s(int s, float dr) {
 // Global-address-space load of a slot array element (the slot table stores
 // generic pointers; this keeps the access a global_load).
 template <typename T>
+using gptr = __attribute__((address_space(1))) T*;
+template <typename T>
 __device__ __forceinline__ T ldg(const T* p) {
-  return *(const __attribute__((address_space(1))) T*)p;
+  return *(gptr<const T>)p;
 }
+template <typename T>
+__device__ __forceinline__ T ldg(gptr<const T> p) {
+  return *p;
+}
+
+// A slot's table entry in scalar registers, for the kernels whose time is one
+// chain of latencies (merges, prefix build): every field is loaded at the
+// kernel's start in one batch, and the arrays are global pointers.  Through
+// the table, each group of fields was a vector load of its own just before
+// its first use (500 to 1000 cycles each, the stores in between keep the
+// compiler from reading them earlier), and the stores were flat ones.
+struct SlotRegs {
+  int N, n, round, maxd, small, rowcap;
+  gptr<const int32_t> xs, ys;
+  gptr<int32_t> tour, xy, w, t32, q32, g32, h32;
+  gptr<int64_t> t64, q64;
+  gptr<BlkSum> blk;
+  gptr<int64_t> info, rows, kcost;  // rows and kept moves of one neighborhood
+  gptr<int32_t> kij;
+};
+// The table entry does not change while such a kernel runs (the fused rounds'
+// launches included).
+__device__ __forceinline__ SlotRegs slot_regs(const SlotDev* table, int id, int nb) {
+  const auto* p = (const __attribute__((address_space(4))) SlotDev*)table +
+                  __builtin_amdgcn_readfirstlane(id);
+  SlotRegs r;
+  r.N = p->N; r.n = p->n; r.round = p->round; r.maxd = p->maxd; r.small = p->small;
+  r.rowcap = p->rowcap;
+#define MLP_FIELD(F) r.F = (decltype(r.F))p->F
+  MLP_FIELD(xs); MLP_FIELD(ys); MLP_FIELD(tour); MLP_FIELD(xy); MLP_FIELD(w); MLP_FIELD(t32);
+  MLP_FIELD(q32); MLP_FIELD(g32); MLP_FIELD(h32); MLP_FIELD(t64); MLP_FIELD(q64); MLP_FIELD(blk);
+  MLP_FIELD(info);
+#undef MLP_FIELD
+  r.rows = (gptr<int64_t>)p->rows[nb];
+  r.kcost = (gptr<int64_t>)p->kept_cost[nb];
+  r.kij = (gptr<int32_t>)p->kept_ij[nb];
+  // all of them are there before the first use of any
+  asm volatile("" : "+s"(r.xs), "+s"(r.ys), "+s"(r.tour), "+s"(r.xy), "+s"(r.w), "+s"(r.t32),
+               "+s"(r.q32), "+s"(r.g32), "+s"(r.h32), "+s"(r.t64), "+s"(r.q64));
+  asm volatile("" : "+s"(r.blk), "+s"(r.info), "+s"(r.rows), "+s"(r.kcost), "+s"(r.kij),
+               "+s"(r.N), "+s"(r.n), "+s"(r.round), "+s"(r.maxd), "+s"(r.rowcap));
+  return r;
+}
+__device__ __forceinline__ gptr<int64_t> slot_rows(const SlotRegs& s, int) { return s.rows; }
+__device__ __forceinline__ gptr<int64_t> kept_cost(const SlotRegs& s, int) { return s.kcost; }
+__device__ __forceinline__ gptr<int32_t> kept_ij(const SlotRegs& s, int) { return s.kij; }
 
 // Packed coordinates (x << 16 | y, x and y in [0, 32767]) as two signed
 // 16-bit lanes: one packed subtraction gives dx and dy exactly (|d| <= 32767)
 // and one 16-bit dot product dx^2 + dy^2 < 2^31 (v_pk_sub_i16, v_dot2).
 typedef short short2v __attribute__((ext_vector_type(2)));
+typedef int int4v __attribute__((ext_vector_type(4)));
+typedef int int2v __attribute__((ext_vector_type(2)));
+typedef int64_t long2v __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ int dist_xy(int a, int b, float dr) {
   const short2v d = __builtin_bit_cast(short2v, a) - __builtin_bit_cast(short2v, b);
   return dist_s(__builtin_amdgcn_sdot2(d, d, 0, false), dr);
@@ -113,6 +164,9 @@ __device__ __forceinline__ int dist_by(int a, int b, const Dist& D) {
 // ---------------------------------------------------------------------------
 // row maps (the reference's launch grids and thread -> move maps, tour = 1)
 // ---------------------------------------------------------------------------
+// 24-bit multiply, the product modulo 2^32
+__device__ __forceinline__ uint32_t umul(uint32_t a, uint32_t b) { return __umul24(a, b); }
+
 __device__ __forceinline__ int nb_k(int nb) { return nb >= 2 ? nb - 1 : 0; }
 
 __device__ __forceinline__ int rows_of(int nb, int rowmap, int N) {
@@ -421,8 +475,8 @@ __device__ __forceinline__ int64_t wave_sum64(int64_t v) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-template <int PER>
-__device__ __forceinline__ void put_summary(const SlotDev& s, int p0, const int (&xy)[PER + 2],
+template <int PER, typename Slot>
+__device__ __forceinline__ void put_summary(const Slot& s, int p0, const int (&xy)[PER + 2],
                                             const int (&w)[PER + 1]);
 
 struct PrepLds {
@@ -552,7 +606,8 @@ __device__ __forceinline__ void prep_segment(const SlotDev& s, const int32_t* to
 }
 
 // The tour's T[N-1] and int32-path flags.
-__device__ __forceinline__ void prep_flags(const SlotDev& s, int64_t Ttot) {
+template <typename Slot>
+__device__ __forceinline__ void prep_flags(const Slot& s, int64_t Ttot) {
   // Moves computed mod 2^32 are exact while |delta| < 2^31.  Node-wise:
   // a 2-opt reversal moves each reversed node's arrival by at most
   // Ttot + 2 maxd, so |delta| <= N (Ttot + 6 maxd) + 3 Ttot; a swap changes
@@ -623,8 +678,8 @@ __device__ __forceinline__ int group_max(int v) {
 // each (p0 on: packed coordinates of p0 - 1 .. p0 + PER and w of p0 .. p0 + PER),
 // joined between neighbouring lanes.  Positions clamped into the tour lie
 // inside the last block's range.
-template <int PER>
-__device__ __forceinline__ void put_summary(const SlotDev& s, int p0, const int (&xy)[PER + 2],
+template <int PER, typename Slot>
+__device__ __forceinline__ void put_summary(const Slot& s, int p0, const int (&xy)[PER + 2],
                                             const int (&w)[PER + 1]) {
   constexpr int G = MLP_BLK / PER;
   short2v lo = __builtin_bit_cast(short2v, xy[0]), hi = lo;
@@ -644,27 +699,28 @@ __device__ __forceinline__ void put_summary(const SlotDev& s, int p0, const int 
   const int b = group_pk<G, false>(__builtin_bit_cast(int, hi));
   wm = group_max<G>(wm);
   wp = group_max<G>(wp);
-  if (threadIdx.x % G == 0 && p0 < s.N) *(int4*)(s.blk + p0 / MLP_BLK) = make_int4(a, b, wm, wp);
+  if (threadIdx.x % G == 0 && p0 < s.N) *(gptr<int4v>)(s.blk + p0 / MLP_BLK) = int4v{a, b, wm, wp};
 }
 
-// n consecutive words of a thread as the widest stores they allow.
-template <int PER>
-__device__ __forceinline__ void put_words(int32_t* d, const int32_t (&v)[PER]) {
+// PER consecutive words of a thread as the widest stores they allow.
+template <int PER, typename P>
+__device__ __forceinline__ void put_words(P p, const int32_t (&v)[PER]) {
+  gptr<int32_t> d = (gptr<int32_t>)p;
   if constexpr (PER >= 4) {
 #pragma unroll
-    for (int h = 0; h < PER; h += 4) *(int4*)(d + h) = make_int4(v[h], v[h + 1], v[h + 2], v[h + 3]);
+    for (int h = 0; h < PER; h += 4) *(gptr<int4v>)(d + h) = int4v{v[h], v[h + 1], v[h + 2], v[h + 3]};
   } else if constexpr (PER == 2) {
-    *(int2*)d = make_int2(v[0], v[1]);
+    *(gptr<int2v>)d = int2v{v[0], v[1]};
   } else {
     d[0] = v[0];
   }
 }
-template <int PER>
-__device__ __forceinline__ void put_words(int64_t* d, const int64_t (&v)[PER]) {
+template <int PER, typename P>
+__device__ __forceinline__ void put_words(P p, const int64_t (&v)[PER]) {
+  gptr<int64_t> d = (gptr<int64_t>)p;
   if constexpr (PER >= 2) {
 #pragma unroll
-    for (int h = 0; h < PER; h += 2)
-      *(longlong2*)(d + h) = make_longlong2((long long)v[h], (long long)v[h + 1]);
+    for (int h = 0; h < PER; h += 2) *(gptr<long2v>)(d + h) = long2v{v[h], v[h + 1]};
   } else {
     d[0] = v[0];
   }
@@ -680,9 +736,9 @@ __device__ __forceinline__ void put_words(int64_t* d, const int64_t (&v)[PER]) {
 // tour's xy, so the new tour needs no gather from the instance arrays), or
 // nullptr to read the instance arrays.  tour_out: where the tour is copied to
 // (nullptr: nowhere).  sum: block summaries too.
-template <int TB, int PER>
-__device__ __forceinline__ void prep_tour(const SlotDev& s, const int32_t* tour, PrepWaves<TB>& P,
-                                          const int32_t* xyc, int32_t* tour_out, bool sum) {
+template <int TB, int PER, typename Slot, typename Tour>
+__device__ __forceinline__ void prep_tour(const Slot& s, Tour tour, PrepWaves<TB>& P,
+                                          const int32_t* xyc, gptr<int32_t> tour_out, bool sum) {
   constexpr int NW = TB / kWave;
   const int N = s.N, tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -717,7 +773,7 @@ __device__ __forceinline__ void prep_tour(const SlotDev& s, const int32_t* tour,
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
       at += w[e];
-      aq += (int64_t)(p0 + e) * w[e];
+      aq += umul(p0 + e, w[e]);  // below 2^31 (positions below 2^15, distances 2^16)
       lt[e] = at;
       lq[e] = aq;
     }
@@ -771,8 +827,8 @@ __device__ __forceinline__ void prep_tour(const SlotDev& s, const int32_t* tour,
       vt[e] = T;
       vq[e] = (int32_t)(uint32_t)(uint64_t)Q;
       const uint32_t Z = 2u * (uint32_t)(uint64_t)Q - (uint32_t)(2 * p + 1) * (uint32_t)T;
-      vg[e] = (int32_t)(0u - (uint32_t)(N - p) * (uint32_t)w[e] - Z);
-      vh[e] = (int32_t)(Z - (uint32_t)(N - p - 1) * (uint32_t)w[e + 1]);
+      vg[e] = (int32_t)(0u - umul(N - p, w[e]) - Z);
+      vh[e] = (int32_t)(Z - umul(N - p - 1, w[e + 1]));
     }
     if (p0 + PER <= N) {
       // p0 is a multiple of PER and every array 256-byte aligned
@@ -823,7 +879,7 @@ __global__ __launch_bounds__(TB) void k_prep(const SlotDev* __restrict__ table,
                                              SlotListInline list, const int32_t* list_dev) {
   __shared__ PrepWaves<TB> P;
   const int id = list_at(list, list_dev, blockIdx.x);
-  const SlotDev& s = table[id];
+  const SlotRegs s = slot_regs(table, id, 0);
   prep_tour<TB, PER>(s, s.tour, P, nullptr, nullptr, false);
   if (threadIdx.x == 0) {
     s.info[MLP_INFO_ROUND_MOVES] = 0;
@@ -863,7 +919,8 @@ namespace {
 // End of a DVND round for one active slot (run by the round's last merge):
 // count the round; a round that applied no move (or reached max_rounds > 0)
 // stops the slot; the next round counts its moves from zero.
-__device__ __forceinline__ void round_tail(const SlotDev& s, int max_rounds) {
+template <typename Slot>
+__device__ __forceinline__ void round_tail(const Slot& s, int max_rounds) {
   const int64_t r = s.info[MLP_INFO_ROUNDS] + 1;
   s.info[MLP_INFO_ROUNDS] = r;
   if (s.info[MLP_INFO_ROUND_MOVES] == 0 || (max_rounds > 0 && r >= max_rounds))
@@ -993,24 +1050,21 @@ __device__ __forceinline__ bool conflicts_kind(int k, int i1, int j1, int i2, in
 // out[q] as (i << 32 | j) (out may be keys: kept moves overwrite only keys of
 // decided batches) and to the slot's kept arrays.  Returns their count.
 // Candidates from index `tail` on are read from gtail (a sort whose keys
-// exceed the LDS buffer).  The next batch's keys and ctx and the key after it
-// are read while a batch is decided.
-template <int KIND>
-__device__ __forceinline__ int greedy_wave(const SlotDev& s, int nb, int N, int rowmap, int M,
+// exceed the LDS buffer); ctx(t, key) is a candidate's row-local index.  The
+// next batch's keys and ctx and the key after it are read while a batch is
+// decided.
+template <int KIND, typename Slot, typename Ctx>
+__device__ __forceinline__ int greedy_wave(const Slot& s, int nb, int N, int rowmap, int M,
                                            const int64_t* keys, int64_t* out, int kept0,
-                                           const uint16_t* ctxL, uint32_t* bits, int lane,
+                                           Ctx ctx, uint32_t* bits, int lane,
                                            const int64_t* gtail, int tail) {
   const int K = KIND == 2 ? nb - 1 : 0;
   auto key_at = [&](int t) -> int64_t {
     return t < M ? (t < tail ? keys[t] : ldg(gtail + t)) : MLP_KEY_NONE;
   };
-  auto ctx_at = [&](int t, int64_t key) -> int {
-    return t < M ? (int)ctxL[(int)(key & MLP_KEY_MASK)] : 0;
-  };
-  // slot fields in registers: the loop's global stores would otherwise make
-  // the compiler reload them (a global load on every batch)
-  int64_t* const kcost = s.kept_cost[nb];
-  int32_t* const kij = s.kept_ij[nb];
+  auto ctx_at = [&](int t, int64_t key) -> int { return t < M ? ctx(t, key) : 0; };
+  const auto kcost = kept_cost(s, nb);
+  const auto kij = kept_ij(s, nb);
   int64_t skc = key_at(lane);
   int ctxc = ctx_at(lane, skc);
   int64_t skn = key_at(kWave + lane);
@@ -1072,12 +1126,12 @@ __device__ __forceinline__ int greedy_wave(const SlotDev& s, int nb, int N, int 
 // ij(q) gives the q-th kept move as (i << 32 | j); tnew ends as the new tour
 // (after the caller's next barrier).  loaded: told and tnew already hold the
 // tour (copied at the kernel's start, its load overlapping the row-key loads).
-template <int TB, typename IJ>
-__device__ __forceinline__ void apply_kept(const SlotDev& s, int nb, int K, IJ ij, int32_t* told,
+template <int TB, typename Slot, typename IJ>
+__device__ __forceinline__ void apply_kept(const Slot& s, int nb, int K, IJ ij, int32_t* told,
                                            int32_t* tnew, int& s_long, int* s_longq,
                                            bool loaded = false) {
   const int N = s.N, tid = threadIdx.x, k = nb_k(nb);
-  int32_t* const tour = s.tour;  // in a register across the loops' stores
+  const auto tour = s.tour;  // in a register across the loops' stores
   if (!loaded)
     for (int p = tid; p < N; p += TB) {
       const int c = tour[p];
@@ -1318,33 +1372,76 @@ struct MergeShared {
 static_assert(sizeof(MergeShared<1024>) <= 8192, "static LDS left beside the merge's dynamic part");
 
 // Sort of list[0..n), n <= 256, distinct keys: a key's rank is the number of
-// smaller keys, counted by TB / 256 threads a key (M reads of LDS broadcasts
-// against the 36 barrier phases of a bitonic sort of 256).
-template <int TB>
-__device__ __forceinline__ void rank_sort(int64_t* list, int n, int* rank) {
+// smaller keys, counted by TB / 256 threads a key, eight LDS broadcasts in
+// flight (against the 36 barrier phases of a bitonic sort of 256; one at a
+// time they had taken 6400 cycles for 145 keys).  list is padded to 256.
+// carry(e): a value that moves with key e, to sorted place in rank[256 ..].
+template <int TB, typename Carry>
+__device__ __forceinline__ void rank_sort(int64_t* list, int n, int* rank, Carry carry) {
   constexpr int G = TB / 256;
   const int tid = threadIdx.x, e = tid & 255, g = tid >> 8;
-  const int64_t my = e < n ? list[e] : 0;
-  int r = 0;
-  if constexpr (G > 1) {
-    if (tid < 256) rank[tid] = 0;
-    __syncthreads();
+  const int per = ((n + G - 1) / G + 7) & ~7;  // G per <= 256
+  const int64_t my = e < n ? list[e] : MLP_KEY_NONE;
+  const int with = g == 0 && e < n ? carry(e) : 0;
+  if (g == 0) {
+    if (e >= n) list[e] = MLP_KEY_NONE;
+    rank[e] = 0;
   }
+  __syncthreads();
+  int r = 0;
   if (e < n) {
-    const int per = (n + G - 1) / G, u1 = min(n, per * (g + 1));
-    for (int u = per * g; u < u1; ++u) r += list[u] < my ? 1 : 0;
+#pragma unroll 1
+    for (int u = per * g; u < per * (g + 1); u += 8) {
+      int64_t v[8];
+#pragma unroll
+      for (int x = 0; x < 8; ++x) v[x] = list[u + x];
+#pragma unroll
+      for (int x = 0; x < 8; ++x) r += v[x] < my ? 1 : 0;
+    }
     if constexpr (G > 1) atomicAdd(&rank[e], r);
   }
   __syncthreads();
-  if (g == 0 && e < n) list[G > 1 ? rank[e] : r] = my;
+  if (g == 0 && e < n) {
+    if constexpr (G > 1) r = rank[e];
+    list[r] = my;
+    rank[256 + r] = with;
+  }
   __syncthreads();
 }
 
 // Selection of the greedy subset without a sort of all M candidates: thread
-// tid looks after candidates t = tid + u TB (u < 32, a bit of `alive` each);
+// tid looks after candidates t = tid + u TB (u < 32, a bit of a mask each);
 // key(t) is t's (cost, row) key and move(t, key) its move (i << 16 | j), both
-// unchanged until the selection ends.
-//
+// unchanged until the selection ends.  A thread's first candidate, the only
+// one of tours up to 1024 positions, stays in registers.
+template <int TB, typename Key, typename Move>
+struct Candidates {
+  Key key;
+  Move move;
+  int64_t k0;
+  int ij0;
+  uint32_t alive;
+  __device__ __forceinline__ Candidates(int M, Key k, Move m) : key(k), move(m), k0(0), ij0(0), alive(0) {
+    const int t = threadIdx.x;
+    if (t < M) {
+      k0 = key(t);
+      ij0 = move(t, k0);
+    }
+    for (int u = 0; t + u * TB < M; ++u) alive |= 1u << u;
+  }
+  // f(bit, key, move) for each candidate of the mask
+  template <typename F>
+  __device__ __forceinline__ void each(uint32_t mask, F f) const {
+    if (mask & 1u) f(1u, k0, ij0);
+#pragma unroll 1
+    for (uint32_t m = mask & ~1u; m; m &= m - 1) {
+      const int t = (int)threadIdx.x + __builtin_ctz(m) * TB;
+      const int64_t k = key(t);
+      f(m & (0u - m), k, move(t, k));
+    }
+  }
+};
+
 // select_spans, for the interval moves (2-opt, or-opt).  The best moves are
 // long and conflict with most others, so the candidates are taken in slices
 // of the best 256 or fewer (by classes of the cost's magnitude, 32 an octave,
@@ -1353,20 +1450,16 @@ __device__ __forceinline__ void rank_sort(int64_t* list, int n, int* rank) {
 // so equal costs stay together and the order is that of the whole sort.
 // Returns -1 (no claims left) when one class exceeds a slice.  out: the kept
 // moves, at most N / 2 (a span claims at least two positions).
-template <int KIND, int TB, typename Key, typename Move>
-__device__ __forceinline__ int select_spans(const SlotDev& s, int nb, int N, int rowmap, int M, Key key,
+template <int KIND, int TB, typename Slot, typename Key, typename Move>
+__device__ __forceinline__ int select_spans(const Slot& s, int nb, int N, int rowmap, int M, Key key,
                                             Move move, int64_t* out, const uint16_t* ctxL,
                                             uint32_t* bits, MergeShared<TB>& S) {
   const int tid = threadIdx.x, lane = tid % kWave, K = KIND == 2 ? nb - 1 : 0;
   // class of a key: the float bits of -cost down to 5 of the mantissa
   auto cls = [](int64_t v) { return __float_as_int((float)(-(v >> MLP_KEY_SHIFT))) >> 18; };
-  uint32_t alive = 0;
+  Candidates<TB, Key, Move> C(M, key, move);
   int mx = 0;
-#pragma unroll 1
-  for (int u = 0; tid + u * TB < M; ++u) {
-    alive |= 1u << u;
-    mx = max(mx, cls(key(tid + u * TB)));
-  }
+  C.each(C.alive, [&](uint32_t, int64_t k, int) { mx = max(mx, cls(k)); });
   if (tid == 0) S.top = S.cnt = 0;
   __syncthreads();
   mx = wave_max_i32(mx);
@@ -1378,11 +1471,9 @@ __device__ __forceinline__ int select_spans(const SlotDev& s, int nb, int N, int
       for (int b = tid; b < kSelClasses; b += TB) S.hist[b] = 0;
       __syncthreads();
       top = S.top;
-#pragma unroll 1
-      for (uint32_t m = alive; m; m &= m - 1) {
-        const int64_t k = key(tid + __builtin_ctz(m) * TB);
+      C.each(C.alive, [&](uint32_t, int64_t k, int) {
         atomicAdd(&S.hist[min(top - cls(k), kSelClasses - 1)], 1);
-      }
+      });
       __syncthreads();
       if (tid < kWave) {  // the classes whose cumulative count fits a slice
         constexpr int PB = kSelClasses / kWave;
@@ -1406,21 +1497,21 @@ __device__ __forceinline__ int select_spans(const SlotDev& s, int nb, int N, int
         return -1;
       }
     }
-#pragma unroll 1
-    for (uint32_t m = alive; m; m &= m - 1) {
-      const int u = __builtin_ctz(m);
-      const int64_t k = key(tid + u * TB);
+    uint32_t take = 0;
+    C.each(C.alive, [&](uint32_t b, int64_t k, int) {
       if (left <= kSelCap || min(top - cls(k), kSelClasses - 1) <= cut) {
         S.list[atomicAdd(&S.cnt, 1)] = k;
-        alive &= ~(1u << u);
+        take |= b;
       }
-    }
+    });
+    C.alive &= ~take;
     __syncthreads();
     const int n = S.cnt;
-    rank_sort<TB>(S.list, n, S.hist);
+    rank_sort<TB>(S.list, n, S.hist, [&](int e) { return (int)ctxL[(int)(S.list[e] & MLP_KEY_MASK)]; });
     if (tid < kWave) {
-      const int kk = greedy_wave<KIND>(s, nb, N, rowmap, n, S.list, out, kept, ctxL, bits, lane,
-                                       nullptr, INT32_MAX);
+      const int kk = greedy_wave<KIND>(
+          s, nb, N, rowmap, n, S.list, out, kept, [&](int t, int64_t) { return S.hist[256 + t]; }, bits,
+          lane, nullptr, INT32_MAX);
       if (lane == 0) {
         S.kept = kk;
         S.cnt = S.top = S.left = 0;
@@ -1431,16 +1522,14 @@ __device__ __forceinline__ int select_spans(const SlotDev& s, int nb, int N, int
     left -= n;
     if (left == 0) break;
     mx = 0;
-#pragma unroll 1
-    for (uint32_t m = alive; m; m &= m - 1) {
-      const int u = __builtin_ctz(m);
-      const int64_t k = key(tid + u * TB);
-      const int ij = move(tid + u * TB, k), i = ij >> 16, j = ij & 0xffff;
-      if (claims_any(bits, N, KIND == 1 ? i : min(i, j), KIND == 1 ? j + 1 : max(i, j) + K))
-        alive &= ~(1u << u);
+    uint32_t drop = 0;
+    C.each(C.alive, [&](uint32_t b, int64_t k, int ij) {
+      const int i = ij >> 16, j = ij & 0xffff;
+      if (claims_any(bits, N, KIND == 1 ? i : min(i, j), KIND == 1 ? j + 1 : max(i, j) + K)) drop |= b;
       else mx = max(mx, cls(k));
-    }
-    const int c = wave_scan_i32(__popc(alive));  // lane 63: the wave's
+    });
+    C.alive &= ~drop;
+    const int c = wave_scan_i32(__popc(C.alive));  // lane 63: the wave's
     mx = wave_max_i32(mx);
     if (lane == kWave - 1 && c) {
       atomicMax(&S.top, mx);
@@ -1457,79 +1546,69 @@ __device__ __forceinline__ int select_spans(const SlotDev& s, int nb, int N, int
 // position of one of its ends, so the candidates decide among themselves, many
 // at a time: the best key at each position (pm, an LDS minimum), then a
 // candidate that is the best at its ends' six positions is kept (nothing
-// before it in the order can conflict), its positions are claimed and the
-// others that touch them leave.  This keeps exactly what the greedy in order
-// keeps; the kept ones are sorted at the end for the list.  Returns -1 as
-// select_spans does when kSwapRounds rounds leave candidates (a chain of
-// conflicts in the order of the costs).  pm: max(N, 512) entries; the kept
-// moves end there.
+// before it in the order can conflict), it marks its ends, and the others
+// that have a marked position among their six leave.  This keeps exactly what
+// the greedy in order keeps; the kept ones are sorted at the end for the
+// list.  A round's keys are lower than the last one's by 2^52 (|key| < 2^51
+// when |delta| < 2^31, which the caller sees to), so nothing is reset between
+// rounds, and the lowest value marks: two barriers a round.  Returns -1 when
+// kSwapRounds rounds leave candidates (a chain of conflicts in the order of
+// the costs).  pm: max(N, 512) entries; the kept moves end there.
 constexpr int kSwapRounds = 24;
-template <int TB, typename Key, typename Move>
-__device__ __forceinline__ int select_swaps(const SlotDev& s, int N, int rowmap, int M, Key key,
+template <int TB, typename Slot, typename Key, typename Move>
+__device__ __forceinline__ int select_swaps(const Slot& s, int N, int rowmap, int M, Key key,
                                             Move move, int64_t* pm, const uint16_t* ctxL,
-                                            uint32_t* bits, MergeShared<TB>& S) {
+                                            MergeShared<TB>& S) {
+  constexpr int64_t kMark = INT64_MIN;
   const int tid = threadIdx.x;
-  uint32_t alive = 0, keep = 0;
-  for (int u = 0; tid + u * TB < M; ++u) alive |= 1u << u;
+  Candidates<TB, Key, Move> C(M, key, move);
+  uint32_t keep = 0;
   if (tid == 0) S.cnt = 0;
   for (int p = tid; p < N; p += TB) pm[p] = MLP_KEY_NONE;
   __syncthreads();
-  bool more = true;
-  for (int round = 0; round < kSwapRounds && more; ++round) {
-#pragma unroll 1
-    for (uint32_t m = alive; m; m &= m - 1) {
-      const int t = tid + __builtin_ctz(m) * TB;
-      const int64_t k = key(t);
-      const int ij = move(t, k);
-      atomicMin((long long*)&pm[ij >> 16], (long long)k);
-      atomicMin((long long*)&pm[ij & 0xffff], (long long)k);
-    }
-    __syncthreads();
-    uint32_t win = 0;
-#pragma unroll 1
-    for (uint32_t m = alive; m; m &= m - 1) {
-      const int u = __builtin_ctz(m), t = tid + u * TB;
-      const int64_t k = key(t);
-      const int ij = move(t, k), i = ij >> 16, j = ij & 0xffff;  // 1 <= i, j <= N - 2
-      const int64_t a = min(min(pm[i - 1], pm[i]), pm[i + 1]);
-      const int64_t b = min(min(pm[j - 1], pm[j]), pm[j + 1]);
-      if (min(a, b) == k) win |= 1u << u;
-    }
-    __syncthreads();
-#pragma unroll 1
-    for (uint32_t m = alive; m; m &= m - 1) {
-      const int u = __builtin_ctz(m), t = tid + u * TB;
-      const int ij = move(t, key(t)), i = ij >> 16, j = ij & 0xffff;
-      pm[i] = pm[j] = MLP_KEY_NONE;
-      if ((win >> u) & 1u) {
-        claims_set(bits, N, i - 1, i + 1);
-        claims_set(bits, N, j - 1, j + 1);
+  // 1 <= i, j <= N - 2
+  auto lowest = [&](int i, int j) {
+    const int64_t a = min(min(pm[i - 1], pm[i]), pm[i + 1]);
+    const int64_t b = min(min(pm[j - 1], pm[j]), pm[j + 1]);
+    return min(a, b);
+  };
+  int64_t stamp = 0;
+  for (int round = 0;; ++round, stamp += 1LL << 52) {
+    uint32_t drop = 0;
+    C.each(C.alive, [&](uint32_t b, int64_t k, int ij) {
+      const int i = ij >> 16, j = ij & 0xffff;
+      if (round > 0 && lowest(i, j) == kMark) {
+        drop |= b;
+      } else {
+        atomicMin((long long*)&pm[i], (long long)(k - stamp));
+        atomicMin((long long*)&pm[j], (long long)(k - stamp));
       }
+    });
+    C.alive &= ~drop;
+    if (!__syncthreads_or(C.alive != 0)) break;
+    if (round == kSwapRounds) {
+      __syncthreads();
+      return -1;
     }
+    uint32_t win = 0;
+    C.each(C.alive, [&](uint32_t b, int64_t k, int ij) {
+      const int i = ij >> 16, j = ij & 0xffff;
+      if (lowest(i, j) == k - stamp) {
+        pm[i] = pm[j] = kMark;
+        win |= b;
+      }
+    });
+    C.alive &= ~win;
     keep |= win;
-    alive &= ~win;
     __syncthreads();
-#pragma unroll 1
-    for (uint32_t m = alive; m; m &= m - 1) {
-      const int u = __builtin_ctz(m), t = tid + u * TB;
-      const int ij = move(t, key(t));
-      if ((int)claimed(bits, N, ij >> 16) | (int)claimed(bits, N, ij & 0xffff)) alive &= ~(1u << u);
-    }
-    more = __syncthreads_or(alive != 0) != 0;
   }
-  if (more) {
-    for (int w = tid; w < claim_words(N); w += TB) bits[w] = 0;
-    __syncthreads();
-    return -1;
-  }
-#pragma unroll 1
-  for (uint32_t m = keep; m; m &= m - 1) pm[atomicAdd(&S.cnt, 1)] = key(tid + __builtin_ctz(m) * TB);
+  C.each(keep, [&](uint32_t, int64_t k, int) { pm[atomicAdd(&S.cnt, 1)] = k; });
   __syncthreads();
   const int n = S.cnt;
-  if (n <= kSelCap) rank_sort<TB>(pm, n, S.hist);
+  if (n <= kSelCap) rank_sort<TB>(pm, n, S.hist, [](int) { return 0; });
   else bitonic_keys<TB>(pm, n);
-  int64_t* const kcost = s.kept_cost[0];
-  int32_t* const kij = s.kept_ij[0];
+  const auto kcost = kept_cost(s, 0);
+  const auto kij = kept_ij(s, 0);
 #pragma unroll 1
   for (int q = tid; q < n; q += TB) {
     const int64_t k = pm[q];
@@ -1551,15 +1630,17 @@ __device__ __forceinline__ int select_swaps(const SlotDev& s, int N, int rowmap,
 // subset from a selection.  Returns the kept count; sk points at LDS or the
 // keys, whose first entries then hold the kept moves as (i << 32 | j).
 // cap: entries of the LDS buffer (the keys' own, or at lds when GMEM); a
-// selection runs where it holds what the selection needs.
+// selection runs where it holds what the selection needs.  p32: |delta| < 2^31.
 // Swaps are selected from 65 candidates on, spans from 257 on (a slice).
 // First merges of a solve, whole sort and serial greedy before and now:
-// n = 9001 swap 320 -> 108 us, 2-opt 116 -> 35; n up to 2000 swap 63 -> 42,
-// or-opt 50 -> 25; n = 1000 swap 30 -> 27, or-opt 24 -> 19.
-template <bool GMEM, int TB>
-__device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap, int N, int M,
-                                           int64_t* keys, int64_t* lds, int cap, const uint16_t* ctxL,
-                                           uint32_t* bits, MergeShared<TB>& S, int64_t*& sk) {
+// n = 9001 swap 320 -> 83 us, 2-opt 116 -> 32, or-opt 240 -> 45; n = 1000
+// swap 30 -> 18, or-opt 24 -> 17.  Mean over a solve: k_mg_select n = 9001
+// 26.7 -> 11.4 us, k_merge_apply n = 1000 8.9 -> 7.9, n = 100 5.2 -> 4.3.
+template <bool GMEM, int TB, typename Slot>
+__device__ __forceinline__ int sort_greedy(const Slot& s, int nb, int rowmap, int N, int M,
+                                           int64_t* keys, int64_t* lds, int cap, bool p32,
+                                           const uint16_t* ctxL, uint32_t* bits, MergeShared<TB>& S,
+                                           int64_t*& sk) {
   const int tid = threadIdx.x;
   const int64_t* gtail = nullptr;  // sorted keys beyond the LDS buffer
   int tail = INT32_MAX;
@@ -1575,7 +1656,7 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
     if constexpr (GMEM) {
       // the moves (and the spans' keys) in LDS, so that no pass gathers
       // them from global memory again
-      const bool swaps = nb == 0 && M > kWave && 2 * N + M <= 2 * kGmemBuf;
+      const bool swaps = nb == 0 && p32 && M > kWave && 2 * N + M <= 2 * kGmemBuf;
       const bool spans = nb > 0 && M > kSelCap && 3 * M + N + 2 <= 2 * kGmemBuf;
       if (swaps || spans) {
         int32_t* const lij = (int32_t*)(lds + (swaps ? N : M + (N + 1) / 2));
@@ -1590,7 +1671,7 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
         sk = swaps ? lds : lds + M;
         if (swaps)
           kept = select_swaps<TB>(s, N, rowmap, M, [&](int t) { return ldg(keys + t); }, move, sk,
-                                  ctxL, bits, S);
+                                  ctxL, S);
         else if (nb == 1)
           kept = select_spans<1, TB>(s, nb, N, rowmap, M, lkey, move, sk, ctxL, bits, S);
         else kept = select_spans<2, TB>(s, nb, N, rowmap, M, lkey, move, sk, ctxL, bits, S);
@@ -1599,8 +1680,8 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
       auto move = [&](int, int64_t key) { return decode(key); };
       auto lkey = [&](int t) { return keys[t]; };
       sk = keys + M;
-      if (nb == 0 && M > kWave && M + max(N, kSortSeg) <= cap)
-        kept = select_swaps<TB>(s, N, rowmap, M, lkey, move, sk, ctxL, bits, S);
+      if (nb == 0 && p32 && M > kWave && M + max(N, kSortSeg) <= cap)
+        kept = select_swaps<TB>(s, N, rowmap, M, lkey, move, sk, ctxL, S);
       else if (nb == 1 && M > kSelCap && M + N / 2 <= cap)
         kept = select_spans<1, TB>(s, nb, N, rowmap, M, lkey, move, sk, ctxL, bits, S);
       else if (nb > 1 && M > kSelCap && M + N / 2 <= cap)
@@ -1609,23 +1690,31 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
     if (kept >= 0) return kept;
   }
   sk = GMEM && M <= cap ? lds : keys;
-  // Up to one key per lane of a wave, keys in LDS: rank sort on wave 0, which
-  // also runs the greedy next (the keys are distinct; a key's rank is the
-  // number of smaller keys; every lane reads all keys before any lane
-  // writes).  Up to 256 the same over the workgroup, else a bitonic sort.
-  if (!GMEM && M <= kWave) {
+  // Up to one key per lane of a wave: rank sort on wave 0, which also runs the
+  // greedy next (the keys are distinct; a key's rank is the number of smaller
+  // keys, each broadcast from its lane).  Up to 256 the same over the
+  // workgroup, else a bitonic sort.
+  auto ctx_of = [&](int64_t key) { return (int)ctxL[(int)(key & MLP_KEY_MASK)]; };
+  if (M <= kWave) {
     if (tid < kWave) {
-      const int64_t my = tid < M ? keys[tid] : 0;
+      const int64_t my = tid < M ? keys[tid] : MLP_KEY_NONE;
+      const int c = tid < M ? ctx_of(my) : 0;
       int rank = 0;
-      for (int u = 0; u < M; ++u) rank += keys[u] < my ? 1 : 0;
-      __builtin_amdgcn_wave_barrier();
-      if (tid < M) keys[rank] = my;
+      for (int u = 0; u < M; u += 4) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) rank += readlane64(my, u + x) < my ? 1 : 0;
+      }
+      if (tid < M) {
+        S.list[rank] = my;
+        S.hist[256 + rank] = c;
+      }
       __builtin_amdgcn_wave_barrier();
     }
+    in = S.list;
   } else if (M <= kSelCap) {
     if (tid < M) S.list[tid] = keys[tid];
     __syncthreads();
-    rank_sort<TB>(S.list, M, S.hist);
+    rank_sort<TB>(S.list, M, S.hist, [&](int e) { return ctx_of(S.list[e]); });
     in = S.list;
   } else if (GMEM && M <= kGmemSortCap) {
     // the slot's working arrays are in global memory, but its improving rows
@@ -1682,9 +1771,19 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
   // 3. greedy filter on wave 0
   if (tid < kWave) {
     int kept = 0;
-    if (nb == 0) kept = greedy_wave<0>(s, nb, N, rowmap, M, in, sk, 0, ctxL, bits, tid, gtail, tail);
-    else if (nb == 1) kept = greedy_wave<1>(s, nb, N, rowmap, M, in, sk, 0, ctxL, bits, tid, gtail, tail);
-    else if (nb < MLP_NB_MAX) kept = greedy_wave<2>(s, nb, N, rowmap, M, in, sk, 0, ctxL, bits, tid, gtail, tail);
+    auto greedy = [&](auto kind) {
+      constexpr int KIND = decltype(kind)::value;
+      if (M <= kSelCap)  // one list, its ctx beside it
+        return greedy_wave<KIND>(
+            s, nb, N, rowmap, M, in, sk, 0, [&](int t, int64_t) { return S.hist[256 + t]; }, bits, tid,
+            nullptr, INT32_MAX);
+      return greedy_wave<KIND>(
+          s, nb, N, rowmap, M, in, sk, 0, [&](int, int64_t key) { return ctx_of(key); }, bits, tid, gtail,
+          tail);
+    };
+    if (nb == 0) kept = greedy(std::integral_constant<int, 0>{});
+    else if (nb == 1) kept = greedy(std::integral_constant<int, 1>{});
+    else if (nb < MLP_NB_MAX) kept = greedy(std::integral_constant<int, 2>{});
     if (tid == 0) S.kept = kept;
   }
   __syncthreads();
@@ -1697,13 +1796,13 @@ __device__ __forceinline__ int sort_greedy(const SlotDev& s, int nb, int rowmap,
 // (strided by TB) before it uses the first.  rows(q) loads row q's key from
 // either buffer; the choice, which waits for the slot's info words, comes
 // when the keys are used: pick(a, b).
-template <int TB, int P, typename Rows, typename Pick, typename Put>
-__device__ __forceinline__ void merge_rows(const SlotDev& s, Rows rows, Pick pick, int R, int q0,
+template <int TB, int P, typename Slot, typename Rows, typename Pick, typename Put>
+__device__ __forceinline__ void merge_rows(const Slot& s, Rows rows, Pick pick, int R, int q0,
                                            int q1, int32_t* told, int32_t* tnew, int32_t* xyc,
                                            uint16_t* ctxL, Put put) {
   const int N = s.N, tid = threadIdx.x;
-  const int32_t* const tour = s.tour;  // in registers across the loop's stores
-  const int32_t* const xy = s.xy;
+  const auto tour = s.tour;  // in registers across the loop's stores
+  const auto xy = s.xy;
   const int rend = min(R, q1), nend = min(N, q1);
   for (int base = q0; base < q1; base += TB * P) {
     int64_t ka[P], kb[P];
@@ -1737,7 +1836,7 @@ __device__ __forceinline__ void merge_rows(const SlotDev& s, Rows rows, Pick pic
 // (mlp_merge_lds_bytes(pcap_l, ncap_l)).  flags bit 0: inside a DVND round;
 // bit 1: block summaries of the new tour are kept.
 template <int TB, int PER>
-__device__ __forceinline__ void merge_slot(const SlotDev& s, int nb, int rowmap, int pcap_l,
+__device__ __forceinline__ void merge_slot(const SlotRegs& s, int nb, int rowmap, int pcap_l,
                                            int ncap_l, int flags, int tail, int64_t* lds,
                                            MergeShared<TB>& S) {
   const int N = s.N, tid = threadIdx.x;
@@ -1752,8 +1851,9 @@ __device__ __forceinline__ void merge_slot(const SlotDev& s, int nb, int rowmap,
   uint32_t* bits = (uint32_t*)(xyc + ncap);
   uint16_t* ctxL = (uint16_t*)((uint32_t*)(xyc + ncap) + claim_words(ncap));  // ctx of each improving row
   int64_t* sk = keys;  // the sorted keys (greedy, apply)
-  const int64_t active = ldg(s.info + MLP_INFO_ACTIVE);
-  const int64_t parity = ldg(s.info + MLP_INFO_PARITY0 + nb);
+  const int64_t active = s.info[MLP_INFO_ACTIVE];
+  const int64_t parity = s.info[MLP_INFO_PARITY0 + nb];
+  const bool p32 = (s.info[MLP_INFO_PATH32] & MLP_P32_SWAP_OROPT) != 0;
 
   if (tid == 0) S.m = 0;
   for (int w = tid; w < nwords; w += TB) bits[w] = 0;
@@ -1766,13 +1866,13 @@ __device__ __forceinline__ void merge_slot(const SlotDev& s, int nb, int rowmap,
   // with the row keys'; both buffers' keys are loaded, so that the loads do
   // not wait for the parity.
   const int par = (int)(parity & 1) ^ (dvnd ? 1 : 0);
-  const int64_t* const rk = s.rows[nb];
+  const auto rk = s.rows;
   const int cap = s.rowcap;
   merge_rows<TB, PER>(
       s,
       [&](int q, int64_t& a, int64_t& b) {
-        a = ldg(rk + q);
-        b = ldg(rk + cap + q);
+        a = rk[q];
+        b = rk[cap + q];
       },
       [&](int64_t a, int64_t b) { return par ? b : a; }, R, 0, max(R, N), told, tnew, xyc, ctxL,
       [&](int64_t k) { keys[atomicAdd(&S.m, 1)] = k; });
@@ -1787,7 +1887,7 @@ __device__ __forceinline__ void merge_slot(const SlotDev& s, int nb, int rowmap,
     }
     return;
   }
-  const int K = sort_greedy<false, TB>(s, nb, rowmap, N, M, keys, lds, pcap, ctxL, bits, S, sk);
+  const int K = sort_greedy<false, TB>(s, nb, rowmap, N, M, keys, lds, pcap, p32, ctxL, bits, S, sk);
   // 4. apply the kept moves, rebuild the prefix arrays
   apply_kept<TB>(s, nb, K, [&](int q) { return sk[q]; }, told, tnew, S.lng, S.longq, true);
   __syncthreads();
@@ -1813,7 +1913,7 @@ __global__ __launch_bounds__(TB) void k_merge_apply(const SlotDev* __restrict__ 
   extern __shared__ int64_t lds[];
   __shared__ MergeShared<TB> S;
   const int id = list_at(list, list_dev, blockIdx.x);
-  merge_slot<TB, PER>(table[id], nb, rowmap, pcap_l, ncap_l, flags, tail, lds, S);
+  merge_slot<TB, PER>(slot_regs(table, id, nb), nb, rowmap, pcap_l, ncap_l, flags, tail, lds, S);
 }
 
 // ---------------------------------------------------------------------------
@@ -1844,7 +1944,9 @@ struct MgArrays {
 // The slot's global working arrays: the one-workgroup merge's layout
 // (keys[pcap] | told[N] | tnew[N] | xyc[N] | bitmap | ctx[pcap]), then the
 // segment sums.
-__device__ __forceinline__ MgArrays mg_arrays(const SlotDev& s) {
+__device__ __forceinline__ MgArrays mg_arrays(const SlotDev* table, int id) {
+  const auto& s = *((const __attribute__((address_space(4))) SlotDev*)table +
+                    __builtin_amdgcn_readfirstlane(id));
   int pcap = 1;
   while (pcap < s.rowcap) pcap <<= 1;
   const int N = s.N;
@@ -1865,20 +1967,21 @@ __global__ __launch_bounds__(kBlock) void k_mg_compact(const SlotDev* __restrict
   __shared__ int64_t lk[MLP_MG_CHUNK];
   __shared__ int lm;
   __shared__ int64_t lbase;
-  const SlotDev& s = table[list_at(list, list_dev, blockIdx.y)];
+  const int id = list_at(list, list_dev, blockIdx.y);
+  const SlotRegs s = slot_regs(table, id, nb);
   if (skip_inactive && s.info[MLP_INFO_ACTIVE] == 0) return;
   const int N = s.N, tid = threadIdx.x, R = rows_of(nb, rowmap, N);
   const int q0 = blockIdx.x * MLP_MG_CHUNK, q1 = min(q0 + MLP_MG_CHUNK, max(R, N));
   if (q0 >= q1) return;
-  const MgArrays a = mg_arrays(s);
+  const MgArrays a = mg_arrays(table, id);
   // the eval of a DVND round wrote the buffer opposite info[PARITY0 + nb]
   // (k_mg_select commits it once every segment has read it)
   const int par = (int)(s.info[MLP_INFO_PARITY0 + nb] & 1) ^ (skip_inactive ? 1 : 0);
-  const int64_t* rk = s.rows[nb] + (par ? s.rowcap : 0);
+  const auto rk = s.rows + (par ? s.rowcap : 0);
   if (tid == 0) lm = 0;
   __syncthreads();
   merge_rows<kBlock, 8>(
-      s, [&](int q, int64_t& ka, int64_t& kb) { ka = kb = ldg(rk + q); },
+      s, [&](int q, int64_t& ka, int64_t& kb) { ka = kb = rk[q]; },
       [&](int64_t ka, int64_t) { return ka; }, R, q0, q1, a.told, a.tnew, a.xyc, a.ctxL,
       [&](int64_t k) { lk[atomicAdd(&lm, 1)] = k; });
   __syncthreads();
@@ -1898,15 +2001,17 @@ __global__ __launch_bounds__(kSelBlock) void k_mg_select(const SlotDev* __restri
                                                       int tail) {
   extern __shared__ int64_t lds[];
   __shared__ MergeShared<kSelBlock> S;
-  const SlotDev& s = table[list_at(list, list_dev, blockIdx.x)];
+  const int id = list_at(list, list_dev, blockIdx.x);
+  const SlotRegs s = slot_regs(table, id, nb);
   const int tid = threadIdx.x;
   if (skip_inactive && s.info[MLP_INFO_ACTIVE] == 0) {
     if (tid == 0) s.info[MLP_INFO_MG_APPLY] = 0;
     return;
   }
   const int N = s.N;
-  const MgArrays a = mg_arrays(s);
+  const MgArrays a = mg_arrays(table, id);
   const int M = (int)s.info[MLP_INFO_MCOUNT];
+  const bool p32 = (s.info[MLP_INFO_PATH32] & MLP_P32_SWAP_OROPT) != 0;
   const int par = (int)(s.info[MLP_INFO_PARITY0 + nb] & 1) ^ (skip_inactive ? 1 : 0);
   uint32_t* bits = (uint32_t*)(lds + kGmemBuf);
   const int nwords = claim_words(N);
@@ -1925,8 +2030,8 @@ __global__ __launch_bounds__(kSelBlock) void k_mg_select(const SlotDev* __restri
     return;
   }
   int64_t* sk = a.keys;
-  const int K = sort_greedy<true, kSelBlock>(s, nb, rowmap, N, M, a.keys, lds, kGmemSortCap, a.ctxL, bits, S,
-                                             sk);
+  const int K = sort_greedy<true, kSelBlock>(s, nb, rowmap, N, M, a.keys, lds, kGmemSortCap, p32, a.ctxL,
+                                             bits, S, sk);
   // tnew becomes the new tour; k_mg_rebuild copies it back
   apply_kept<kSelBlock>(s, nb, K, [&](int q) { return sk[q]; }, a.told, a.tnew, S.lng, S.longq, true);
   if (tid == 0) {
@@ -1941,11 +2046,12 @@ __global__ __launch_bounds__(kSelBlock) void k_mg_select(const SlotDev* __restri
 __global__ __launch_bounds__(kBlock) void k_mg_sums(const SlotDev* __restrict__ table,
                                                     SlotListInline list, const int32_t* list_dev) {
   __shared__ PrepLds P;
-  const SlotDev& s = table[list_at(list, list_dev, blockIdx.y)];
+  const int id = list_at(list, list_dev, blockIdx.y);
+  const SlotDev& s = table[id];
   if (s.info[MLP_INFO_MG_APPLY] == 0) return;
   const int base = blockIdx.x * MLP_MG_CHUNK;
   if (base >= s.N) return;
-  const MgArrays a = mg_arrays(s);
+  const MgArrays a = mg_arrays(table, id);
   int64_t segT, segQ, lacc = 0;
   prep_segment<false>(s, a.tnew, a.xyc, base, 0, 0, P, segT, segQ, lacc);
   if (threadIdx.x == 0) {
@@ -1959,12 +2065,13 @@ __global__ __launch_bounds__(kBlock) void k_mg_rebuild(const SlotDev* __restrict
                                                        SlotListInline list,
                                                        const int32_t* list_dev, int sum) {
   __shared__ PrepLds P;
-  const SlotDev& s = table[list_at(list, list_dev, blockIdx.y)];
+  const int id = list_at(list, list_dev, blockIdx.y);
+  const SlotDev& s = table[id];
   if (s.info[MLP_INFO_MG_APPLY] == 0) return;
   const int N = s.N, base = blockIdx.x * MLP_MG_CHUNK;
   if (base >= N) return;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-  const MgArrays a = mg_arrays(s);
+  const MgArrays a = mg_arrays(table, id);
   const int nseg = (N + MLP_MG_CHUNK - 1) / MLP_MG_CHUNK;
   int64_t cT = 0, cQ = 0, Ttot = 0;
   for (int c = 0; c < nseg; ++c) {
@@ -2256,13 +2363,14 @@ __global__ __launch_bounds__(kBlock) void k_total_merge(const SlotDev* __restric
     if (stop) break;
   }
   const int K = T.kept;
-  const int32_t* kij = s.kept_ij[nb];
+  const SlotRegs r = slot_regs(table, id, nb);
+  const auto kij = r.kij;
   apply_kept<kBlock>(
-      s, nb, K,
+      r, nb, K,
       [&](int q) { return ((int64_t)kij[3 * q] << 32) | (uint32_t)kij[3 * q + 1]; }, told, tnew,
       T.nlong, T.longq);
   __syncthreads();
-  prep_tour<kBlock, 8>(s, tnew, PL, nullptr, s.tour, false);
+  prep_tour<kBlock, 8>(r, tnew, PL, nullptr, r.tour, false);
   if (tid == 0) {
     s.info[MLP_INFO_KEPT0 + nb] = K;
     s.info[MLP_INFO_ROUND_MOVES] += K;
@@ -2609,7 +2717,6 @@ union SweepLds {
   DiagLds<C> d;
 };
 
-__device__ __forceinline__ uint32_t umul(uint32_t a, uint32_t b) { return __umul24(a, b); }
 // signed 24-bit multiply, wrapped to 32 bits (|a|, |b| < 2^23)
 __device__ __forceinline__ uint32_t smul(int a, int b) { return (uint32_t)__mul24(a, b); }
 
@@ -3704,7 +3811,7 @@ __global__ __launch_bounds__(kBlock) void k_dvnd_fused(const SlotDev* __restrict
       }
       wait_at_least(merged + q, rr * MLP_NB_COUNT + nb, timeout);
       wait_at_least(done + q, rr * all + upto, timeout);
-      merge_slot<kBlock, 8>(table[P.slots[q]], nb, 0, P.pcap, P.ncap, 1,
+      merge_slot<kBlock, 8>(slot_regs(table, P.slots[q], nb), nb, 0, P.pcap, P.ncap, 1,
                         nb == MLP_NB_COUNT - 1 ? P.tail : 0, dyn, MS);
       signal_done(merged + q);
     } else {  // up to P.group tiles of the evaluation of nb for slot q
