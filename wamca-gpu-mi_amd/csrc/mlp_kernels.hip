@@ -1041,6 +1041,91 @@ __device__ __forceinline__ bool conflicts_kind(int k, int i1, int j1, int i2, in
   return ((int)(max(i1, j1) + k < min(i2, j2)) | (int)(min(i1, j1) > max(i2, j2) + k)) == 0;
 }
 
+template <int KIND>
+__device__ __forceinline__ bool conflicts_ij(int k, int a, int b) {  // moves (i << 16 | j)
+  return conflicts_kind<KIND>(k, a >> 16, a & 0xffff, b >> 16, b & 0xffff);
+}
+
+// The greedy over at most 64 P unsorted candidates whose deltas fit 32 bits,
+// on one wave: the best remaining one is kept and those it conflicts with
+// leave, as often as there are kept moves (a merge of up to 64 candidates
+// keeps 2 to 7, one of spans up to 256 keeps 5).  A kept move costs two wave
+// minima at most, no sort and no claimed positions are needed: 16 candidates
+// of which 2 are kept, sort and greedy 4400 cycles, 2700 now.  The kept
+// moves follow the kept0 ones of earlier calls; returns their count, or -1,
+// nothing kept, when a delta does not fit.
+template <int KIND, int P, typename Slot, typename Ctx>
+__device__ __forceinline__ int pick_wave(const Slot& s, int nb, int N, int rowmap, int M,
+                                         const int64_t* keys, int64_t* out, int kept0, Ctx ctx,
+                                         int lane) {
+  const int K = KIND == 2 ? nb - 1 : 0;
+  int32_t c[P], row[P];
+  int ij[P];
+  bool wide = false;
+#pragma unroll
+  for (int u = 0; u < P; ++u) {
+    const int t = lane + u * kWave;
+    const int64_t key = t < M ? keys[t] : MLP_KEY_NONE;
+    const int64_t cost = key >> MLP_KEY_SHIFT;
+    c[u] = t < M ? (int32_t)cost : INT32_MAX;
+    row[u] = (int)(key & MLP_KEY_MASK);
+    ij[u] = 0;
+    if (t < M) {
+      wide = wide || cost < INT32_MIN;
+      int i, j;
+      move_ij(nb, rowmap, N, row[u], ctx(key), i, j);
+      ij[u] = (i << 16) | j;
+    }
+  }
+  if (__ballot(wide)) return -1;
+  const auto kcost = kept_cost(s, nb);
+  const auto kij = kept_ij(s, nb);
+  // lane q holds the kept move kept0 + base + q until 64 are stored
+  int base = kept0, kept = 0;
+  int32_t kc = 0;
+  int kr = 0, km = 0;
+  auto store = [&]() {
+    if (lane < kept) {
+      const int q = base + lane;
+      out[q] = ((int64_t)(km >> 16) << 32) | (uint32_t)(km & 0xffff);
+      kcost[q] = kc;
+      kij[3 * q + 0] = km >> 16;
+      kij[3 * q + 1] = km & 0xffff;
+      kij[3 * q + 2] = kr;
+    }
+    base += kept;
+    kept = 0;
+  };
+  for (;;) {
+    int32_t lc = c[0];
+#pragma unroll
+    for (int u = 1; u < P; ++u) lc = min(lc, c[u]);
+    const int32_t m = wave_min_i32(lc);
+    if (m == INT32_MAX) break;
+    // the lowest row among equal costs (one lane's candidates first)
+    int32_t lr = INT32_MAX;
+    int lm = 0;
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+      const bool lt = c[u] == m && row[u] < lr;
+      lr = lt ? row[u] : lr;
+      lm = lt ? ij[u] : lm;
+    }
+    uint64_t own = __ballot(lc == m);
+    if (own & (own - 1)) own = __ballot(lr == wave_min_i32(lr));
+    const int l = __builtin_ctzll(own);
+    const int w = __builtin_amdgcn_readlane(lm, l), r = __builtin_amdgcn_readlane(lr, l);
+#pragma unroll
+    for (int u = 0; u < P; ++u) c[u] = conflicts_ij<KIND>(K, w, ij[u]) ? INT32_MAX : c[u];
+    kc = lane == kept ? m : kc;
+    km = lane == kept ? w : km;
+    kr = lane == kept ? r : kr;
+    if (++kept == kWave) store();
+  }
+  store();
+  return base;
+}
+
 // Greedy over the M candidates keys[0..M) sorted by (cost, row), on one wave,
 // 64 at a time.  The bitmap of positions claimed by kept moves is an exact
 // conflict test against every move kept so far (swap: positions i-1..i+1,
@@ -1365,6 +1450,7 @@ struct MergeShared {
   int m, kept, lng;
   int cnt, top, cut, left;  // selection
   int longq[kLongMoves];
+  int best[2][3][TB / kWave];  // select_spans: each wave's best cost, its row and move
   int hist[kSelClasses];    // candidates per class; ranks
   int64_t list[kSelCap];
   PrepWaves<TB> PL;
@@ -1443,28 +1529,120 @@ struct Candidates {
 };
 
 // select_spans, for the interval moves (2-opt, or-opt).  The best moves are
-// long and conflict with most others, so the candidates are taken in slices
-// of the best 256 or fewer (by classes of the cost's magnitude, 32 an octave,
-// counted in LDS): sort the slice, greedy on wave 0, then every thread drops
-// those of its candidates that now conflict.  A slice ends between classes,
-// so equal costs stay together and the order is that of the whole sort.
-// Returns -1 (no claims left) when one class exceeds a slice.  out: the kept
-// moves, at most N / 2 (a span claims at least two positions).
+// long and conflict with most others (500 candidates keep 9), so the first
+// ones are kept one by one over the workgroup: the best remaining candidate,
+// one barrier each (1700 cycles, 16 waves' minima), and every thread drops
+// those of its own that it conflicts with.  As soon as a wave can hold what is
+// left (looked at every kPicks moves), it goes on alone (pick_wave).  What is
+// left after kOneByOne moves goes in slices of the best 256 or fewer (by classes of
+// the cost's magnitude, 32 an octave, counted in LDS): sort the slice, greedy
+// on wave 0, then every thread drops those that now conflict.  A slice ends
+// between classes, so equal costs stay together and the order is that of the
+// whole sort.  Returns -1 (no claims left) when one class exceeds a slice.
+// out: the kept moves, at most N / 2 (a span claims at least two positions).
+// wide: deltas beyond 32 bits (slices only).
+constexpr int kPicks = 2, kOneByOne = 16;
 template <int KIND, int TB, typename Slot, typename Key, typename Move>
 __device__ __forceinline__ int select_spans(const Slot& s, int nb, int N, int rowmap, int M, Key key,
                                             Move move, int64_t* out, const uint16_t* ctxL,
                                             uint32_t* bits, MergeShared<TB>& S) {
+  constexpr int NW = TB / kWave;
   const int tid = threadIdx.x, lane = tid % kWave, K = KIND == 2 ? nb - 1 : 0;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   // class of a key: the float bits of -cost down to 5 of the mantissa
   auto cls = [](int64_t v) { return __float_as_int((float)(-(v >> MLP_KEY_SHIFT))) >> 18; };
   Candidates<TB, Key, Move> C(M, key, move);
-  int mx = 0;
+  int mx = 0, kept = 0;
+  // the thread's best candidate
+  int64_t bk = MLP_KEY_NONE;
+  int bm = 0;
+  bool wide = false;
+  auto better = [&](int64_t k, int ij) {
+    bm = k < bk ? ij : bm;
+    bk = k < bk ? k : bk;
+  };
+  C.each(C.alive, [&](uint32_t, int64_t k, int ij) {
+    better(k, ij);
+    wide = wide || (k >> MLP_KEY_SHIFT) < INT32_MIN;
+  });
+  if (tid == 0) S.top = S.cnt = S.left = 0;
+  int left = M;
+  if (!__syncthreads_or(wide)) {
+    const auto kcost = kept_cost(s, nb);
+    const auto kij = kept_ij(s, nb);
+    for (;;) {
+      // the wave's best (cost, row): by cost, then the lowest row of those
+      const int32_t c = bk == MLP_KEY_NONE ? INT32_MAX : (int32_t)(bk >> MLP_KEY_SHIFT);
+      const int32_t m = wave_min_i32(c);
+      uint64_t own = __ballot(c == m);
+      if (own & (own - 1)) {
+        const int r = c == m ? (int)(bk & MLP_KEY_MASK) : INT32_MAX;
+        own = __ballot(r == wave_min_i32(r));
+      }
+      const int buf = kept & 1;
+      if (lane == __builtin_ctzll(own)) {
+        S.best[buf][0][wave] = c;
+        S.best[buf][1][wave] = (int)(bk & MLP_KEY_MASK);
+        S.best[buf][2][wave] = bm;
+      }
+      __syncthreads();
+      // the workgroup's best, in every wave
+      const int wc = S.best[buf][0][lane % NW], wr = S.best[buf][1][lane % NW];
+      const int wm = S.best[buf][2][lane % NW];
+      const int32_t cost = wave_min_i32(wc);
+      if (cost == INT32_MAX) return kept;
+      own = __ballot(wc == cost) & ((1ull << NW) - 1ull);
+      if (own & (own - 1)) {
+        const int r = wc == cost ? wr : INT32_MAX;
+        own = __ballot(r == wave_min_i32(r));
+      }
+      const int l = __builtin_ctzll(own);
+      const int w = __builtin_amdgcn_readlane(wm, l), row = __builtin_amdgcn_readlane(wr, l);
+      if (tid == 0) {
+        out[kept] = ((int64_t)(w >> 16) << 32) | (uint32_t)(w & 0xffff);
+        kcost[kept] = cost;
+        kij[3 * kept + 0] = w >> 16;
+        kij[3 * kept + 1] = w & 0xffff;
+        kij[3 * kept + 2] = row;
+      }
+      ++kept;
+      uint32_t drop = 0;
+      bk = MLP_KEY_NONE;
+      C.each(C.alive, [&](uint32_t b, int64_t k, int ij) {
+        if (conflicts_ij<KIND>(K, w, ij)) drop |= b;
+        else better(k, ij);
+      });
+      C.alive &= ~drop;
+      if (kept % kPicks) continue;
+      const int c0 = wave_scan_i32(__popc(C.alive));
+      if (lane == kWave - 1 && c0) atomicAdd(&S.left, c0);
+      __syncthreads();
+      left = S.left;
+      __syncthreads();
+      if (tid == 0) S.left = 0;
+      if (left <= kSelCap) {
+        C.each(C.alive, [&](uint32_t, int64_t k, int) { S.list[atomicAdd(&S.cnt, 1)] = k; });
+        __syncthreads();
+        if (tid < kWave) {
+          const int kk = pick_wave<KIND, kSelCap / kWave>(
+              s, nb, N, rowmap, left, S.list, out, kept,
+              [&](int64_t key) { return (int)ctxL[(int)(key & MLP_KEY_MASK)]; }, lane);
+          if (tid == 0) S.kept = kk;
+        }
+        __syncthreads();
+        return S.kept;
+      }
+      if (kept >= kOneByOne) break;
+    }
+    for (int q = tid; q < kept; q += TB) {
+      const int i = (int)(out[q] >> 32), j = (int)(uint32_t)out[q];
+      claims_set(bits, N, KIND == 1 ? i : min(i, j), KIND == 1 ? j + 1 : max(i, j) + K);
+    }
+  }
   C.each(C.alive, [&](uint32_t, int64_t k, int) { mx = max(mx, cls(k)); });
-  if (tid == 0) S.top = S.cnt = 0;
-  __syncthreads();
   mx = wave_max_i32(mx);
-  if (lane == 0) atomicMax(&S.top, mx);
-  int left = M, kept = 0;
+  if (lane == kWave - 1) atomicMax(&S.top, mx);
+  __syncthreads();
   for (;;) {
     int top = 0, cut = 0;
     if (left > kSelCap) {
@@ -1631,11 +1809,11 @@ __device__ __forceinline__ int select_swaps(const Slot& s, int N, int rowmap, in
 // keys, whose first entries then hold the kept moves as (i << 32 | j).
 // cap: entries of the LDS buffer (the keys' own, or at lds when GMEM); a
 // selection runs where it holds what the selection needs.  p32: |delta| < 2^31.
-// Swaps are selected from 65 candidates on, spans from 257 on (a slice).
+// Swaps are selected from 65 candidates on, spans from 257 on; below that
+// wave 0 picks.
 // First merges of a solve, whole sort and serial greedy before and now:
-// n = 9001 swap 320 -> 83 us, 2-opt 116 -> 32, or-opt 240 -> 45; n = 1000
-// swap 30 -> 18, or-opt 24 -> 17.  Mean over a solve: k_mg_select n = 9001
-// 26.7 -> 11.4 us, k_merge_apply n = 1000 8.9 -> 7.9, n = 100 5.2 -> 4.3.
+// n = 9001 swap 320 -> 85 us, 2-opt 116 -> 18, or-opt 240 -> 50.  Mean over a
+// solve: k_mg_select n = 9001 26.7 -> 8.9 us, k_merge_apply n = 1000 8.9 -> 7.4.
 template <bool GMEM, int TB, typename Slot>
 __device__ __forceinline__ int sort_greedy(const Slot& s, int nb, int rowmap, int N, int M,
                                            int64_t* keys, int64_t* lds, int cap, bool p32,
@@ -1690,28 +1868,27 @@ __device__ __forceinline__ int sort_greedy(const Slot& s, int nb, int rowmap, in
     if (kept >= 0) return kept;
   }
   sk = GMEM && M <= cap ? lds : keys;
-  // Up to one key per lane of a wave: rank sort on wave 0, which also runs the
-  // greedy next (the keys are distinct; a key's rank is the number of smaller
-  // keys, each broadcast from its lane).  Up to 256 the same over the
-  // workgroup, else a bitonic sort.
   auto ctx_of = [&](int64_t key) { return (int)ctxL[(int)(key & MLP_KEY_MASK)]; };
-  if (M <= kWave) {
+  // Few candidates: wave 0 picks them one by one
+  if (M <= kWave || (nb > 0 && M <= kSelCap)) {
     if (tid < kWave) {
-      const int64_t my = tid < M ? keys[tid] : MLP_KEY_NONE;
-      const int c = tid < M ? ctx_of(my) : 0;
-      int rank = 0;
-      for (int u = 0; u < M; u += 4) {
-#pragma unroll
-        for (int x = 0; x < 4; ++x) rank += readlane64(my, u + x) < my ? 1 : 0;
-      }
-      if (tid < M) {
-        S.list[rank] = my;
-        S.hist[256 + rank] = c;
-      }
-      __builtin_amdgcn_wave_barrier();
+      int kept;
+      if (nb == 0) kept = pick_wave<0, 1>(s, nb, N, rowmap, M, keys, sk, 0, ctx_of, tid);
+      else if (nb == 1)
+        kept = M <= kWave ? pick_wave<1, 1>(s, nb, N, rowmap, M, keys, sk, 0, ctx_of, tid)
+                          : pick_wave<1, 4>(s, nb, N, rowmap, M, keys, sk, 0, ctx_of, tid);
+      else
+        kept = M <= kWave ? pick_wave<2, 1>(s, nb, N, rowmap, M, keys, sk, 0, ctx_of, tid)
+                          : pick_wave<2, 4>(s, nb, N, rowmap, M, keys, sk, 0, ctx_of, tid);
+      if (tid == 0) S.kept = kept;
     }
-    in = S.list;
-  } else if (M <= kSelCap) {
+    __syncthreads();
+    const int kept = S.kept;
+    if (kept >= 0) return kept;
+    __syncthreads();
+  }
+  // Up to 256 candidates a rank sort over the workgroup, else a bitonic sort.
+  if (M <= kSelCap) {
     if (tid < M) S.list[tid] = keys[tid];
     __syncthreads();
     rank_sort<TB>(S.list, M, S.hist, [&](int e) { return ctx_of(S.list[e]); });
