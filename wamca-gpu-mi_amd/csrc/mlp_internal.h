@@ -178,6 +178,11 @@ struct FusedPlan {
 #define MLP_SLOTS_INLINE 128
 // 64-bit word ranges of a slot block holding row buffers (set to KEY_NONE
 // when the slot is created)
+// Row buffers read by mlp_eval_static's output.
+struct RowsOut {
+  const int64_t* p[MLP_NB_COUNT];
+};
+
 struct SlotInitRows {
   int64_t start[MLP_NB_MAX];
   int64_t count[MLP_NB_MAX];

@@ -889,6 +889,38 @@ __global__ __launch_bounds__(TB) void k_prep(const SlotDev* __restrict__ table,
   }
 }
 
+// Start of a one-call evaluation of a tour in device memory: block 0 writes
+// the slot's table entry and info words and builds its prefix arrays, the
+// others empty the row buffers, all in one launch (k_slot_init and k_prep, one
+// after the other, took 3.4 and 4.6 us at n = 1000, each mostly its launch and
+// the wait for the table; the whole call 17.2 -> 14.8 us, n = 100 16.3 -> 13.0).
+template <int TB, int PER>
+__global__ __launch_bounds__(TB) void k_static_begin(SlotDev* table, SlotDev d) {
+  const int tid = threadIdx.x;
+  if (blockIdx.x > 0) {
+    const int pairs = d.rowcap;  // two buffers of rowcap keys each
+    for (int nb = 0; nb < MLP_NB_COUNT; ++nb)
+      for (int t = (blockIdx.x - 1) * TB + tid; t < pairs; t += (gridDim.x - 1) * TB)
+        ((gptr<long2v>)d.rows[nb])[t] = long2v{MLP_KEY_NONE, MLP_KEY_NONE};
+    return;
+  }
+  __shared__ PrepWaves<TB> P;
+  SlotRegs s;
+  s.N = d.N; s.n = d.n; s.round = d.round; s.maxd = d.maxd; s.small = d.small; s.rowcap = d.rowcap;
+#define MLP_FIELD(F) s.F = (decltype(s.F))d.F
+  MLP_FIELD(xs); MLP_FIELD(ys); MLP_FIELD(tour); MLP_FIELD(xy); MLP_FIELD(w); MLP_FIELD(t32);
+  MLP_FIELD(q32); MLP_FIELD(g32); MLP_FIELD(h32); MLP_FIELD(t64); MLP_FIELD(q64); MLP_FIELD(blk);
+  MLP_FIELD(info);
+#undef MLP_FIELD
+  s.rows = s.kcost = nullptr;
+  s.kij = nullptr;
+  prep_tour<TB, PER>(s, s.tour, P, nullptr, nullptr, false);
+  if (tid == 0) *table = d;
+  // the words that prep_tour does not write
+  if (tid < MLP_INFO_WORDS && tid != MLP_INFO_LATENCY && tid != MLP_INFO_TTOT && tid != MLP_INFO_PATH32)
+    s.info[tid] = tid == MLP_INFO_ACTIVE;
+}
+
 // Start of a DVND run: every listed slot becomes active with no rounds; the
 // summaries of its position blocks are written (the run's merges keep them up
 // to date, other rebuilds of a tour leave them).
@@ -2569,37 +2601,48 @@ __device__ __forceinline__ uint64_t move64_of(int64_t key, int nb, int rowmap, i
 }
 
 // Rows of the last evaluation of nb (the buffer info[PARITY0 + nb] names).
-__global__ void k_rows_moves64(const SlotDev* __restrict__ table, int id, int nb, int rowmap,
-                               int R, uint64_t* out) {
-  const SlotDev& s = table[id];
-  const int par = (int)(s.info[MLP_INFO_PARITY0 + nb] & 1);
-  const int64_t* keys = s.rows[nb] + (par ? s.rowcap : 0);
-  for (int r = blockIdx.x * kBlock + threadIdx.x; r < R; r += gridDim.x * kBlock)
-    out[r] = move64_of(keys[r], nb, rowmap, s.N, r);
+// The slot's fields come with the launch and both buffers' keys are loaded
+// beside the parity: one wait instead of a chain of three (8 tours n = 4001,
+// evaluation and 40 of these: 500 -> 495 us).
+__global__ __launch_bounds__(kBlock) void k_rows_moves64(gptr<const int64_t> info,
+                                                         gptr<const int64_t> rows, int rowcap, int N,
+                                                         int nb, int rowmap, int R,
+                                                         gptr<uint64_t> out) {
+  const int64_t parity = info[MLP_INFO_PARITY0 + nb];
+  for (int r = blockIdx.x * kBlock + threadIdx.x; r < R; r += gridDim.x * kBlock) {
+    const int64_t a = rows[r], b = rows[rowcap + r];
+    out[r] = move64_of((parity & 1) ? b : a, nb, rowmap, N, r);
+  }
 }
 
-// Rows of the last evaluation of every neighborhood in mask (ids 0..4, in
-// id order, rows_of(nb) entries each) as cost (INT64_MAX without a move),
-// i and j: the records mlp_get_rows returns, written to device arrays.
-__global__ void k_rows_out(const SlotDev* __restrict__ table, int id, int mask, int rowmap,
-                           int total, int64_t* cost, int32_t* oi, int32_t* oj) {
-  const SlotDev& s = table[id];
+// Rows of an evaluation of every neighborhood in mask (ids 0..4, in id order,
+// rows_of(nb) entries each) as cost (INT64_MAX without a move), i and j: the
+// records mlp_get_rows returns, written to device arrays.  rows.p[nb]: the
+// buffer the evaluation wrote.
+__global__ __launch_bounds__(kBlock) void k_rows_out(RowsOut rows, int N, int mask, int rowmap,
+                                                     int total, gptr<int64_t> cost,
+                                                     gptr<int32_t> oi, gptr<int32_t> oj) {
   for (int e = blockIdx.x * kBlock + threadIdx.x; e < total; e += gridDim.x * kBlock) {
-    int nb = 0, r = e;
-    for (; nb < MLP_NB_COUNT; ++nb) {
-      if (!((mask >> nb) & 1)) continue;
-      const int R = max(rows_of(nb, rowmap, s.N), 0);
-      if (r < R) break;
-      r -= R;
+    int nb = -1, r = e;
+    const int64_t* p = nullptr;
+    int first = 0;
+#pragma unroll
+    for (int q = 0; q < MLP_NB_COUNT; ++q) {
+      const int R = (mask >> q) & 1 ? max(rows_of(q, rowmap, N), 0) : 0;
+      if (e >= first && e < first + R) {
+        nb = q;
+        r = e - first;
+        p = rows.p[q];
+      }
+      first += R;
     }
-    if (nb >= MLP_NB_COUNT) continue;
-    const int par = (int)(s.info[MLP_INFO_PARITY0 + nb] & 1);
-    const int64_t key = s.rows[nb][(par ? s.rowcap : 0) + r];
+    if (nb < 0) continue;
+    const int64_t key = ldg(p + r);
     int i = 0, j = 0;
     int64_t c = INT64_MAX;
     if (key != MLP_KEY_NONE) {
       c = key >> MLP_KEY_SHIFT;
-      move_ij(nb, rowmap, s.N, r, (int)(key & MLP_KEY_MASK), i, j);
+      move_ij(nb, rowmap, N, r, (int)(key & MLP_KEY_MASK), i, j);
     }
     cost[e] = c;
     oi[e] = i;
@@ -4070,6 +4113,18 @@ hipError_t mlp_launch_prep(hipStream_t st, const SlotDev* table, const SlotListI
   return hipGetLastError();
 }
 
+hipError_t mlp_launch_static_begin(hipStream_t st, SlotDev* table, const SlotDev& d) {
+#define MLP_STATIC(TB, PER)                                                                       \
+  hipLaunchKernelGGL((k_static_begin<TB, PER>), dim3(1 + (d.rowcap + TB - 1) / TB), dim3(TB), 0, st, \
+                     table, d)
+  if (d.N <= 256) MLP_STATIC(256, 1);
+  else if (d.N <= 1024) MLP_STATIC(1024, 1);
+  else if (d.N <= 2048) MLP_STATIC(1024, 2);
+  else MLP_STATIC(1024, 4);
+#undef MLP_STATIC
+  return hipGetLastError();
+}
+
 hipError_t mlp_launch_dvnd_start(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
                                  const int32_t* list_dev, int count) {
   hipLaunchKernelGGL(k_dvnd_start, dim3(count), dim3(kBlock), 0, st, table, inl, list_dev);
@@ -4314,19 +4369,20 @@ hipError_t mlp_launch_ads(hipStream_t st, const SlotDev* table, int id, int N, u
   return hipGetLastError();
 }
 
-hipError_t mlp_launch_rows_moves64(hipStream_t st, const SlotDev* table, int id, int nb,
-                                  int rowmap, int R, uint64_t* out) {
+hipError_t mlp_launch_rows_moves64(hipStream_t st, const SlotDev& d, int nb, int rowmap, int R,
+                                   uint64_t* out) {
   const int grid = std::max(1, std::min((R + kBlock - 1) / kBlock, 1024));
-  hipLaunchKernelGGL(k_rows_moves64, dim3(grid), dim3(kBlock), 0, st, table, id, nb, rowmap, R,
-                     out);
+  hipLaunchKernelGGL(k_rows_moves64, dim3(grid), dim3(kBlock), 0, st, (gptr<const int64_t>)d.info,
+                     (gptr<const int64_t>)d.rows[nb], d.rowcap, d.N, nb, rowmap, R,
+                     (gptr<uint64_t>)out);
   return hipGetLastError();
 }
 
-hipError_t mlp_launch_rows_out(hipStream_t st, const SlotDev* table, int id, int mask, int rowmap,
-                              int total, int64_t* cost, int32_t* i, int32_t* j) {
+hipError_t mlp_launch_rows_out(hipStream_t st, const RowsOut& rows, int N, int mask, int rowmap,
+                               int total, int64_t* cost, int32_t* i, int32_t* j) {
   const int grid = std::max(1, std::min((total + kBlock - 1) / kBlock, 1024));
-  hipLaunchKernelGGL(k_rows_out, dim3(grid), dim3(kBlock), 0, st, table, id, mask, rowmap, total,
-                     cost, i, j);
+  hipLaunchKernelGGL(k_rows_out, dim3(grid), dim3(kBlock), 0, st, rows, N, mask, rowmap, total,
+                     (gptr<int64_t>)cost, (gptr<int32_t>)i, (gptr<int32_t>)j);
   return hipGetLastError();
 }
 

@@ -11,6 +11,9 @@
 // max_n: the largest N among the slots.
 hipError_t mlp_launch_prep(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
                            const int32_t* list_dev, int count, int max_n);
+// The slot of a one-call evaluation: table entry d, info words, prefix arrays
+// of d.tour, empty row buffers of ids 0 .. MLP_NB_COUNT-1.
+hipError_t mlp_launch_static_begin(hipStream_t st, SlotDev* table, const SlotDev& d);
 hipError_t mlp_launch_dvnd_start(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
                                  const int32_t* list_dev, int count);
 hipError_t mlp_launch_round_begin(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
@@ -71,10 +74,10 @@ hipError_t mlp_sort_pairs_u64(void* tmp, size_t* tmp_bytes, const uint64_t* kin,
 hipError_t mlp_launch_ads(hipStream_t st, const SlotDev* table, int id, int N, uint32_t* S,
                           uint32_t* out);
 // MLMove64 words of the rows of the last evaluation of nb / of TOTAL entries.
-hipError_t mlp_launch_rows_moves64(hipStream_t st, const SlotDev* table, int id, int nb,
-                                  int rowmap, int R, uint64_t* out);
-hipError_t mlp_launch_rows_out(hipStream_t st, const SlotDev* table, int id, int mask, int rowmap,
-                              int total, int64_t* cost, int32_t* i, int32_t* j);
+hipError_t mlp_launch_rows_moves64(hipStream_t st, const SlotDev& d, int nb, int rowmap, int R,
+                                   uint64_t* out);
+hipError_t mlp_launch_rows_out(hipStream_t st, const RowsOut& rows, int N, int mask, int rowmap,
+                               int total, int64_t* cost, int32_t* i, int32_t* j);
 hipError_t mlp_launch_total_moves64(hipStream_t st, const int64_t* tk, int64_t M, int B, int nb,
                                    int N, uint64_t* out);
 hipError_t mlp_launch_dist_table(hipStream_t st, int s0, int count, int round, int32_t* out);

@@ -2444,7 +2444,7 @@ int mlp_rows_moves64_device(mlp_ctx* ctx, int32_t slot, int32_t nb, uint64_t* de
   const int R = std::max(0, rows_of(nb, rm, s.N));
   if (R > cap) return fail(ctx, MLP_EINVAL, "%d rows do not fit %lld entries", R, (long long)cap);
   if (rows) *rows = R;
-  if (R > 0) HCK(mlp_launch_rows_moves64(ctx->stream, ctx->d_table, slot, nb, rm, R, dev));
+  if (R > 0) HCK(mlp_launch_rows_moves64(ctx->stream, s.dev, nb, rm, R, dev));
   return MLP_OK;
 }
 
@@ -2561,22 +2561,15 @@ int mlp_eval_static(mlp_ctx* ctx, int32_t inst, const int32_t* tour, uint32_t nb
   d.blk = (BlkSum*)(b + L.blk);
   d.info = (int64_t*)(b + L.info);
   d.nbs = MLP_NB_COUNT;
-  SlotInitRows rows{};
-  rows.nbs = d.nbs;
+  RowsOut rows{};
   for (int nb = 0; nb < d.nbs; ++nb) {
     d.rows[nb] = (int64_t*)(b + L.rows[nb]);
     d.kept_cost[nb] = (int64_t*)(b + L.kc[nb]);
     d.kept_ij[nb] = (int32_t*)(b + L.kij[nb]);
-    rows.start[nb] = (int64_t)(L.rows[nb] / 8);
-    rows.count[nb] = 2 * (int64_t)d.rowcap;
+    rows.p[nb] = d.rows[nb] + d.rowcap;
   }
   d.mscratch = nullptr;
-  // the block is cleared by a kernel (info zero, row buffers KEY_NONE) and
-  // the table entry written with it; then the ADS of the tour
-  HCK(mlp_launch_slot_init(ctx->stream, table, 0, d, (int64_t*)b, (int64_t)(L.ms / 8), rows));
-  SlotListInline one{};
-  one.id[0] = 0;
-  HCK(mlp_launch_prep(ctx->stream, table, one, nullptr, 1, N));
+  HCK(mlp_launch_static_begin(ctx->stream, table, d));
   // every neighborhood writes buffer 1 (the first tile records it)
   int total_rows = 0;
   for (int nb = 0; nb < MLP_NB_COUNT; ++nb)
@@ -2617,8 +2610,7 @@ int mlp_eval_static(mlp_ctx* ctx, int32_t inst, const int32_t* tour, uint32_t nb
       HCK(mlp_launch_sweep(ctx->stream, tile, table, segs, nullptr, nsegs, total, nullptr, total, 0));
   }
   if (total_rows > 0)
-    HCK(mlp_launch_rows_out(ctx->stream, table, 0, (int)nb_mask, rowmap, total_rows, cost, is,
-                            js));
+    HCK(mlp_launch_rows_out(ctx->stream, rows, N, (int)nb_mask, rowmap, total_rows, cost, is, js));
   return MLP_OK;
 }
 
