@@ -162,8 +162,8 @@ struct FusedPlan {
   int32_t group;              // tiles per eval item (one wait, one signal)
   int32_t* sync;              // [4 + 2 count]: work, exits, timeout flag, -, done[count], merged[count]
 };
-// positions per workgroup of the many-workgroup merge stages (kBlock threads
-// x 8 positions)
+// positions per workgroup of the many-workgroup merge's compaction (kBlock
+// threads x 8 positions)
 #define MLP_MG_CHUNK 2048
 #define MLP_FUSED_R 8
 #define MLP_FUSED_C 512

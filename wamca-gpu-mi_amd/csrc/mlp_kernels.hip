@@ -479,132 +479,6 @@ template <int PER, typename Slot>
 __device__ __forceinline__ void put_summary(const Slot& s, int p0, const int (&xy)[PER + 2],
                                             const int (&w)[PER + 1]);
 
-struct PrepLds {
-  int64_t wt[kBlock / kWave][2];
-  int64_t carry[2];  // T, Q before this segment
-  int64_t lsum[kBlock / kWave];
-};
-
-// One segment of kBlock * kPrepPer positions from `base` (thread t owns
-// kPrepPer consecutive positions): w, T and Q (offset by carryT, carryQ,
-// the prefixes before the segment) and the 2-opt constants G, H; WRITE
-// false only sums.  segT / segQ receive the segment's sums of w and p w, lacc
-// gains the thread's share of sum_p T[p].  Ends with every thread past its
-// reads of P.wt.
-// xyc: packed coordinates indexed by client (the merge's copy of the old
-// tour's xy, so the new tour needs no gather from the instance arrays), or
-// nullptr to read the instance arrays.
-template <bool WRITE>
-__device__ __forceinline__ void prep_segment(const SlotDev& s, const int32_t* tour, const int32_t* xyc,
-                                             int base, int64_t carryT, int64_t carryQ, PrepLds& P,
-                                             int64_t& segT, int64_t& segQ, int64_t& lacc,
-                                             bool sum = false) {
-  const int N = s.N, tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-  const float dr = round_dr(s.round);
-  const int p0 = base + tid * kPrepPer;
-  // xy of positions p0 - 1 .. p0 + kPrepPer (clamped into the tour): every
-  // client id is loaded before the first coordinate gather
-  int cl[kPrepPer + 2], xy[kPrepPer + 2];
-#pragma unroll
-  for (int e = 0; e < kPrepPer + 2; ++e) cl[e] = tour[min(max(p0 - 1 + e, 0), N - 1)];
-#pragma unroll
-  for (int e = 0; e < kPrepPer + 2; ++e) {
-    // client ids clamped into the instance: a tour read from caller memory
-    // never indexes outside the coordinate arrays
-    const int c = min(max(cl[e], 0), s.n - 1);
-    xy[e] = xyc ? xyc[c] : (ldg(s.xs + c) << 16) | ldg(s.ys + c);
-  }
-  int w[kPrepPer + 1];  // w[e]: edge into position p0 + e
-#pragma unroll
-  for (int e = 0; e <= kPrepPer; ++e) {
-    const int p = p0 + e;
-    w[e] = (p >= 1 && p < N) ? dist_xy(xy[e], xy[e + 1], dr) : 0;
-  }
-  if (WRITE && sum) put_summary<kPrepPer>(s, p0, xy, w);
-  int64_t lt[kPrepPer], lq[kPrepPer], at = 0, aq = 0;
-#pragma unroll
-  for (int e = 0; e < kPrepPer; ++e) {
-    at += w[e];
-    aq += (int64_t)(p0 + e) * w[e];
-    lt[e] = at;
-    lq[e] = aq;
-  }
-  const int64_t it = wave_scan_incl(at, lane), iq = wave_scan_incl(aq, lane);
-  if (lane == kWave - 1) {
-    P.wt[wave][0] = it;
-    P.wt[wave][1] = iq;
-  }
-  __syncthreads();
-  int64_t offT = carryT + it - at, offQ = carryQ + iq - aq;
-  segT = 0;
-  segQ = 0;
-#pragma unroll
-  for (int q = 0; q < kBlock / kWave; ++q) {
-    if (q < wave) {
-      offT += P.wt[q][0];
-      offQ += P.wt[q][1];
-    }
-    segT += P.wt[q][0];
-    segQ += P.wt[q][1];
-  }
-  if (WRITE) {
-    int32_t vt[kPrepPer], vq[kPrepPer], vg[kPrepPer], vh[kPrepPer];
-    int64_t T8[kPrepPer], Q8[kPrepPer];
-#pragma unroll
-    for (int e = 0; e < kPrepPer; ++e) {
-      const int p = p0 + e;
-      const int64_t T = offT + lt[e], Q = offQ + lq[e];
-      T8[e] = T;
-      Q8[e] = Q;
-      vt[e] = (int32_t)(uint32_t)(uint64_t)T;
-      vq[e] = (int32_t)(uint32_t)(uint64_t)Q;
-      const uint32_t Z = 2u * (uint32_t)(uint64_t)Q - (uint32_t)(2 * p + 1) * (uint32_t)(uint64_t)T;
-      vg[e] = (int32_t)(0u - (uint32_t)(N - p) * (uint32_t)w[e] - Z);
-      vh[e] = (int32_t)(Z - (uint32_t)(N - p - 1) * (uint32_t)w[e + 1]);
-      if (p < N) lacc += T;
-    }
-    if (p0 + kPrepPer <= N) {
-      // the thread's eight consecutive positions as 16-byte stores (p0 is a
-      // multiple of 8 and every array 256-byte aligned): a quarter of the
-      // store instructions of one word per position
-      auto put4 = [](int32_t* d, int a, int b, int c, int e) { *(int4*)d = make_int4(a, b, c, e); };
-      auto put2 = [](int64_t* d, int64_t a, int64_t b) {
-        *(longlong2*)d = make_longlong2((long long)a, (long long)b);
-      };
-#pragma unroll
-      for (int h = 0; h < kPrepPer; h += 4) {
-        put4(s.xy + p0 + h, xy[h + 1], xy[h + 2], xy[h + 3], xy[h + 4]);
-        put4(s.w + p0 + h, w[h], w[h + 1], w[h + 2], w[h + 3]);
-        put4(s.t32 + p0 + h, vt[h], vt[h + 1], vt[h + 2], vt[h + 3]);
-        put4(s.q32 + p0 + h, vq[h], vq[h + 1], vq[h + 2], vq[h + 3]);
-        put4(s.g32 + p0 + h, vg[h], vg[h + 1], vg[h + 2], vg[h + 3]);
-        put4(s.h32 + p0 + h, vh[h], vh[h + 1], vh[h + 2], vh[h + 3]);
-      }
-#pragma unroll
-      for (int h = 0; h < kPrepPer; h += 2) {
-        put2(s.t64 + p0 + h, T8[h], T8[h + 1]);
-        put2(s.q64 + p0 + h, Q8[h], Q8[h + 1]);
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < kPrepPer; ++e) {
-        const int p = p0 + e;
-        if (p < N) {
-          s.xy[p] = xy[e + 1];
-          s.w[p] = w[e];
-          s.t64[p] = T8[e];
-          s.q64[p] = Q8[e];
-          s.t32[p] = vt[e];
-          s.q32[p] = vq[e];
-          s.g32[p] = vg[e];
-          s.h32[p] = vh[e];
-        }
-      }
-    }
-  }
-  __syncthreads();  // every thread has read wt
-}
-
 // The tour's T[N-1] and int32-path flags.
 template <typename Slot>
 __device__ __forceinline__ void prep_flags(const Slot& s, int64_t Ttot) {
@@ -735,18 +609,21 @@ __device__ __forceinline__ void put_words(P p, const int64_t (&v)[PER]) {
 // xyc: packed coordinates indexed by client (the merge's copy of the old
 // tour's xy, so the new tour needs no gather from the instance arrays), or
 // nullptr to read the instance arrays.  tour_out: where the tour is copied to
-// (nullptr: nowhere).  sum: block summaries too.
-template <int TB, int PER, typename Slot, typename Tour>
+// (nullptr: nowhere).  sum: block summaries too.  From position p_lo up to
+// p_hi only, given the prefixes before it (the info words come with the end of
+// the tour).
+template <int TB, int PER, typename Slot, typename Tour, typename Coord>
 __device__ __forceinline__ void prep_tour(const Slot& s, Tour tour, PrepWaves<TB>& P,
-                                          const int32_t* xyc, gptr<int32_t> tour_out, bool sum) {
+                                          Coord xyc, gptr<int32_t> tour_out, bool sum, int p_lo = 0,
+                                          int p_hi = MLP_MAX_N + 1, int carryT = 0,
+                                          int64_t carryQ = 0) {
   constexpr int NW = TB / kWave;
   const int N = s.N, tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const float dr = round_dr(s.round);
-  int carryT = 0;  // T[N-1] < 2^31 (every instance: N maxd < 2^30)
-  int64_t carryQ = 0;
+  // carryT, carryQ: T, Q so far; T[N-1] < 2^31 (every instance: N maxd < 2^30)
   int buf = 0;
-  for (int base = 0; base < N; base += TB * PER, buf ^= 1) {
+  for (int base = p_lo; base < min(N, p_hi); base += TB * PER, buf ^= 1) {
     const int p0 = base + tid * PER;
     // positions p0 - 1 .. p0 + PER (clamped into the tour): every client id is
     // loaded before the first coordinate gather
@@ -859,7 +736,7 @@ __device__ __forceinline__ void prep_tour(const Slot& s, Tour tour, PrepWaves<TB
       }
     }
   }
-  if (tid == 0) {  // positions past N-1 add nothing to the carries
+  if (tid == 0 && p_hi >= N) {  // positions past N-1 add nothing to the carries
     s.info[MLP_INFO_LATENCY] = (int64_t)N * carryT - carryQ;
     prep_flags(s, carryT);
   }
@@ -880,7 +757,7 @@ __global__ __launch_bounds__(TB) void k_prep(const SlotDev* __restrict__ table,
   __shared__ PrepWaves<TB> P;
   const int id = list_at(list, list_dev, blockIdx.x);
   const SlotRegs s = slot_regs(table, id, 0);
-  prep_tour<TB, PER>(s, s.tour, P, nullptr, nullptr, false);
+  prep_tour<TB, PER>(s, s.tour, P, (const int32_t*)nullptr, nullptr, false);
   if (threadIdx.x == 0) {
     s.info[MLP_INFO_ROUND_MOVES] = 0;
     s.info[MLP_INFO_TOTAL_MOVES] = 0;
@@ -914,7 +791,7 @@ __global__ __launch_bounds__(TB) void k_static_begin(SlotDev* table, SlotDev d) 
 #undef MLP_FIELD
   s.rows = s.kcost = nullptr;
   s.kij = nullptr;
-  prep_tour<TB, PER>(s, s.tour, P, nullptr, nullptr, false);
+  prep_tour<TB, PER>(s, s.tour, P, (const int32_t*)nullptr, nullptr, false);
   if (tid == 0) *table = d;
   // the words that prep_tour does not write
   if (tid < MLP_INFO_WORDS && tid != MLP_INFO_LATENCY && tid != MLP_INFO_TTOT && tid != MLP_INFO_PATH32)
@@ -2133,13 +2010,12 @@ __global__ __launch_bounds__(TB) void k_merge_apply(const SlotDev* __restrict__ 
 //                 copied to told / tnew, the coordinates by client;
 //   k_mg_select   one workgroup per slot: sort, greedy, the kept moves'
 //                 spans written into tnew, the merge's and round's counters;
-//   k_mg_sums     per segment of the new tour: sums of w and p w;
-//   k_mg_rebuild  per segment: the prefix arrays with the preceding
-//                 segments' sums as carries, the tour, the latency (one
-//                 atomic add per segment), T[N-1] and the int32 flags.
+//   k_mg_rebuild  per segment of 1024 positions of the new tour: the prefixes
+//                 before it, summed from the edges, then the prefix arrays
+//                 and the tour; the last segment the latency, T[N-1] and the
+//                 int32 flags.
 // The one-workgroup merge runs these steps one after another over the whole
 // tour; here the O(N) steps are spread over the GPU.
-static_assert(MLP_MG_CHUNK == kBlock * kPrepPer, "one segment per workgroup");
 
 struct MgArrays {
   int64_t* keys;
@@ -2147,12 +2023,10 @@ struct MgArrays {
   int32_t* tnew;
   int32_t* xyc;
   uint16_t* ctxL;
-  int64_t* csum;  // [segments][2]
 };
 
 // The slot's global working arrays: the one-workgroup merge's layout
-// (keys[pcap] | told[N] | tnew[N] | xyc[N] | bitmap | ctx[pcap]), then the
-// segment sums.
+// (keys[pcap] | told[N] | tnew[N] | xyc[N] | bitmap | ctx[pcap]).
 __device__ __forceinline__ MgArrays mg_arrays(const SlotDev* table, int id) {
   const auto& s = *((const __attribute__((address_space(4))) SlotDev*)table +
                     __builtin_amdgcn_readfirstlane(id));
@@ -2165,7 +2039,6 @@ __device__ __forceinline__ MgArrays mg_arrays(const SlotDev* table, int id) {
   a.tnew = a.told + N;
   a.xyc = a.tnew + N;
   a.ctxL = (uint16_t*)((uint32_t*)(a.xyc + N) + claim_words(N));
-  a.csum = (int64_t*)(((uintptr_t)(a.ctxL + pcap) + 7) & ~(uintptr_t)7);
   return a;
 }
 
@@ -2252,57 +2125,60 @@ __global__ __launch_bounds__(kSelBlock) void k_mg_select(const SlotDev* __restri
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_mg_sums(const SlotDev* __restrict__ table,
-                                                    SlotListInline list, const int32_t* list_dev) {
-  __shared__ PrepLds P;
+// Each segment sums the edges before it again, a thread a run of neighbouring
+// positions: at most N / 1024 edges a thread, instead of a launch of its own
+// for the segments' sums (2048 positions by 256 threads each: 4.9 us for the
+// sums and 8.2 us for the rebuild at n = 9001; 10.1 us now).
+constexpr int kRebuild = 1024;
+__global__ __launch_bounds__(kRebuild) void k_mg_rebuild(const SlotDev* __restrict__ table,
+                                                         SlotListInline list,
+                                                         const int32_t* list_dev, int sum) {
+  constexpr int NW = kRebuild / kWave;
+  __shared__ PrepWaves<kRebuild> P;
+  __shared__ int64_t wsum[NW][2];
   const int id = list_at(list, list_dev, blockIdx.y);
-  const SlotDev& s = table[id];
-  if (s.info[MLP_INFO_MG_APPLY] == 0) return;
-  const int base = blockIdx.x * MLP_MG_CHUNK;
-  if (base >= s.N) return;
+  const SlotRegs s = slot_regs(table, id, 0);
+  const int N = s.N, base = blockIdx.x * kRebuild, tid = threadIdx.x;
   const MgArrays a = mg_arrays(table, id);
-  int64_t segT, segQ, lacc = 0;
-  prep_segment<false>(s, a.tnew, a.xyc, base, 0, 0, P, segT, segQ, lacc);
-  if (threadIdx.x == 0) {
-    a.csum[2 * blockIdx.x] = segT;
-    a.csum[2 * blockIdx.x + 1] = segQ;
-    if (blockIdx.x == 0) s.info[MLP_INFO_LATENCY] = 0;  // k_mg_rebuild adds the segments
-  }
-}
-
-__global__ __launch_bounds__(kBlock) void k_mg_rebuild(const SlotDev* __restrict__ table,
-                                                       SlotListInline list,
-                                                       const int32_t* list_dev, int sum) {
-  __shared__ PrepLds P;
-  const int id = list_at(list, list_dev, blockIdx.y);
-  const SlotDev& s = table[id];
-  if (s.info[MLP_INFO_MG_APPLY] == 0) return;
-  const int N = s.N, base = blockIdx.x * MLP_MG_CHUNK;
-  if (base >= N) return;
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-  const MgArrays a = mg_arrays(table, id);
-  const int nseg = (N + MLP_MG_CHUNK - 1) / MLP_MG_CHUNK;
-  int64_t cT = 0, cQ = 0, Ttot = 0;
-  for (int c = 0; c < nseg; ++c) {
-    const int64_t t = a.csum[2 * c], q = a.csum[2 * c + 1];
-    if (c < (int)blockIdx.x) {
-      cT += t;
-      cQ += q;
+  const auto tnew = (gptr<const int32_t>)a.tnew, xyc = (gptr<const int32_t>)a.xyc;
+  const int64_t applied = s.info[MLP_INFO_MG_APPLY];
+  if (applied == 0 || base >= N) return;
+  int64_t cT = 0, cQ = 0;
+  if (base > 0) {
+    // positions 1 .. base - 1, per = base / 1024 of them a thread
+    const int per = blockIdx.x, c0 = 1 + tid * per, c1 = min(c0 + per, base);
+    const float dr = round_dr(s.round);
+    constexpr int U = 8;
+    int last = xyc[tnew[min(c0, N) - 1]];
+    for (int p0 = c0; p0 < c1; p0 += U) {
+      int cl[U], xy[U];
+#pragma unroll
+      for (int e = 0; e < U; ++e) cl[e] = tnew[min(p0 + e, c1 - 1)];
+#pragma unroll
+      for (int e = 0; e < U; ++e) xy[e] = xyc[cl[e]];
+#pragma unroll
+      for (int e = 0; e < U; ++e) {
+        const int w = p0 + e < c1 ? dist_xy(last, xy[e], dr) : 0;
+        last = xy[e];
+        cT += w;
+        cQ += umul(p0 + e, w);
+      }
     }
-    Ttot += t;
+    cT = wave_sum64(cT);
+    cQ = wave_sum64(cQ);
+    if (tid % kWave == 0) {
+      wsum[tid / kWave][0] = cT;
+      wsum[tid / kWave][1] = cQ;
+    }
+    __syncthreads();
+    cT = cQ = 0;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {
+      cT += wsum[q][0];
+      cQ += wsum[q][1];
+    }
   }
-  int64_t segT, segQ, lacc = 0;
-  prep_segment<true>(s, a.tnew, a.xyc, base, cT, cQ, P, segT, segQ, lacc, sum != 0);
-  for (int p = base + tid; p < min(base + MLP_MG_CHUNK, N); p += kBlock) s.tour[p] = a.tnew[p];
-  const int64_t lw = wave_sum64(lacc);
-  if (lane == 0) P.lsum[wave] = lw;
-  __syncthreads();
-  if (tid == 0) {
-    int64_t L = 0;
-    for (int q = 0; q < kBlock / kWave; ++q) L += P.lsum[q];
-    atomicAdd((unsigned long long*)&s.info[MLP_INFO_LATENCY], (unsigned long long)L);
-    if (blockIdx.x == 0) prep_flags(s, Ttot);
-  }
+  prep_tour<kRebuild, 1>(s, tnew, P, xyc, s.tour, sum != 0, base, base + kRebuild, (int)cT, cQ);
 }
 
 // ---------------------------------------------------------------------------
@@ -2579,7 +2455,7 @@ __global__ __launch_bounds__(kBlock) void k_total_merge(const SlotDev* __restric
       [&](int q) { return ((int64_t)kij[3 * q] << 32) | (uint32_t)kij[3 * q + 1]; }, told, tnew,
       T.nlong, T.longq);
   __syncthreads();
-  prep_tour<kBlock, 8>(r, tnew, PL, nullptr, r.tour, false);
+  prep_tour<kBlock, 8>(r, tnew, PL, (const int32_t*)nullptr, r.tour, false);
   if (tid == 0) {
     s.info[MLP_INFO_KEPT0 + nb] = K;
     s.info[MLP_INFO_ROUND_MOVES] += K;
@@ -4304,9 +4180,8 @@ hipError_t mlp_launch_merge_gmem(hipStream_t st, const SlotDev* table, const Slo
                      skip_inactive);
   hipLaunchKernelGGL(k_mg_select, dim3(count), dim3(kSelBlock), kGmemMergeLds, st, table, inl,
                      list_dev, nb, rowmap, skip_inactive, tail);
-  hipLaunchKernelGGL(k_mg_sums, seg, dim3(kBlock), 0, st, table, inl, list_dev);
-  hipLaunchKernelGGL(k_mg_rebuild, seg, dim3(kBlock), 0, st, table, inl, list_dev,
-                     skip_inactive & 2);
+  hipLaunchKernelGGL(k_mg_rebuild, dim3((max_n + kRebuild - 1) / kRebuild, count), dim3(kRebuild), 0,
+                     st, table, inl, list_dev, skip_inactive & 2);
   return hipGetLastError();
 }
 

@@ -47,7 +47,7 @@ hipError_t mlp_launch_merge_apply(hipStream_t st, const SlotDev* table, const Sl
                                   const int32_t* list_dev, int count, int nb, int rowmap,
                                   int pcap, int ncap, int skip_inactive, int tail);
 // The merge of slots whose working arrays exceed LDS over many workgroups
-// per slot (four launches; max_n: the largest N among the slots).
+// per slot (three launches; max_n: the largest N among the slots).
 hipError_t mlp_launch_merge_gmem(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
                                  const int32_t* list_dev, int count, int nb, int rowmap,
                                  int skip_inactive, int tail, int max_n);

@@ -100,11 +100,8 @@ int merge_pcap(int N) {
   return p;
 }
 size_t merge_bytes(int N) { return mlp_merge_lds_bytes(merge_pcap(N), N); }
-// The merge's working arrays in the slot's device memory: that layout, then
-// the many-workgroup merge's per-segment sums.
-size_t merge_gmem_bytes(int N) {
-  return merge_bytes(N) + 8 + 16 * (size_t)((N + MLP_MG_CHUNK - 1) / MLP_MG_CHUNK);
-}
+// The merge's working arrays in the slot's device memory have that layout.
+size_t merge_gmem_bytes(int N) { return merge_bytes(N); }
 
 // Byte layout of one slot's device block.
 struct SlotLayout {
