@@ -2273,13 +2273,14 @@ __global__ void k_total_keys(const int64_t* __restrict__ tk, int64_t M, int B, u
 
 namespace {
 
-constexpr int kTotalPer = 8;                       // candidates per thread per chunk
-constexpr int kTotalChunk = kTotalPer * kBlock;    // candidates decoded per chunk
+constexpr int kTotalBlock = 1024;
+constexpr int kTotalPer = 8;                         // candidates per thread per chunk
+constexpr int kTotalChunk = kTotalPer * kTotalBlock;  // candidates decoded per chunk
 
 struct TotalLds {
-  int32_t ci[kTotalChunk], cj[kTotalChunk], ce[kTotalChunk];
-  int64_t cc[kTotalChunk];
-  int wc[kTotalPer][kBlock / kWave];
+  int64_t cc[kTotalChunk];  // a surviving candidate's cost
+  int32_t cv[kTotalChunk];  // and its row << 15 | ctx
+  int wc[kTotalPer][kTotalBlock / kWave];
   int end, kept, nlong;
   int longq[kLongMoves];
 };
@@ -2288,7 +2289,7 @@ struct TotalLds {
 // list of `base` moves: same batch logic as greedy_wave.
 template <int NB>
 __device__ int greedy_list(const SlotDev& s, int S, const TotalLds& T, uint32_t* bits, int lane,
-                           int base_kept) {
+                           int base_kept, int B) {
   constexpr int K = NB >= 2 ? NB - 1 : 0;
   // slot fields in registers (the loop's global stores would reload them)
   const int n = s.N;
@@ -2298,7 +2299,9 @@ __device__ int greedy_list(const SlotDev& s, int S, const TotalLds& T, uint32_t*
   for (int base = 0; base < S; base += kWave) {
     const int t = base + lane;
     const bool valid = t < S;
-    const int i = valid ? T.ci[t] : 0, j = valid ? T.cj[t] : 0;
+    const int row = valid ? T.cv[t] >> 15 : 0, ctx = valid ? T.cv[t] & 0x7fff : 0;
+    int i = 0, j = 0;
+    if (valid) move_ij(NB, 0, n, row, ctx, i, j);
     const int a = NB == 1 ? i : min(i, j);
     const int b = NB == 1 ? j + 1 : max(i, j) + K;
     bool pre = valid;
@@ -2328,7 +2331,7 @@ __device__ int greedy_list(const SlotDev& s, int S, const TotalLds& T, uint32_t*
       kcost[q] = T.cc[t];
       kij[3 * q + 0] = i;
       kij[3 * q + 1] = j;
-      kij[3 * q + 2] = T.ce[t];
+      kij[3 * q + 2] = row * B + ctx % B;
     }
     kept_total += __popcll(kept);
   }
@@ -2342,17 +2345,20 @@ __device__ int greedy_list(const SlotDev& s, int S, const TotalLds& T, uint32_t*
 // candidates that already conflict with a kept move (the kept set only
 // grows, so they would be dropped anyway), keeping the survivors in order;
 // wave 0 then runs the greedy over the survivors while the next chunk's keys
-// are already being loaded.  The first non-improving key ends the list.
+// are already being loaded.  The first non-improving key ends the list.  The
+// first chunk, which nothing filters, is one candidate a thread; the rest of
+// the list (0.4 million candidates at n = 1000 and 896 thread slots) costs its
+// chunks' barriers and decoding: 256 threads 1344 us, 1024 threads 416.
 // Dynamic LDS: bits | told[N] | tnew[N] (told/tnew in the slot's merge
 // scratch when GMEM).
 template <bool GMEM>
-__global__ __launch_bounds__(kBlock) void k_total_merge(const SlotDev* __restrict__ table, int id,
+__global__ __launch_bounds__(kTotalBlock) void k_total_merge(const SlotDev* __restrict__ table, int id,
                                                         int nb, int B, int64_t M, uint64_t bias,
                                                         const uint64_t* __restrict__ ku,
                                                         const int32_t* __restrict__ ve) {
   extern __shared__ int64_t lds[];
   __shared__ TotalLds T;
-  __shared__ PrepWaves<kBlock> PL;
+  __shared__ PrepWaves<kTotalBlock> PL;
   const SlotDev& s = table[id];
   const int N = s.N, tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const int k = nb_k(nb);
@@ -2360,7 +2366,7 @@ __global__ __launch_bounds__(kBlock) void k_total_merge(const SlotDev* __restric
   uint32_t* bits = (uint32_t*)lds;
   int32_t* told = GMEM ? (int32_t*)s.mscratch : (int32_t*)(bits + nwords);
   int32_t* tnew = told + N;
-  for (int w = tid; w < nwords; w += kBlock) bits[w] = 0;
+  for (int w = tid; w < nwords; w += kTotalBlock) bits[w] = 0;
   if (tid == 0) {
     T.end = 0;
     T.kept = 0;
@@ -2371,39 +2377,36 @@ __global__ __launch_bounds__(kBlock) void k_total_merge(const SlotDev* __restric
   int32_t nv[kTotalPer];
 #pragma unroll
   for (int u = 0; u < kTotalPer; ++u) {
-    const int64_t q = (int64_t)u * kBlock + tid;
-    nk[u] = q < M ? ku[q] : bias;
-    nv[u] = q < M ? ve[q] : 0;
+    const int64_t q = (int64_t)u * kTotalBlock + tid;
+    nk[u] = u == 0 && q < M ? ku[q] : bias;
+    nv[u] = u == 0 && q < M ? ve[q] : 0;
   }
   __syncthreads();
-  for (int64_t base = 0; base < M; base += kTotalChunk) {
+  int size = kTotalBlock;  // of the chunk
+  for (int64_t base = 0; base < M; base += size, size = kTotalChunk) {
     uint64_t ck[kTotalPer];
     int32_t cv[kTotalPer];
 #pragma unroll
     for (int u = 0; u < kTotalPer; ++u) {
       ck[u] = nk[u];
       cv[u] = nv[u];
-      const int64_t q = base + kTotalChunk + (int64_t)u * kBlock + tid;
+      const int64_t q = base + size + (int64_t)u * kTotalBlock + tid;
       nk[u] = q < M ? ku[q] : bias;
       nv[u] = q < M ? ve[q] : 0;
     }
-    int ci[kTotalPer], cj[kTotalPer];
     uint64_t bal[kTotalPer];
     bool end = false;
 #pragma unroll
     for (int u = 0; u < kTotalPer; ++u) {
       bool pass = false;
-      ci[u] = cj[u] = 0;
       if (ck[u] < bias) {
         const int row = cv[u] >> 15, ctx = cv[u] & 0x7fff;
         int i, j;
         move_ij(nb, 0, N, row, ctx, i, j);
-        ci[u] = i;
-        cj[u] = j;
         if (nb == 0) pass = !claimed(bits, N, i) && !claimed(bits, N, j);
         else if (nb == 1) pass = !claims_any(bits, N, i, j + 1);
         else pass = !claims_any(bits, N, min(i, j), max(i, j) + k);
-      } else {
+      } else if (u * kTotalBlock < size) {
         end = true;  // past the list or the first non-improving key
       }
       bal[u] = __ballot(pass);
@@ -2415,16 +2418,13 @@ __global__ __launch_bounds__(kBlock) void k_total_merge(const SlotDev* __restric
 #pragma unroll
     for (int u = 0; u < kTotalPer; ++u) {
       int off = S;
-      for (int w = 0; w < kBlock / kWave; ++w) {
+      for (int w = 0; w < kTotalBlock / kWave; ++w) {
         if (w < wave) off += T.wc[u][w];
         S += T.wc[u][w];
       }
       if ((bal[u] >> lane) & 1ull) {
         const int at = off + __popcll(bal[u] & lt);
-        const int row = cv[u] >> 15, ctx = cv[u] & 0x7fff;
-        T.ci[at] = ci[u];
-        T.cj[at] = cj[u];
-        T.ce[at] = row * B + ctx % B;
+        T.cv[at] = cv[u];
         T.cc[at] = (int64_t)ck[u] - (int64_t)bias;
       }
     }
@@ -2434,7 +2434,7 @@ __global__ __launch_bounds__(kBlock) void k_total_merge(const SlotDev* __restric
     if (wave == 0 && S > 0) {
       int kept = T.kept;
 #define MLP_TGREEDY(NB) \
-  case NB: kept = greedy_list<NB>(s, S, T, bits, lane, kept); break
+  case NB: kept = greedy_list<NB>(s, S, T, bits, lane, kept, B); break
       switch (nb) {
         MLP_TGREEDY(0); MLP_TGREEDY(1); MLP_TGREEDY(2); MLP_TGREEDY(3); MLP_TGREEDY(4);
         MLP_TGREEDY(5); MLP_TGREEDY(6); MLP_TGREEDY(7); MLP_TGREEDY(8); MLP_TGREEDY(9);
@@ -2450,12 +2450,12 @@ __global__ __launch_bounds__(kBlock) void k_total_merge(const SlotDev* __restric
   const int K = T.kept;
   const SlotRegs r = slot_regs(table, id, nb);
   const auto kij = r.kij;
-  apply_kept<kBlock>(
+  apply_kept<kTotalBlock>(
       r, nb, K,
       [&](int q) { return ((int64_t)kij[3 * q] << 32) | (uint32_t)kij[3 * q + 1]; }, told, tnew,
       T.nlong, T.longq);
   __syncthreads();
-  prep_tour<kBlock, 8>(r, tnew, PL, (const int32_t*)nullptr, r.tour, false);
+  prep_tour<kTotalBlock, 4>(r, tnew, PL, (const int32_t*)nullptr, r.tour, false);
   if (tid == 0) {
     s.info[MLP_INFO_KEPT0 + nb] = K;
     s.info[MLP_INFO_ROUND_MOVES] += K;
@@ -4191,8 +4191,8 @@ size_t mlp_total_merge_lds_bytes(int N) {
 
 // The merge kernel's own static LDS (chunk arrays, prefix scratch) is below
 // kTotalStaticLds; its dynamic part may use the rest.
-constexpr size_t kTotalStaticLds = 48 * 1024;
-static_assert(sizeof(TotalLds) + sizeof(PrepWaves<kBlock>) <= kTotalStaticLds, "static LDS estimate");
+constexpr size_t kTotalStaticLds = 104 * 1024;
+static_assert(sizeof(TotalLds) + sizeof(PrepWaves<kTotalBlock>) <= kTotalStaticLds, "static LDS estimate");
 
 size_t mlp_total_static_lds() { return kTotalStaticLds; }
 
@@ -4226,10 +4226,10 @@ hipError_t mlp_launch_total_merge(hipStream_t st, const SlotDev* table, int id, 
                                   int B, int64_t M, uint64_t bias, const uint64_t* ku,
                                   const int32_t* ve, int gmem) {
   if (gmem)
-    hipLaunchKernelGGL(k_total_merge<true>, dim3(1), dim3(kBlock), (size_t)claim_words(N) * 4,
+    hipLaunchKernelGGL(k_total_merge<true>, dim3(1), dim3(kTotalBlock), (size_t)claim_words(N) * 4,
                        st, table, id, nb, B, M, bias, ku, ve);
   else
-    hipLaunchKernelGGL(k_total_merge<false>, dim3(1), dim3(kBlock), mlp_total_merge_lds_bytes(N),
+    hipLaunchKernelGGL(k_total_merge<false>, dim3(1), dim3(kTotalBlock), mlp_total_merge_lds_bytes(N),
                        st, table, id, nb, B, M, bias, ku, ve);
   return hipGetLastError();
 }
