@@ -1943,14 +1943,14 @@ __device__ __forceinline__ void merge_slot(const SlotRegs& s, int nb, int rowmap
 
   if (tid == 0) S.m = 0;
   for (int w = tid; w < nwords; w += TB) bits[w] = 0;
-  if (dvnd && active == 0) return;
   __syncthreads();
   // 1. improving rows -> (cost, row) keys.  Inside a DVND round the eval
   // wrote the buffer opposite info[PARITY0 + nb]; this merge commits it.
   // The tour (for the apply step) and its coordinates (for the prefix
   // rebuild, by client) are copied in the same loop, so their loads go out
-  // with the row keys'; both buffers' keys are loaded, so that the loads do
-  // not wait for the parity.
+  // with the row keys'; both buffers' keys are loaded, and whether the slot
+  // is active is looked at afterwards, so that no load waits for the info
+  // words (a merge n = 1000 7.4 -> 6.8 us, n = 100 4.3 -> 3.6).
   const int par = (int)(parity & 1) ^ (dvnd ? 1 : 0);
   const auto rk = s.rows;
   const int cap = s.rowcap;
@@ -1962,6 +1962,7 @@ __device__ __forceinline__ void merge_slot(const SlotRegs& s, int nb, int rowmap
       },
       [&](int64_t a, int64_t b) { return par ? b : a; }, R, 0, max(R, N), told, tnew, xyc, ctxL,
       [&](int64_t k) { keys[atomicAdd(&S.m, 1)] = k; });
+  if (dvnd && active == 0) return;
   __syncthreads();
   // every thread has read the old parity
   if (dvnd && tid == 0) s.info[MLP_INFO_PARITY0 + nb] = par;

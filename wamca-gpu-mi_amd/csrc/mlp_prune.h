@@ -48,6 +48,27 @@ constexpr int kPWg = kPR * kBlock / kWave;  // rows of a workgroup
 constexpr int kPMaxW = 1024;              // columns of a wave at most
 constexpr int kPMaxBlk = kPMaxW / MLP_BLK;
 
+// What a wave reads first: xy, w and T of position b0 + lane % 16, and the
+// summary of the lane's first block with T before it.  All of it is loaded
+// beside the slot's info words, before any of them is looked at (one wait
+// instead of three: n = 1000 FIRSTUS a neighborhood).
+struct PruneFirst {
+  int rxy, rw, rt, tp;
+  int4v sm;
+  __device__ __forceinline__ PruneFirst(const SlotDev& s, int b0, int wb0) {
+    const int lane = threadIdx.x % kWave, rp = min(b0 + (lane & 15), s.N - 1);
+    const int B = min(wb0 + lane, (s.N + MLP_BLK - 1) / MLP_BLK - 1);
+    rxy = ldg(s.xy + rp);
+    rw = ldg(s.w + rp);
+    rt = ldg(s.t32 + rp);
+    sm = *(gptr<const int4v>)(s.blk + B);
+    tp = ldg(s.t32 + max(B * MLP_BLK - 1, 0));
+  }
+  __device__ __forceinline__ void arrive() {
+    asm volatile("" : "+v"(rxy), "+v"(rw), "+v"(rt), "+v"(tp), "+v"(sm));
+  }
+};
+
 struct PruneLds {
   uint16_t list[kBlock / kWave][kPMaxBlk];  // surviving blocks of each wave
 };
@@ -98,9 +119,10 @@ __device__ __forceinline__ int box_gap(int alo, int ahi, int blo, int bhi, float
 
 // A wave's eight rows x W columns of neighborhood NB (0 swap, 1 2-opt,
 // 2..4 or-opt-1..3).  WIDE: 2-opt deltas or their bounds beyond 32 bits.
+// first: the loads that every wave begins with, issued by the caller.
 template <int NB, bool WIDE>
 __device__ __forceinline__ void prune_wave(const SlotDev& s, int b0, int ct, int W, uint16_t* list,
-                                           PruneDiag* G, int dlo, int par) {
+                                           PruneDiag* G, int dlo, int par, const PruneFirst& first) {
   constexpr int K = NB >= 2 ? NB - 1 : 0;
   // positions b0 + A0 .. b0 + A1 appear in the rows' distances
   constexpr int A0 = NB >= 2 ? 1 : 0;
@@ -125,7 +147,7 @@ __device__ __forceinline__ void prune_wave(const SlotDev& s, int b0, int ct, int
   // row side: position b0 + (lane & 15) in each row of 16 lanes
   const int rl = lane & 15;
   const int rp = min(b0 + rl, N - 1);
-  const int rxy = ldg(s.xy + rp), rw = ldg(s.w + rp), rt = ldg(s.t32 + rp);
+  const int rxy = first.rxy, rw = first.rw, rt = first.rt;
   int64_t rq = 0;
   int rg = 0;
   if (NB == 1) {
@@ -214,8 +236,13 @@ __device__ __forceinline__ void prune_wave(const SlotDev& s, int b0, int ct, int
     const int B = q0 + lane;
     const int Bc = min(B, wb1 - 1);
     const int c0 = Bc * MLP_BLK, c1 = min(c0 + MLP_BLK - 1, N - 1);
-    const int4 sm = *(const int4*)(s.blk + Bc);
-    const int tp = ldg(s.t32 + max(c0 - 1, 0));  // T[c0 - 1]
+    // block Bc's summary and T[c0 - 1]
+    int4v sm = first.sm;
+    int tp = first.tp;
+    if (q0 > wb0) {
+      sm = *(gptr<const int4v>)(s.blk + Bc);
+      tp = ldg(s.t32 + max(c0 - 1, 0));
+    }
     bool keep;
     const uint32_t D = (uint32_t)box_gap(boxlo, boxhi, sm.x, sm.y, dr);
     if (NB == 0) {
@@ -458,13 +485,15 @@ __global__ __launch_bounds__(kBlock) void k_psweep(const SlotDev* __restrict__ t
   const int item = blockIdx.x;
   const SweepSeg sg = segs_dev ? find_sweep(segs_dev, nsegs, item) : find_sweep_inline(inl, nsegs, item);
   const SlotDev& s = table[sg.slot];
-  if (s.info[MLP_INFO_ACTIVE] == 0) return;
   const int N = s.N, tid = threadIdx.x, wave = wave_id();
-  const int par = 1 - (int)(s.info[MLP_INFO_PARITY0 + NB] & 1);
   const int b = item - sg.blk0;
   const int rb = b / sg.ncols, ct = b % sg.ncols;
   const int w0 = rb * kPWg, rows = rows_of(NB, 0, N);
-  const int64_t pf = ldg(s.info + MLP_INFO_PATH32);
+  PruneFirst first(s, w0 + wave * kPR, ct * (W / MLP_BLK));
+  const int64_t active = ldg(s.info + MLP_INFO_ACTIVE), pf = ldg(s.info + MLP_INFO_PATH32);
+  const int par = 1 - (int)(ldg(s.info + MLP_INFO_PARITY0 + NB) & 1);
+  first.arrive();
+  if (active == 0) return;
   if (b == 0 && tid == 0) s.info[MLP_INFO_PARTIAL] = 1;
   if (ct == 0) reset_other(s, NB, par, w0, min(w0 + kPWg, rows), rb == 0);
   if constexpr (NB != 1) {
@@ -474,7 +503,7 @@ __global__ __launch_bounds__(kBlock) void k_psweep(const SlotDev* __restrict__ t
         eval_row<NB == 0 ? 0 : 2, false>(s, NB, 0, by, tid % kWave, row_buf(s, NB, par) + by);
       return;
     }
-    prune_wave<NB, false>(s, w0 + wave * kPR, ct, W, L.list[wave], nullptr, 0, par);
+    prune_wave<NB, false>(s, w0 + wave * kPR, ct, W, L.list[wave], nullptr, 0, par, first);
   } else {
     PruneDiag* G = reinterpret_cast<PruneDiag*>(pdyn);
     // diagonals D = c - 1 - i of the workgroup's rows i = w0 + 1 .. w0 + 32
@@ -485,8 +514,8 @@ __global__ __launch_bounds__(kBlock) void k_psweep(const SlotDev* __restrict__ t
     for (int q = tid; q < nd; q += kBlock) dg[q] = MLP_KEY_NONE;
     if (tid < 4) G->dgx[tid] = MLP_KEY_NONE;
     __syncthreads();
-    if (pf & MLP_LB32_2OPT) prune_wave<1, false>(s, w0 + wave * kPR, ct, W, L.list[wave], G, dlo, par);
-    else prune_wave<1, true>(s, w0 + wave * kPR, ct, W, L.list[wave], G, dlo, par);
+    if (pf & MLP_LB32_2OPT) prune_wave<1, false>(s, w0 + wave * kPR, ct, W, L.list[wave], G, dlo, par, first);
+    else prune_wave<1, true>(s, w0 + wave * kPR, ct, W, L.list[wave], G, dlo, par, first);
     __syncthreads();
     const int rows2 = (N + 1) >> 1, mid0 = N - 1 - rows2;
     int64_t* out = row_buf(s, 1, par);
