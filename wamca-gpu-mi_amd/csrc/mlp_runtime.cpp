@@ -1732,20 +1732,28 @@ int mlp_get_total(mlp_ctx* ctx, int32_t slot, int64_t* cost, int32_t* i, int32_t
   if (entries) *entries = M;
   const int64_t take = std::min<int64_t>(M, std::max<int64_t>(cap, 0));
   if (take == 0) return MLP_OK;
-  std::vector<int64_t> keys((size_t)take);
+  // the keys land in the caller's cost array and are decoded there, a row at a
+  // time (a vector of their own, cleared first, and a division an entry took
+  // 0.8 of 3.7 ms of a TOTAL pass with 0.9 million entries)
+  std::vector<int64_t> own(cost ? 0 : (size_t)take);
+  int64_t* const keys = cost ? cost : own.data();
   HCK(hipStreamSynchronize(ctx->stream));
-  HCK(hipMemcpy(keys.data(), s.total, 8 * (size_t)take, hipMemcpyDeviceToHost));
-  for (int64_t e = 0; e < take; ++e) {
-    const int64_t k = keys[(size_t)e];
-    int ii = 0, jj = 0;
-    int64_t c = INT64_MAX;
-    if (k != MLP_KEY_NONE) {
-      c = k >> MLP_KEY_SHIFT;
-      move_ij(s.total_nb, 0, s.N, (int)(e / s.total_block), (int)(k & MLP_KEY_MASK), ii, jj);
+  HCK(hipMemcpy(keys, s.total, 8 * (size_t)take, hipMemcpyDeviceToHost));
+  const int nb = s.total_nb, N = s.N;
+  for (int64_t e0 = 0, row = 0; e0 < take; e0 += s.total_block, ++row) {
+    const int64_t e1 = std::min<int64_t>(take, e0 + s.total_block);
+    for (int64_t e = e0; e < e1; ++e) {
+      const int64_t k = keys[e];
+      int ii = 0, jj = 0;
+      int64_t c = INT64_MAX;
+      if (k != MLP_KEY_NONE) {
+        c = k >> MLP_KEY_SHIFT;
+        move_ij(nb, 0, N, (int)row, (int)(k & MLP_KEY_MASK), ii, jj);
+      }
+      if (cost) cost[e] = c;
+      if (i) i[e] = ii;
+      if (j) j[e] = jj;
     }
-    if (cost) cost[e] = c;
-    if (i) i[e] = ii;
-    if (j) j[e] = jj;
   }
   return MLP_OK;
 }
