@@ -2478,17 +2478,17 @@ __device__ __forceinline__ uint64_t move64_of(int64_t key, int nb, int rowmap, i
 }
 
 // Rows of the last evaluation of nb (the buffer info[PARITY0 + nb] names).
-// The slot's fields come with the launch and both buffers' keys are loaded
-// beside the parity: one wait instead of a chain of three (8 tours n = 4001,
-// evaluation and 40 of these: 500 -> 495 us).
-__global__ __launch_bounds__(kBlock) void k_rows_moves64(gptr<const int64_t> info,
-                                                         gptr<const int64_t> rows, int rowcap, int N,
-                                                         int nb, int rowmap, int R,
-                                                         gptr<uint64_t> out) {
-  const int64_t parity = info[MLP_INFO_PARITY0 + nb];
+// The slot's fields are scalar loads and both buffers' keys are loaded beside
+// the parity: two waits instead of a chain of three (8 tours n = 4001,
+// evaluation and 40 of these: 503 -> 500 us).  The table names the slot's
+// arrays at the time of the launch, also in a recorded graph's replay.
+__global__ __launch_bounds__(kBlock) void k_rows_moves64(const SlotDev* table, int id, int nb,
+                                                         int rowmap, int R, gptr<uint64_t> out) {
+  const SlotRegs s = slot_regs(table, id, nb);
+  const int64_t parity = s.info[MLP_INFO_PARITY0 + nb];
   for (int r = blockIdx.x * kBlock + threadIdx.x; r < R; r += gridDim.x * kBlock) {
-    const int64_t a = rows[r], b = rows[rowcap + r];
-    out[r] = move64_of((parity & 1) ? b : a, nb, rowmap, N, r);
+    const int64_t a = s.rows[r], b = s.rows[s.rowcap + r];
+    out[r] = move64_of((parity & 1) ? b : a, nb, rowmap, s.N, r);
   }
 }
 
@@ -4245,11 +4245,10 @@ hipError_t mlp_launch_ads(hipStream_t st, const SlotDev* table, int id, int N, u
   return hipGetLastError();
 }
 
-hipError_t mlp_launch_rows_moves64(hipStream_t st, const SlotDev& d, int nb, int rowmap, int R,
-                                   uint64_t* out) {
+hipError_t mlp_launch_rows_moves64(hipStream_t st, const SlotDev* table, int id, int nb,
+                                   int rowmap, int R, uint64_t* out) {
   const int grid = std::max(1, std::min((R + kBlock - 1) / kBlock, 1024));
-  hipLaunchKernelGGL(k_rows_moves64, dim3(grid), dim3(kBlock), 0, st, (gptr<const int64_t>)d.info,
-                     (gptr<const int64_t>)d.rows[nb], d.rowcap, d.N, nb, rowmap, R,
+  hipLaunchKernelGGL(k_rows_moves64, dim3(grid), dim3(kBlock), 0, st, table, id, nb, rowmap, R,
                      (gptr<uint64_t>)out);
   return hipGetLastError();
 }

@@ -2449,7 +2449,7 @@ int mlp_rows_moves64_device(mlp_ctx* ctx, int32_t slot, int32_t nb, uint64_t* de
   const int R = std::max(0, rows_of(nb, rm, s.N));
   if (R > cap) return fail(ctx, MLP_EINVAL, "%d rows do not fit %lld entries", R, (long long)cap);
   if (rows) *rows = R;
-  if (R > 0) HCK(mlp_launch_rows_moves64(ctx->stream, s.dev, nb, rm, R, dev));
+  if (R > 0) HCK(mlp_launch_rows_moves64(ctx->stream, ctx->d_table, slot, nb, rm, R, dev));
   return MLP_OK;
 }
 
