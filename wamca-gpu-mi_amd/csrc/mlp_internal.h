@@ -154,6 +154,7 @@ struct SweepSegsInline {
 // tiles of its own eval phase), so the queue always drains.
 struct FusedPlan {
   int32_t count, per_round, rounds, tail, pcap, ncap;
+  int32_t keep;               // merges keep the block summaries
   int32_t phase[11];          // first item of each phase within a round; [10] = per_round
   const int32_t* slots;       // [count]
   const int32_t* prefix;      // [5][count + 1]: eval items of nb before slot q

@@ -3908,7 +3908,7 @@ __global__ __launch_bounds__(kBlock) void k_dvnd_fused(const SlotDev* __restrict
       }
       wait_at_least(merged + q, rr * MLP_NB_COUNT + nb, timeout);
       wait_at_least(done + q, rr * all + upto, timeout);
-      merge_slot<kBlock, 8>(slot_regs(table, P.slots[q], nb), nb, 0, P.pcap, P.ncap, 1,
+      merge_slot<kBlock, 8>(slot_regs(table, P.slots[q], nb), nb, 0, P.pcap, P.ncap, P.keep ? 3 : 1,
                         nb == MLP_NB_COUNT - 1 ? P.tail : 0, dyn, MS);
       signal_done(merged + q);
     } else {  // up to P.group tiles of the evaluation of nb for slot q

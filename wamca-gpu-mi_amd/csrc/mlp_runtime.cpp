@@ -1933,9 +1933,11 @@ bool fused_ok(const mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, i
   return true;
 }
 
-// One fused launch of `rounds` DVND rounds over the slots.
+// One fused launch of `rounds` DVND rounds over the slots.  keep: as in
+// enqueue_round (a later call's rounds may be pruned: the form of a round is a
+// setting that can change between two calls on the same run).
 int enqueue_fused(mlp_ctx* ctx, const int32_t* slots, int count, int max_rounds, int rounds,
-                  int pcap, int ncap) {
+                  int pcap, int ncap, bool keep) {
   constexpr int R = MLP_FUSED_R, C = MLP_FUSED_C;
   // MLP_FUSED_G tiles per item: a workgroup takes them with one work-counter
   // atomic, one dependency wait and one completion signal
@@ -1949,6 +1951,7 @@ int enqueue_fused(mlp_ctx* ctx, const int32_t* slots, int count, int max_rounds,
   P.tail = max_rounds + 1;
   P.pcap = pcap;
   P.ncap = ncap;
+  P.keep = keep ? 1 : 0;
   int at = 0;
   for (int nb = 0; nb < MLP_NB_COUNT; ++nb) {
     P.phase[2 * nb] = at;
@@ -2016,7 +2019,7 @@ int enqueue_rounds(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, in
   const bool fused = fused_ok(ctx, slots, count, rowmap, &pcap, &ncap);
   if (!prune_ok(ctx, slots, count, rowmap)) pruned = 0;
   for (int r = 0; r < rounds; ++r) {
-    const int st = fused ? enqueue_fused(ctx, slots, count, max_rounds, 1, pcap, ncap)
+    const int st = fused ? enqueue_fused(ctx, slots, count, max_rounds, 1, pcap, ncap, keep)
                          : enqueue_round(ctx, slots, count, rowmap, max_rounds, r < pruned,
                                          keep || r < pruned);
     if (st) return st;
