@@ -1,0 +1,79 @@
+// Checks of mlp_dvnd's host logic against a runtime of the host (fake_hip.h).
+#include <cstdio>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "fake_hip.h"
+#include "mlp_gpu.h"
+
+namespace {
+
+#define CHECK(c, ...)                              \
+  do {                                             \
+    if (!(c)) {                                    \
+      printf("%s:%d: ", __FILE__, __LINE__);       \
+      printf(__VA_ARGS__);                         \
+      printf("\n");                                \
+      return 1;                                    \
+    }                                              \
+  } while (0)
+
+struct Run {
+  mlp_ctx* ctx = nullptr;
+  std::vector<int32_t> slots;
+  explicit Run(const std::vector<int>& ns) {
+    mlp_ctx_create(0, &ctx);
+    for (int n : ns) {
+      std::vector<int32_t> x(n), y(n);
+      for (int c = 0; c < n; ++c) {
+        x[c] = c;
+        y[c] = 7 * c % 101;
+      }
+      int32_t inst = -1, s = -1;
+      mlp_instance_create(ctx, x.data(), y.data(), n, 1, &inst);
+      mlp_slot_create(ctx, inst, &s);
+      slots.push_back(s);
+    }
+  }
+  ~Run() { mlp_ctx_destroy(ctx); }
+  int dvnd(int rowmap, int max_rounds, std::vector<int32_t>* rounds = nullptr) {
+    std::vector<int32_t> r(slots.size());
+    const int st = mlp_dvnd(ctx, slots.data(), (int)slots.size(), rowmap, max_rounds, r.data());
+    if (rounds) *rounds = r;
+    return st;
+  }
+};
+
+// A call repeated on the same slots replays its chunks' graphs: from its third
+// time on nothing is launched one by one (a chunk is seen, then captured) and
+// no graph is made.
+int graphs() {
+  for (const std::vector<int>& ns : {std::vector<int>{150}, {600}, {600, 150}, {600, 500, 90}})
+    for (int rowmap = 0; rowmap < 2; ++rowmap)
+      for (int max_rounds = 0; max_rounds <= 17; ++max_rounds) {
+        rounds_of_slot = [](int) { return 30; };
+        Run r(ns);
+        for (int call = 0; call < 5; ++call) {
+          counts = Counts();
+          std::vector<int32_t> rounds;
+          CHECK(r.dvnd(rowmap, max_rounds, &rounds) == MLP_OK, "%s", mlp_ctx_error(r.ctx));
+          for (int32_t k : rounds) CHECK(k == (max_rounds ? max_rounds : 30), "%d rounds", k);
+          if (call < 2) continue;
+          CHECK(counts.instantiated == 0 && counts.eager <= counts.fills && counts.replayed > 0,
+                "%d slots, n = %d, row map %d, max_rounds %d, call %d: %d launches one by one, %d graphs made, %d replayed",
+                (int)ns.size(), ns[0], rowmap, max_rounds, call, counts.eager, counts.instantiated,
+                counts.replayed);
+        }
+      }
+  return 0;
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  const int bad = what == "graphs" ? graphs() : 2;
+  if (!bad) printf("%s ok\n", what.c_str());
+  return bad;
+}

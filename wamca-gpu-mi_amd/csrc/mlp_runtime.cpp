@@ -228,9 +228,16 @@ struct mlp_ctx {
   };
   std::vector<std::vector<GraphOp>> user_graph_ops;
   std::vector<GraphOp> capture_ops;
-  // cached DVND chunk graphs, one per slot group of a DVND call
-  hipGraphExec_t graph_exec[MLP_DVND_GROUPS] = {};
-  std::string graph_key[MLP_DVND_GROUPS];
+  // cached DVND chunk graphs of each slot group of a DVND call.  A call with
+  // max_rounds runs whole chunks and then a last one of other rounds, so one
+  // graph a group would be replaced in every call.
+  struct ChunkGraph {
+    std::string key;  // of the chunk seen (exec: captured since), empty: none
+    hipGraphExec_t exec = nullptr;
+    uint64_t used = 0;  // the least recently used one is replaced
+  };
+  ChunkGraph graphs[MLP_DVND_GROUPS][MLP_DVND_GRAPHS];
+  uint64_t graph_clock = 0;
   // DVND slot groups: the largest slots on the context stream, the others
   // on streams of their own, so one group's merges overlap another's sweeps
   int dvnd_groups = 2;
@@ -324,12 +331,13 @@ int device_list(mlp_ctx* ctx, const int32_t* v, int count, const int32_t** out) 
   }
   if (ctx->lists.size() >= 8192 && !ctx->capturing) {
     HCK(sync_streams(ctx));
-    for (int g = 0; g < MLP_DVND_GROUPS; ++g)
-      if (ctx->graph_exec[g]) {  // its launches point into the lists
-        HCK(hipGraphExecDestroy(ctx->graph_exec[g]));
-        ctx->graph_exec[g] = nullptr;
-        ctx->graph_key[g].clear();
-      }
+    for (auto& group : ctx->graphs)
+      for (auto& c : group)
+        if (c.exec) {  // its launches point into the lists
+          HCK(hipGraphExecDestroy(c.exec));
+          c.exec = nullptr;
+          c.key.clear();
+        }
     bool user_graphs = false;
     for (hipGraphExec_t g : ctx->user_graphs) user_graphs = user_graphs || g;
     if (!user_graphs) {  // recorded graphs may point into the lists: keep them
@@ -514,8 +522,9 @@ int mlp_ctx_destroy(mlp_ctx* ctx) {
   for (void* p : ctx->pool_all) hipFree(p);
   for (auto& kv : ctx->lists) hipFree(kv.second.p);
   if (ctx->d_table) hipFree(ctx->d_table);
-  for (hipGraphExec_t g : ctx->graph_exec)
-    if (g) hipGraphExecDestroy(g);
+  for (auto& group : ctx->graphs)
+    for (auto& c : group)
+      if (c.exec) hipGraphExecDestroy(c.exec);
   for (hipGraphExec_t g : ctx->user_graphs)
     if (g) hipGraphExecDestroy(g);
   if (ctx->d_counter) hipFree(ctx->d_counter);
@@ -1039,17 +1048,18 @@ int auto_tile(const mlp_ctx* ctx, const int32_t* slots, int count, uint32_t mask
 constexpr int64_t kPruneWaves = 2048;
 constexpr int kPruneMinN = 256;
 
-// Forget the cached DVND chunk graph (its launches embed the neighborhood
-// set, tile choices and merge mode of the moment it was captured).
+// Forget the cached DVND chunk graphs (their launches embed the neighborhood
+// set, tile choices and merge mode of the moment they were captured).
 int drop_dvnd_graph(mlp_ctx* ctx) {
-  for (int g = 0; g < MLP_DVND_GROUPS; ++g) {
-    if (ctx->graph_exec[g]) {
-      if (!ctx->capturing) HCK(sync_streams(ctx));
-      HCK(hipGraphExecDestroy(ctx->graph_exec[g]));
-      ctx->graph_exec[g] = nullptr;
+  for (auto& group : ctx->graphs)
+    for (auto& c : group) {
+      if (c.exec) {
+        if (!ctx->capturing) HCK(sync_streams(ctx));
+        HCK(hipGraphExecDestroy(c.exec));
+        c.exec = nullptr;
+      }
+      c.key.clear();
     }
-    ctx->graph_key[g].clear();
-  }
   return MLP_OK;
 }
 
@@ -2007,17 +2017,16 @@ int enqueue_fused(mlp_ctx* ctx, const int32_t* slots, int count, int max_rounds,
   return MLP_OK;
 }
 
-// `rounds` DVND rounds over `slots`, as one captured graph when enabled.  A
-// chunk is captured the second time the same (slots, settings) is seen, so
-// every device list it needs already exists (no copies inside a capture).
-// The first `pruned` rounds may leave out rows that do not improve; the block
-// summaries are kept if they are pruned, or if another call on some of the
-// slots may be (keep).
+// `rounds` DVND rounds over `slots`, as one captured graph when enabled
+// (run_chunk).  A chunk is captured the second time the same (slots, settings)
+// is seen, so every device list it needs already exists (no copies inside a
+// capture).  The first `pruned` rounds may leave out rows that do not improve;
+// the block summaries are kept if they are pruned, or if another call on some
+// of the slots may be (keep).
 int enqueue_rounds(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max_rounds,
                    int rounds, int pruned, bool keep) {
   int pcap = 0, ncap = 0;
   const bool fused = fused_ok(ctx, slots, count, rowmap, &pcap, &ncap);
-  if (!prune_ok(ctx, slots, count, rowmap)) pruned = 0;
   for (int r = 0; r < rounds; ++r) {
     const int st = fused ? enqueue_fused(ctx, slots, count, max_rounds, 1, pcap, ncap, keep)
                          : enqueue_round(ctx, slots, count, rowmap, max_rounds, r < pruned,
@@ -2029,7 +2038,9 @@ int enqueue_rounds(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, in
 
 int run_chunk(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max_rounds,
               int rounds, int pruned, bool keep = false, int gc = 0) {
-  pruned = std::max(0, std::min(pruned, rounds));
+  // what the launches are, not what was asked for: calls whose rounds are not
+  // pruned have one key whatever their limit
+  pruned = prune_ok(ctx, slots, count, rowmap) ? std::max(0, std::min(pruned, rounds)) : 0;
   if (!ctx->dvnd_graph || ctx->user_capture)
     return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
   int tile = ctx->tile_override;  // (the per-neighborhood shapes follow from the slots)
@@ -2045,8 +2056,25 @@ int run_chunk(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max
     const int32_t Nn[2] = {ctx->slots[slots[q]].N, ctx->slots[slots[q]].nbs};
     key.append((const char*)Nn, sizeof Nn);
   }
-  if (key == ctx->graph_key[gc] && ctx->graph_exec[gc]) {
-    HCK(hipGraphLaunch(ctx->graph_exec[gc], ctx->stream));
+  mlp_ctx::ChunkGraph* c = &ctx->graphs[gc][0];
+  for (auto& e : ctx->graphs[gc]) {
+    if (e.key == key) {
+      c = &e;
+      break;
+    }
+    if (e.used < c->used) c = &e;
+  }
+  c->used = ++ctx->graph_clock;
+  if (c->key != key) {  // first sight: run eagerly, remember the key
+    if (c->exec) {
+      HCK(hipGraphExecDestroy(c->exec));
+      c->exec = nullptr;
+    }
+    c->key = key;
+    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
+  }
+  if (c->exec) {
+    HCK(hipGraphLaunch(c->exec, ctx->stream));
     // the launches' host bookkeeping (evaluated / merged flags)
     for (int q = 0; q < count; ++q) {
       Slot& s = ctx->slots[slots[q]];
@@ -2058,14 +2086,6 @@ int run_chunk(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max
     }
     return MLP_OK;
   }
-  if (key != ctx->graph_key[gc]) {  // first sight: run eagerly, remember the key
-    if (ctx->graph_exec[gc]) {
-      HCK(hipGraphExecDestroy(ctx->graph_exec[gc]));
-      ctx->graph_exec[gc] = nullptr;
-    }
-    ctx->graph_key[gc] = key;
-    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
-  }
   hipGraph_t g = nullptr;
   HCK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeRelaxed));
   ctx->capturing = true;
@@ -2074,16 +2094,16 @@ int run_chunk(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max
   const hipError_t ec = hipStreamEndCapture(ctx->stream, &g);
   if (st || ec != hipSuccess) {  // nothing captured ran: run the chunk eagerly instead
     if (g) hipGraphDestroy(g);
-    ctx->graph_key[gc].clear();
+    c->key.clear();
     return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
   }
-  const hipError_t ei = hipGraphInstantiate(&ctx->graph_exec[gc], g, nullptr, nullptr, 0);
+  const hipError_t ei = hipGraphInstantiate(&c->exec, g, nullptr, nullptr, 0);
   hipGraphDestroy(g);
   if (ei != hipSuccess) {
-    ctx->graph_exec[gc] = nullptr;
+    c->exec = nullptr;
     return fail(ctx, MLP_EDEVICE, "graph instantiate: %s", hipGetErrorString(ei));
   }
-  HCK(hipGraphLaunch(ctx->graph_exec[gc], ctx->stream));
+  HCK(hipGraphLaunch(c->exec, ctx->stream));
   return MLP_OK;
 }
 
