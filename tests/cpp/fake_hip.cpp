@@ -12,6 +12,8 @@
 Counts counts;
 std::function<int(int)> rounds_of_slot = [](int) { return 1 << 20; };
 int fail_sync = 0;
+static const SlotDev* last_table = nullptr;
+bool left_out(int slot) { return last_table[slot].info[MLP_INFO_PARTIAL] == 1; }
 
 namespace {
 
@@ -122,6 +124,7 @@ hipError_t mlp_launch_slot_init(hipStream_t st, SlotDev* table, int id, const Sl
 }
 hipError_t mlp_launch_dvnd_start(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
                                  const int32_t* dev, int count) {
+  last_table = table;
   submit(st, [=] {
     for (int32_t id : listed(inl.id, dev, count)) {
       table[id].info[MLP_INFO_ACTIVE] = 1;
@@ -133,8 +136,11 @@ hipError_t mlp_launch_dvnd_start(hipStream_t st, const SlotDev* table, const Slo
 hipError_t mlp_launch_sweep(hipStream_t st, int, const SlotDev* table, const SweepSegsInline& inl,
                             const SweepSeg* dev, int nsegs, int, int*, int, int flags) {
   submit_eval(st, flags & 8 ? &Counts::fills : &Counts::evals, [=] {
-    for (const SweepSeg& g : listed(inl.s, dev, nsegs))
-      if (!(flags & 8) && table[g.slot].info[MLP_INFO_ACTIVE]) table[g.slot].info[MLP_INFO_PARTIAL] = 0;
+    for (const SweepSeg& g : listed(inl.s, dev, nsegs)) {
+      int64_t* info = table[g.slot].info;
+      if (flags & 8) info[MLP_INFO_PARTIAL] *= 2;  // (the device's word stays 1: nothing reads it again)
+      else if (info[MLP_INFO_ACTIVE]) info[MLP_INFO_PARTIAL] = 0;
+    }
   });
   return hipSuccess;
 }

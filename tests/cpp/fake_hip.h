@@ -22,5 +22,7 @@ extern Counts counts;
 extern std::function<int(int)> rounds_of_slot;
 // The stream synchronisation with this number (from 1) fails; 0: none.
 extern int fail_sync;
+// Whether the slot's last round left rows out and nothing completed them since.
+bool left_out(int slot);
 
 #endif  // FAKE_HIP_H_

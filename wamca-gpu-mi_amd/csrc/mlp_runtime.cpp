@@ -2369,23 +2369,13 @@ int mlp_dvnd_fused(mlp_ctx* ctx, int32_t on) {
   return drop_dvnd_graph(ctx);
 }
 
-int mlp_dvnd(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
-             int32_t max_rounds, int32_t* rounds_out) {
-  NO_CAPTURE(ctx);
-  int st = check_slots(ctx, slots, count);
-  if (st) return st;
-  if (rowmap != 0 && rowmap != 1) return fail(ctx, MLP_EINVAL, "rowmap must be 0 or 1");
-  if (count == 0) return MLP_OK;
-  st = check_mask(ctx, slots, count, (1u << ctx->dvnd_nbs) - 1u);
-  if (st) return st;
-  st = mlp_dvnd_start(ctx, slots, count);
-  if (st) return st;
+// The rounds of an mlp_dvnd call until every slot has stopped.
+static int dvnd_run(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
+                    int32_t max_rounds) {
+  int st = MLP_OK;
   std::vector<int32_t> active(slots, slots + count), flag((size_t)count);
-  if (count >= 2 && ctx->dvnd_groups > 1 && !ctx->dvnd_fused && !ctx->dvnd_persistent) {
-    st = dvnd_independent(ctx, slots, count, rowmap, max_rounds);
-    if (st) return st;
-    active.clear();
-  }
+  if (count >= 2 && ctx->dvnd_groups > 1 && !ctx->dvnd_fused && !ctx->dvnd_persistent)
+    return dvnd_independent(ctx, slots, count, rowmap, max_rounds);
   int done = 0;
   while (!active.empty()) {
     const int c = (int)active.size();
@@ -2400,10 +2390,31 @@ int mlp_dvnd(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
       if (flag[(size_t)q]) next.push_back(active[(size_t)q]);
     active.swap(next);
   }
-  // (a round is pruned for its active slots only if it is for all of them)
-  if (prunable(max_rounds, 0) > 0 && prune_ok(ctx, slots, count, rowmap))
-    st = complete_rows(ctx, slots, count, rowmap);
+  return MLP_OK;
+}
+
+int mlp_dvnd(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
+             int32_t max_rounds, int32_t* rounds_out) {
+  NO_CAPTURE(ctx);
+  int st = check_slots(ctx, slots, count);
   if (st) return st;
+  if (rowmap != 0 && rowmap != 1) return fail(ctx, MLP_EINVAL, "rowmap must be 0 or 1");
+  if (count == 0) return MLP_OK;
+  st = check_mask(ctx, slots, count, (1u << ctx->dvnd_nbs) - 1u);
+  if (st) return st;
+  st = mlp_dvnd_start(ctx, slots, count);
+  if (st) return st;
+  // (a round is pruned for its active slots only if it is for all of them)
+  const bool pruned = prunable(max_rounds, 0) > 0 && prune_ok(ctx, slots, count, rowmap);
+  st = dvnd_run(ctx, slots, count, rowmap, max_rounds);
+  if (!st && pruned) st = complete_rows(ctx, slots, count, rowmap);
+  if (st) {
+    // rows that a pruned round left out are still missing: none can be read
+    // until the next evaluation
+    for (int q = 0; q < count && pruned; ++q)
+      for (int nb = 0; nb < MLP_NB_COUNT; ++nb) ctx->slots[slots[q]].eval_rowmap[nb] = -1;
+    return st;
+  }
   if (rounds_out) return mlp_dvnd_status(ctx, slots, count, nullptr, rounds_out);
   return MLP_OK;
 }
