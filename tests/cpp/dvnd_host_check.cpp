@@ -100,11 +100,40 @@ int failed_rows() {
   return 0;
 }
 
+// A slot evaluates each neighborhood once a round, and once more after its last
+// one if rows were left out there; a slot that stops in its first round (a tour
+// at its optimum) does not.
+int evaluations() {
+  for (const std::vector<int>& ns : {std::vector<int>{150}, {600}, {600, 150}, {600, 500, 90}})
+    for (int rowmap = 0; rowmap < 2; ++rowmap)
+      for (int max_rounds : {0, 1, 2, 3, 4, 5, 9})
+        for (int large = 1; large < 8; ++large)
+          for (int small = 1; small < 8; small += 3) {
+            rounds_of_slot = [=](int N) { return N > 400 ? large : small; };
+            Run r(ns);
+            for (int call = 0; call < 3; ++call) {
+              counts = Counts();
+              std::vector<int32_t> rounds;
+              CHECK(r.dvnd(rowmap, max_rounds, &rounds) == MLP_OK, "%s", mlp_ctx_error(r.ctx));
+              int least = 0, most = 0;
+              for (int32_t k : rounds) {
+                least += 5 * k;
+                most += 5 * (k > 1 && k != max_rounds ? k + 1 : k);
+              }
+              CHECK(counts.worked >= least && counts.worked <= most,
+                    "%d slots, n = %d, row map %d, max_rounds %d, %d and %d rounds: %d evaluations, expected %d to %d",
+                    (int)ns.size(), ns[0], rowmap, max_rounds, large, small, counts.worked, least, most);
+            }
+          }
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
-  const int bad = what == "graphs" ? graphs() : what == "failed_rows" ? failed_rows() : 2;
+  const int bad = what == "graphs" ? graphs() : what == "failed_rows" ? failed_rows()
+                  : what == "evaluations" ? evaluations() : 2;
   if (!bad) printf("%s ok\n", what.c_str());
   return bad;
 }

@@ -138,6 +138,7 @@ hipError_t mlp_launch_sweep(hipStream_t st, int, const SlotDev* table, const Swe
   submit_eval(st, flags & 8 ? &Counts::fills : &Counts::evals, [=] {
     for (const SweepSeg& g : listed(inl.s, dev, nsegs)) {
       int64_t* info = table[g.slot].info;
+      if (flags & 8 ? info[MLP_INFO_PARTIAL] : info[MLP_INFO_ACTIVE]) counts.worked += __builtin_popcount(g.mask);
       if (flags & 8) info[MLP_INFO_PARTIAL] *= 2;  // (the device's word stays 1: nothing reads it again)
       else if (info[MLP_INFO_ACTIVE]) info[MLP_INFO_PARTIAL] = 0;
     }
@@ -148,7 +149,10 @@ hipError_t mlp_launch_psweep(hipStream_t st, const SlotDev* table, const SweepSe
                              const SweepSeg* dev, int nsegs, int, int, int) {
   submit_eval(st, &Counts::pruned, [=] {
     for (const SweepSeg& g : listed(inl.s, dev, nsegs))
-      if (table[g.slot].info[MLP_INFO_ACTIVE]) table[g.slot].info[MLP_INFO_PARTIAL] = 1;
+      if (table[g.slot].info[MLP_INFO_ACTIVE]) {
+        table[g.slot].info[MLP_INFO_PARTIAL] = 1;
+        ++counts.worked;
+      }
   });
   return hipSuccess;
 }

@@ -16,6 +16,7 @@ struct Counts {
   int eager = 0;         // of these, launched outside a graph
   int instantiated = 0;  // graphs
   int replayed = 0;
+  int worked = 0;        // evaluations of a neighborhood of a slot that did not return at once
 };
 extern Counts counts;
 // rounds after which a slot of N positions finds nothing more

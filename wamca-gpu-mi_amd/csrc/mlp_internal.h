@@ -171,8 +171,9 @@ struct FusedPlan {
 // Streams (slot groups) a DVND call may use (64 instances, n in [50, 2000]:
 // 42.3 ms with one, 37.7 with two, 51.6 with three, 48.6 with four).
 #define MLP_DVND_GROUPS 2
-// Cached chunk graphs of a group: a limited call's whole chunks and its last.
-#define MLP_DVND_GRAPHS 2
+// Cached chunk graphs of a group: a limited call's first chunk, whole chunks
+// and last one.
+#define MLP_DVND_GRAPHS 3
 
 #ifndef MLP_FUSED_G
 #define MLP_FUSED_G 8

@@ -2017,38 +2017,44 @@ int enqueue_fused(mlp_ctx* ctx, const int32_t* slots, int count, int max_rounds,
   return MLP_OK;
 }
 
-// `rounds` DVND rounds over `slots`, as one captured graph when enabled
+// The rounds of a chunk: rounds [from, to) may leave out rows that do not
+// improve; the merges of the first `keep` rounds keep the block summaries (a
+// pruned round can follow them, in this chunk or later).
+struct ChunkPlan {
+  int rounds, from, to, keep;
+};
+
+// A chunk of DVND rounds over `slots`, as one captured graph when enabled
 // (run_chunk).  A chunk is captured the second time the same (slots, settings)
 // is seen, so every device list it needs already exists (no copies inside a
-// capture).  The first `pruned` rounds may leave out rows that do not improve;
-// the block summaries are kept if they are pruned, or if another call on some
-// of the slots may be (keep).
+// capture).
 int enqueue_rounds(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max_rounds,
-                   int rounds, int pruned, bool keep) {
+                   const ChunkPlan& plan) {
   int pcap = 0, ncap = 0;
   const bool fused = fused_ok(ctx, slots, count, rowmap, &pcap, &ncap);
-  for (int r = 0; r < rounds; ++r) {
+  for (int r = 0; r < plan.rounds; ++r) {
+    const bool keep = r < plan.keep;
     const int st = fused ? enqueue_fused(ctx, slots, count, max_rounds, 1, pcap, ncap, keep)
-                         : enqueue_round(ctx, slots, count, rowmap, max_rounds, r < pruned,
-                                         keep || r < pruned);
+                         : enqueue_round(ctx, slots, count, rowmap, max_rounds,
+                                         r >= plan.from && r < plan.to, keep);
     if (st) return st;
   }
   return MLP_OK;
 }
 
 int run_chunk(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max_rounds,
-              int rounds, int pruned, bool keep = false, int gc = 0) {
-  // what the launches are, not what was asked for: calls whose rounds are not
-  // pruned have one key whatever their limit
-  pruned = prune_ok(ctx, slots, count, rowmap) ? std::max(0, std::min(pruned, rounds)) : 0;
+              ChunkPlan plan, int gc = 0) {
+  // what the launches are, not what was asked for: chunks without pruned
+  // rounds have one key
+  if (!prune_ok(ctx, slots, count, rowmap) || plan.from >= plan.to) plan.from = plan.to = 0;
   if (!ctx->dvnd_graph || ctx->user_capture)
-    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
+    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, plan);
   int tile = ctx->tile_override;  // (the per-neighborhood shapes follow from the slots)
   // the captured launches embed the slot table address, every slot's id and
   // size (segment tables, merge capacities) and the settings
-  const int32_t hdr[11] = {rowmap, max_rounds, rounds, ctx->dvnd_persistent, tile, count,
+  const int32_t hdr[12] = {rowmap, max_rounds, plan.rounds, ctx->dvnd_persistent, tile, count,
                            ctx->dvnd_nbs, ctx->merge_force_global ? 1 : 0, ctx->dvnd_fused,
-                           pruned, keep ? 1 : 0};
+                           plan.from, plan.to, plan.keep};
   std::string key((const char*)hdr, sizeof hdr);
   key.append((const char*)&ctx->d_table, sizeof ctx->d_table);
   key.append((const char*)slots, 4 * (size_t)count);
@@ -2071,7 +2077,7 @@ int run_chunk(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max
       c->exec = nullptr;
     }
     c->key = key;
-    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
+    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, plan);
   }
   if (c->exec) {
     HCK(hipGraphLaunch(c->exec, ctx->stream));
@@ -2089,13 +2095,13 @@ int run_chunk(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max
   hipGraph_t g = nullptr;
   HCK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeRelaxed));
   ctx->capturing = true;
-  int st = enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
+  int st = enqueue_rounds(ctx, slots, count, rowmap, max_rounds, plan);
   ctx->capturing = false;
   const hipError_t ec = hipStreamEndCapture(ctx->stream, &g);
   if (st || ec != hipSuccess) {  // nothing captured ran: run the chunk eagerly instead
     if (g) hipGraphDestroy(g);
     c->key.clear();
-    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
+    return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, plan);
   }
   const hipError_t ei = hipGraphInstantiate(&c->exec, g, nullptr, nullptr, 0);
   hipGraphDestroy(g);
@@ -2164,16 +2170,16 @@ int group_streams(mlp_ctx* ctx, int groups) {
   return MLP_OK;
 }
 
-// `rounds` DVND rounds over the slots, split into groups on streams of
+// A chunk of DVND rounds over the slots, split into groups on streams of
 // their own when enabled (the fused and persistent forms share device
 // counters across slots, so they keep one stream; so does a caller's
 // capture).  Work queued after the call on the context stream follows every
 // group.
 int run_grouped(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max_rounds,
-                int rounds, int pruned, bool keep = false) {
+                const ChunkPlan& plan) {
   const int groups = std::min(ctx->dvnd_groups, count);
   if (groups < 2 || ctx->dvnd_fused || ctx->dvnd_persistent || ctx->user_capture)
-    return run_chunk(ctx, slots, count, rowmap, max_rounds, rounds, pruned, keep);
+    return run_chunk(ctx, slots, count, rowmap, max_rounds, plan);
   int st = group_streams(ctx, groups);
   if (st) return st;
   std::vector<int32_t> active(slots, slots + count), part[MLP_DVND_GROUPS];
@@ -2184,7 +2190,7 @@ int run_grouped(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int m
   for (int g = 1; g < groups; ++g) HCK(hipStreamWaitEvent(ctx->stream_grp[g], ctx->ev_fork, 0));
   for (int g = 0; g < groups && !st; ++g) {
     ctx->stream = g ? ctx->stream_grp[g] : ctx->stream_main;
-    st = run_chunk(ctx, part[g].data(), (int)part[g].size(), rowmap, max_rounds, rounds, pruned, keep, g);
+    st = run_chunk(ctx, part[g].data(), (int)part[g].size(), rowmap, max_rounds, plan, g);
   }
   ctx->stream = ctx->stream_main;
   // joined also after a failed enqueue, so later work still follows it
@@ -2195,19 +2201,25 @@ int run_grouped(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int m
   return st;
 }
 
-// Rounds of an mlp_dvnd call's next chunk after `done` ones: none beyond
+// An mlp_dvnd call's next chunk after `done` rounds.  No rounds beyond
 // max_rounds, which would be launches over slots that have all stopped (256
-// tours n = 784, one round: 30 of 40 launches, 1.82 ms against 1.62).
-int chunk_rounds(const mlp_ctx* ctx, int max_rounds, int done) {
-  return max_rounds > 0 ? std::max(1, std::min(ctx->dvnd_chunk, max_rounds - done)) : ctx->dvnd_chunk;
-}
-
-// Rounds after `done` ones of an mlp_dvnd call that may leave out rows that
-// do not improve: all but the one that max_rounds makes the last, whose rows
-// the caller can read (those of a round that applied nothing are completed
-// after it, complete_rows).
-int prunable(int max_rounds, int done) {
-  return max_rounds > 0 ? max_rounds - 1 - done : INT_MAX;
+// tours n = 784, one round: 30 of 40 launches, 1.82 ms against 1.62).  Rounds
+// may leave out rows that do not improve, except the one that max_rounds makes
+// the last, whose rows the caller can read, and the call's first: a tour that
+// is at its optimum already would be evaluated twice, the rows that the round
+// left out once more after it (complete_rows; n = 2047 at its optimum 209 us,
+// 190 with every move evaluated once; longer solves lose nothing, few blocks
+// of a random or constructed tour can be left out).
+ChunkPlan next_chunk(const mlp_ctx* ctx, const int32_t* slots, int count, int rowmap,
+                     int max_rounds, int done) {
+  ChunkPlan p{ctx->dvnd_chunk, 0, 0, 0};
+  const int last = max_rounds > 0 ? max_rounds - 1 : INT_MAX;
+  if (max_rounds > 0) p.rounds = std::max(1, std::min(ctx->dvnd_chunk, max_rounds - done));
+  if (!prune_ok(ctx, slots, count, rowmap)) return p;
+  auto within = [&](int r) { return std::max(0, std::min(r, p.rounds)); };
+  p.from = within(1 - done);
+  p.to = p.keep = within(last - done);
+  return p;
 }
 
 // The rows of slots whose DVND run ended in a pruned round, completed in
@@ -2227,11 +2239,11 @@ int complete_rows(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap) {
 // groups are fixed for the call; the context stream waits for every group
 // at the end.
 int dvnd_independent(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap,
-                     int max_rounds) {
+                     int max_rounds, std::vector<int32_t>& ran) {
   const int groups = std::min(ctx->dvnd_groups, count);
   int st = group_streams(ctx, groups);
   if (st) return st;
-  std::vector<int32_t> active(slots, slots + count), part[MLP_DVND_GROUPS], flag;
+  std::vector<int32_t> active(slots, slots + count), part[MLP_DVND_GROUPS], flag, r;
   st = split_groups(ctx, active, groups, part);
   if (st) return st;
   HCK(hipEventRecord(ctx->ev_fork, ctx->stream_main));
@@ -2242,10 +2254,10 @@ int dvnd_independent(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap,
     for (int g = 0; g < groups && !st; ++g)
       if (!pending[g] && !part[g].empty()) {
         ctx->stream = g ? ctx->stream_grp[g] : ctx->stream_main;
-        const int rounds = chunk_rounds(ctx, max_rounds, done[g]);
-        st = run_chunk(ctx, part[g].data(), (int)part[g].size(), rowmap, max_rounds, rounds,
-                       prunable(max_rounds, done[g]), false, g);
-        done[g] += rounds;
+        const int c = (int)part[g].size();
+        const ChunkPlan plan = next_chunk(ctx, part[g].data(), c, rowmap, max_rounds, done[g]);
+        st = run_chunk(ctx, part[g].data(), c, rowmap, max_rounds, plan, g);
+        done[g] += plan.rounds;
         if (!st && hipEventRecord(ctx->ev_chunk[g], ctx->stream) != hipSuccess)
           st = fail(ctx, MLP_EDEVICE, "DVND chunk event");
         pending[g] = !st;
@@ -2270,7 +2282,9 @@ int dvnd_independent(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap,
     pending[g] = false;
     ctx->stream = g ? ctx->stream_grp[g] : ctx->stream_main;
     flag.resize(part[g].size());
-    st = mlp_dvnd_status(ctx, part[g].data(), (int)part[g].size(), flag.data(), nullptr);
+    r.resize(part[g].size());
+    st = mlp_dvnd_status(ctx, part[g].data(), (int)part[g].size(), flag.data(), r.data());
+    for (size_t q = 0; q < part[g].size() && !st; ++q) ran[(size_t)part[g][q]] = r[q];
     std::vector<int32_t> next;
     for (size_t q = 0; q < part[g].size() && !st; ++q)
       if (flag[q]) next.push_back(part[g][q]);
@@ -2318,7 +2332,8 @@ static int dvnd_rounds_impl(mlp_ctx* ctx, const int32_t* slots, int32_t count, i
   if (rowmap != 0 && rowmap != 1) return fail(ctx, MLP_EINVAL, "rowmap must be 0 or 1");
   if (rounds < 0) return fail(ctx, MLP_EINVAL, "rounds must be >= 0");
   if (count == 0 || rounds == 0) return MLP_OK;
-  return run_grouped(ctx, slots, count, rowmap, max_rounds, rounds, improving ? INT_MAX : 0, improving);
+  const int all = improving ? rounds : 0;
+  return run_grouped(ctx, slots, count, rowmap, max_rounds, ChunkPlan{rounds, 0, all, all});
 }
 
 int mlp_dvnd_rounds(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
@@ -2369,22 +2384,24 @@ int mlp_dvnd_fused(mlp_ctx* ctx, int32_t on) {
   return drop_dvnd_graph(ctx);
 }
 
-// The rounds of an mlp_dvnd call until every slot has stopped.
+// The rounds of an mlp_dvnd call until every slot has stopped; ran: by slot,
+// the rounds it ran.
 static int dvnd_run(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
-                    int32_t max_rounds) {
+                    int32_t max_rounds, std::vector<int32_t>& ran) {
   int st = MLP_OK;
-  std::vector<int32_t> active(slots, slots + count), flag((size_t)count);
+  std::vector<int32_t> active(slots, slots + count), flag((size_t)count), r((size_t)count);
   if (count >= 2 && ctx->dvnd_groups > 1 && !ctx->dvnd_fused && !ctx->dvnd_persistent)
-    return dvnd_independent(ctx, slots, count, rowmap, max_rounds);
+    return dvnd_independent(ctx, slots, count, rowmap, max_rounds, ran);
   int done = 0;
   while (!active.empty()) {
     const int c = (int)active.size();
-    const int rounds = chunk_rounds(ctx, max_rounds, done);
-    st = run_grouped(ctx, active.data(), c, rowmap, max_rounds, rounds, prunable(max_rounds, done));
-    done += rounds;
+    const ChunkPlan plan = next_chunk(ctx, active.data(), c, rowmap, max_rounds, done);
+    st = run_grouped(ctx, active.data(), c, rowmap, max_rounds, plan);
+    done += plan.rounds;
     if (st) return st;
-    st = mlp_dvnd_status(ctx, active.data(), c, flag.data(), nullptr);
+    st = mlp_dvnd_status(ctx, active.data(), c, flag.data(), r.data());
     if (st) return st;
+    for (int q = 0; q < c; ++q) ran[(size_t)active[(size_t)q]] = r[(size_t)q];
     std::vector<int32_t> next;
     for (int q = 0; q < c; ++q)
       if (flag[(size_t)q]) next.push_back(active[(size_t)q]);
@@ -2404,10 +2421,19 @@ int mlp_dvnd(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
   if (st) return st;
   st = mlp_dvnd_start(ctx, slots, count);
   if (st) return st;
-  // (a round is pruned for its active slots only if it is for all of them)
-  const bool pruned = prunable(max_rounds, 0) > 0 && prune_ok(ctx, slots, count, rowmap);
-  st = dvnd_run(ctx, slots, count, rowmap, max_rounds);
-  if (!st && pruned) st = complete_rows(ctx, slots, count, rowmap);
+  // whether rounds after the first may be pruned (a round is for its active
+  // slots only if it is for all of them)
+  const bool pruned = (max_rounds <= 0 || max_rounds > 2) && prune_ok(ctx, slots, count, rowmap);
+  std::vector<int32_t> ran(ctx->slots.size());
+  st = dvnd_run(ctx, slots, count, rowmap, max_rounds, ran);
+  bool incomplete = false;
+  for (int q = 0; q < count; ++q) incomplete = incomplete || (pruned && ran[(size_t)slots[q]] > 1);
+  if (!st && incomplete) {
+    st = complete_rows(ctx, slots, count, rowmap);
+    // the slots' rounds are known, only the rows are waited for
+    if (!st && rounds_out && hipStreamSynchronize(ctx->stream) != hipSuccess)
+      st = fail(ctx, MLP_EDEVICE, "DVND rows: %s", hipGetErrorString(hipGetLastError()));
+  }
   if (st) {
     // rows that a pruned round left out are still missing: none can be read
     // until the next evaluation
@@ -2415,7 +2441,7 @@ int mlp_dvnd(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t rowmap,
       for (int nb = 0; nb < MLP_NB_COUNT; ++nb) ctx->slots[slots[q]].eval_rowmap[nb] = -1;
     return st;
   }
-  if (rounds_out) return mlp_dvnd_status(ctx, slots, count, nullptr, rounds_out);
+  for (int q = 0; q < count && rounds_out; ++q) rounds_out[q] = ran[(size_t)slots[q]];
   return MLP_OK;
 }
 
