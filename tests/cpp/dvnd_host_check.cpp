@@ -128,12 +128,34 @@ int evaluations() {
   return 0;
 }
 
+// Between mlp_timing_begin and mlp_timing_end every evaluation of a round
+// launched outside a graph is timed, also of rounds that leave rows out, and no
+// other: a ring of that many launches is enough.
+int timed() {
+  for (const std::vector<int>& ns : {std::vector<int>{150}, {600}, {600, 150}})
+    for (int rowmap = 0; rowmap < 2; ++rowmap) {
+      rounds_of_slot = [](int) { return 6; };
+      Run r(ns);
+      mlp_dvnd_config(r.ctx, 4, 0, 0);
+      counts = Counts();
+      CHECK(mlp_timing_begin(r.ctx, (int)ns.size() * 40) == MLP_OK && r.dvnd(rowmap, 0) == MLP_OK, "%s", mlp_ctx_error(r.ctx));
+      double ms = 0;
+      int32_t launches = 0;
+      CHECK(mlp_timing_end(r.ctx, &ms, &launches) == MLP_OK, "%s", mlp_ctx_error(r.ctx));
+      const int ran = counts.evals + counts.pruned;
+      CHECK(launches == ran, "%d slots, n = %d, row map %d: %d of %d launches timed", (int)ns.size(), ns[0], rowmap,
+            launches, ran);
+    }
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   const int bad = what == "graphs" ? graphs() : what == "failed_rows" ? failed_rows()
-                  : what == "evaluations" ? evaluations() : 2;
+                  : what == "evaluations" ? evaluations()
+                  : what == "timed" ? timed() : 2;
   if (!bad) printf("%s ok\n", what.c_str());
   return bad;
 }

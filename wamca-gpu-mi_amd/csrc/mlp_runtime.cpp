@@ -990,6 +990,7 @@ struct EvalArgs {
   const SweepSeg* sdev;
   int nsegs, total, rowmap, grid, skip;
   int* counter;
+  int nb, W;  // pruned evaluations
 };
 
 hipError_t launch_eval_cb(mlp_ctx* ctx, void* p) {
@@ -1073,6 +1074,11 @@ hipError_t launch_sweep_cb(mlp_ctx* ctx, void* p) {
   EvalArgs& a = *(EvalArgs*)p;
   return mlp_launch_sweep(ctx->stream, a.rowmap, ctx->d_table, a.sinl, a.sdev, a.nsegs, a.total,
                           a.counter, a.grid, a.skip);
+}
+
+hipError_t launch_psweep_cb(mlp_ctx* ctx, void* p) {
+  EvalArgs& a = *(EvalArgs*)p;
+  return mlp_launch_psweep(ctx->stream, ctx->d_table, a.sinl, a.sdev, a.nsegs, a.total, a.nb, a.W);
 }
 
 }  // namespace
@@ -1873,17 +1879,19 @@ int prune_impl(mlp_ctx* ctx, const int32_t* slots, int count, int nb) {
     if (rows > 0) total += (rows + R - 1) / R * ncols;
   }
   if (total == 0) return MLP_OK;
-  SweepSegsInline inl{};
-  const SweepSeg* dev = nullptr;
+  EvalArgs a{};
+  a.nsegs = count;
+  a.total = total;
+  a.nb = nb;
+  a.W = W;
   if (count <= MLP_SEGS_INLINE) {
-    for (int q = 0; q < count; ++q) inl.s[q] = segs[(size_t)q];
+    for (int q = 0; q < count; ++q) a.sinl.s[q] = segs[(size_t)q];
   } else {
     const int st = device_list(ctx, (const int32_t*)segs.data(), count * MLP_SWEEPSEG_INTS,
-                               (const int32_t**)&dev);
+                               (const int32_t**)&a.sdev);
     if (st) return st;
   }
-  HCK(mlp_launch_psweep(ctx->stream, ctx->d_table, inl, dev, count, total, nb, W));
-  return MLP_OK;
+  return timed_launch(ctx, launch_psweep_cb, &a);
 }
 
 // One DVND round over `slots`: round begin, {eval, merge + apply} for each
@@ -2224,9 +2232,13 @@ ChunkPlan next_chunk(const mlp_ctx* ctx, const int32_t* slots, int count, int ro
 
 // The rows of slots whose DVND run ended in a pruned round, completed in
 // place: that round applied no move, so the tour is the one they belong to.
+// Not one of the timed launches, which are those of the rounds.
 int complete_rows(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap) {
   const int nbs = std::min(ctx->dvnd_nbs, MLP_NB_COUNT);
+  const bool timing = ctx->timing;
+  ctx->timing = false;
   const int st = eval_impl(ctx, slots, count, (1u << nbs) - 1u, rowmap, 0, 1 | 8, nullptr);
+  ctx->timing = timing;
   for (int q = 0; q < count; ++q)
     for (int nb = 0; nb < nbs; ++nb) ctx->slots[slots[q]].merged[nb] = true;
   return st;
