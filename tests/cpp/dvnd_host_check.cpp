@@ -149,13 +149,29 @@ int timed() {
   return 0;
 }
 
+// A fused round's launch has no more workgroups than its dynamic and static LDS
+// leave room for at once.
+int fused_grid() {
+  for (int n = 100; n < 5000; n += 50) {
+    rounds_of_slot = [](int) { return 2; };
+    Run r({n, n - 20});
+    mlp_dvnd_fused(r.ctx, 1);
+    counts = Counts();
+    CHECK(r.dvnd(0, 0) == MLP_OK, "%s", mlp_ctx_error(r.ctx));
+    const int fit = 256 * (int)(160 * 1024 / counts.fused_lds);
+    CHECK(counts.fused_grid > 0 && counts.fused_grid <= fit, "n = %d: %d workgroups, %d fit", n, counts.fused_grid, fit);
+  }
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   const int bad = what == "graphs" ? graphs() : what == "failed_rows" ? failed_rows()
                   : what == "evaluations" ? evaluations()
-                  : what == "timed" ? timed() : 2;
+                  : what == "timed" ? timed()
+                  : what == "fused_grid" ? fused_grid() : 2;
   if (!bad) printf("%s ok\n", what.c_str());
   return bad;
 }

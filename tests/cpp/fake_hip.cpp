@@ -192,6 +192,15 @@ size_t mlp_merge_lds_bytes(int pcap, int ncap) { return 10 * (size_t)pcap + 13 *
 size_t mlp_fused_lds_bytes(int pcap, int ncap) { return mlp_merge_lds_bytes(pcap, ncap); }
 size_t mlp_total_merge_lds_bytes(int N) { return 9 * (size_t)N; }
 size_t mlp_total_static_lds() { return 48 * 1024; }
+size_t mlp_fused_static_lds() { return 6500; }
+hipError_t mlp_launch_fused(hipStream_t st, const SlotDev* table, const FusedPlan& plan, int grid) {
+  counts.fused_grid = grid;
+  counts.fused_lds = mlp_fused_lds_bytes(plan.pcap, plan.ncap) + mlp_fused_static_lds();
+  const std::vector<int32_t> ids(plan.slots, plan.slots + plan.count);
+  const int tail = plan.tail;
+  submit(st, [=] { merge(table, ids, tail); });
+  return hipSuccess;
+}
 hipError_t mlp_merge_setup(size_t) { return hipSuccess; }
 hipError_t mlp_fused_setup(size_t) { return hipSuccess; }
 hipError_t mlp_total_setup(size_t) { return hipSuccess; }
@@ -205,7 +214,6 @@ NOTHING(mlp_launch_round_begin, hipStream_t, const SlotDev*, const SlotListInlin
 NOTHING(mlp_launch_round_end, hipStream_t, const SlotDev*, const SlotListInline&, const int32_t*, int, int)
 NOTHING(mlp_launch_eval, hipStream_t, const SlotDev*, const EvalSegsInline&, const EvalSeg*, int, int, int, int*,
         int, int)
-NOTHING(mlp_launch_fused, hipStream_t, const SlotDev*, const FusedPlan&, int)
 NOTHING(mlp_launch_total_eval, hipStream_t, const SlotDev*, int, int, int, int, int64_t*)
 NOTHING(mlp_launch_total_keys, hipStream_t, const int64_t*, int64_t, int, uint64_t, uint64_t*, int32_t*)
 NOTHING(mlp_launch_total_merge, hipStream_t, const SlotDev*, int, int, int, int, int64_t, uint64_t, const uint64_t*,

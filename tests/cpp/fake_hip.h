@@ -6,6 +6,7 @@
 #ifndef FAKE_HIP_H_
 #define FAKE_HIP_H_
 
+#include <cstddef>
 #include <functional>
 #include <vector>
 
@@ -16,6 +17,8 @@ struct Counts {
   int eager = 0;         // of these, launched outside a graph
   int instantiated = 0;  // graphs
   int replayed = 0;
+  int fused_grid = 0;    // workgroups of the last launch of a fused round, LDS of each
+  size_t fused_lds = 0;
   int worked = 0;        // evaluations of a neighborhood of a slot that did not return at once
 };
 extern Counts counts;

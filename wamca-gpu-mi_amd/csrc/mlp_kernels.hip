@@ -4149,6 +4149,9 @@ size_t mlp_fused_lds_bytes(int pcap, int ncap) {
   return std::max(sizeof(SweepLds<MLP_FUSED_R, MLP_FUSED_C, kPlain>), mlp_merge_lds_bytes(pcap, ncap));
 }
 
+// its shared variables and item number
+size_t mlp_fused_static_lds() { return sizeof(MergeShared<kBlock>) + sizeof(int64_t); }
+
 hipError_t mlp_fused_setup(size_t max_dyn_lds) {
   hipError_t e = hipFuncSetAttribute((const void*)k_dvnd_fused<MLP_FUSED_R, MLP_FUSED_C>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_dyn_lds);

@@ -51,8 +51,10 @@ hipError_t mlp_launch_merge_apply(hipStream_t st, const SlotDev* table, const Sl
 hipError_t mlp_launch_merge_gmem(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
                                  const int32_t* list_dev, int count, int nb, int rowmap,
                                  int skip_inactive, int tail, int max_n);
-// Fused DVND rounds (FusedPlan): dynamic LDS of a launch, its limit, the launch.
+// Fused DVND rounds (FusedPlan): dynamic and static LDS of a launch, the limit
+// of the former, the launch.
 size_t mlp_fused_lds_bytes(int pcap, int ncap);
+size_t mlp_fused_static_lds();
 hipError_t mlp_fused_setup(size_t max_dyn_lds);
 hipError_t mlp_launch_fused(hipStream_t st, const SlotDev* table, const FusedPlan& plan, int grid);
 // TOTAL mode: entries rows * B of nb, their sort keys, the merge + apply.

@@ -2010,7 +2010,7 @@ int enqueue_fused(mlp_ctx* ctx, const int32_t* slots, int count, int max_rounds,
     ctx->sync_cap = cap;
   }
   P.sync = ctx->d_sync;
-  const size_t lds = mlp_fused_lds_bytes(pcap, ncap) + 4096;
+  const size_t lds = mlp_fused_lds_bytes(pcap, ncap) + mlp_fused_static_lds();
   const int per_cu = std::max(1, std::min(4, (int)((160 * 1024) / lds)));
   const int grid = std::max(1, std::min(P.per_round * rounds, ctx->cu_count * per_cu));
   HCK(mlp_launch_fused(ctx->stream, ctx->d_table, P, grid));
