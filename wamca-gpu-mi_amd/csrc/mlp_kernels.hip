@@ -1358,19 +1358,30 @@ template <int TB>
 struct MergeShared {
   int m, kept, lng;
   int cnt, top, cut, left;  // selection
-  int longq[kLongMoves];
   int best[2][3][TB / kWave];  // select_spans: each wave's best cost, its row and move
-  int hist[kSelClasses];    // candidates per class; ranks
-  int64_t list[kSelCap];
   PrepWaves<TB> PL;
+  // rank_sort: ranks (with several threads a key) from 0, carried values from
+  static constexpr int kCarry = TB > kSelCap ? kSelCap : 0;
+  union {  // the sorts and the selection end before the first long move is queued
+    struct {
+      int64_t list[kSelCap];
+      int hist[kCarry + kSelCap];  // candidates per class; ranks and carried values
+    };
+    int longq[kLongMoves];
+  };
 };
 static_assert(sizeof(MergeShared<1024>) <= 8192, "static LDS left beside the merge's dynamic part");
+static_assert(kSelClasses <= MergeShared<512>::kCarry + kSelCap, "the classes' counts fit");
+// A fused round's workgroups hold a merge's dynamic LDS beside these: at 6.3 KB
+// one workgroup fitted a CU where two had (n = 3000, eight rounds: 6.01 ms ->
+// 6.28, 5.71 now).
+static_assert(sizeof(MergeShared<kBlock>) + sizeof(int64_t) <= 4096, "workgroups of a fused round on a CU");
 
 // Sort of list[0..n), n <= 256, distinct keys: a key's rank is the number of
 // smaller keys, counted by TB / 256 threads a key, eight LDS broadcasts in
 // flight (against the 36 barrier phases of a bitonic sort of 256; one at a
 // time they had taken 6400 cycles for 145 keys).  list is padded to 256.
-// carry(e): a value that moves with key e, to sorted place in rank[256 ..].
+// carry(e): a value that moves with key e, to sorted place in rank[kCarry ..].
 template <int TB, typename Carry>
 __device__ __forceinline__ void rank_sort(int64_t* list, int n, int* rank, Carry carry) {
   constexpr int G = TB / 256;
@@ -1380,7 +1391,7 @@ __device__ __forceinline__ void rank_sort(int64_t* list, int n, int* rank, Carry
   const int with = g == 0 && e < n ? carry(e) : 0;
   if (g == 0) {
     if (e >= n) list[e] = MLP_KEY_NONE;
-    rank[e] = 0;
+    if constexpr (G > 1) rank[e] = 0;
   }
   __syncthreads();
   int r = 0;
@@ -1399,7 +1410,7 @@ __device__ __forceinline__ void rank_sort(int64_t* list, int n, int* rank, Carry
   if (g == 0 && e < n) {
     if constexpr (G > 1) r = rank[e];
     list[r] = my;
-    rank[256 + r] = with;
+    rank[MergeShared<TB>::kCarry + r] = with;
   }
   __syncthreads();
 }
@@ -1597,7 +1608,7 @@ __device__ __forceinline__ int select_spans(const Slot& s, int nb, int N, int ro
     rank_sort<TB>(S.list, n, S.hist, [&](int e) { return (int)ctxL[(int)(S.list[e] & MLP_KEY_MASK)]; });
     if (tid < kWave) {
       const int kk = greedy_wave<KIND>(
-          s, nb, N, rowmap, n, S.list, out, kept, [&](int t, int64_t) { return S.hist[256 + t]; }, bits,
+          s, nb, N, rowmap, n, S.list, out, kept, [&](int t, int64_t) { return S.hist[S.kCarry + t]; }, bits,
           lane, nullptr, INT32_MAX);
       if (lane == 0) {
         S.kept = kk;
@@ -1861,7 +1872,7 @@ __device__ __forceinline__ int sort_greedy(const Slot& s, int nb, int rowmap, in
       constexpr int KIND = decltype(kind)::value;
       if (M <= kSelCap)  // one list, its ctx beside it
         return greedy_wave<KIND>(
-            s, nb, N, rowmap, M, in, sk, 0, [&](int t, int64_t) { return S.hist[256 + t]; }, bits, tid,
+            s, nb, N, rowmap, M, in, sk, 0, [&](int t, int64_t) { return S.hist[S.kCarry + t]; }, bits, tid,
             nullptr, INT32_MAX);
       return greedy_wave<KIND>(
           s, nb, N, rowmap, M, in, sk, 0, [&](int, int64_t key) { return ctx_of(key); }, bits, tid, gtail,
