@@ -164,6 +164,20 @@ int fused_grid() {
   return 0;
 }
 
+// Merges of more slots than the GPU has CUs (256) say so to their launch.
+int wide_merges() {
+  for (int count : {1, 255, 256, 257, 300}) {
+    Run r(std::vector<int>(count, 20));
+    counts = Counts();
+    CHECK(mlp_eval(r.ctx, r.slots.data(), count, 3, 0, 0) == MLP_OK &&
+              mlp_merge_apply(r.ctx, r.slots.data(), count, 1) == MLP_OK,
+          "%s", mlp_ctx_error(r.ctx));
+    CHECK(counts.wide == (count > 256) && counts.narrow == (count <= 256), "%d slots: %d wide, %d not", count,
+          counts.wide, counts.narrow);
+  }
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -171,7 +185,8 @@ int main(int argc, char** argv) {
   const int bad = what == "graphs" ? graphs() : what == "failed_rows" ? failed_rows()
                   : what == "evaluations" ? evaluations()
                   : what == "timed" ? timed()
-                  : what == "fused_grid" ? fused_grid() : 2;
+                  : what == "fused_grid" ? fused_grid()
+                  : what == "wide_merges" ? wide_merges() : 2;
   if (!bad) printf("%s ok\n", what.c_str());
   return bad;
 }

@@ -168,7 +168,8 @@ void merge(const SlotDev* table, const std::vector<int32_t>& ids, int tail) {
 }
 }  // namespace
 hipError_t mlp_launch_merge_apply(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
-                                  const int32_t* dev, int count, int, int, int, int, int, int tail) {
+                                  const int32_t* dev, int count, int, int, int, int, int flags, int tail) {
+  ++(flags & MLP_MERGE_WIDE ? counts.wide : counts.narrow);
   submit(st, [=] { merge(table, listed(inl.id, dev, count), tail); });
   return hipSuccess;
 }

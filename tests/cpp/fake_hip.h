@@ -19,6 +19,7 @@ struct Counts {
   int replayed = 0;
   int fused_grid = 0;    // workgroups of the last launch of a fused round, LDS of each
   size_t fused_lds = 0;
+  int narrow = 0, wide = 0;  // merges by MLP_MERGE_WIDE
   int worked = 0;        // evaluations of a neighborhood of a slot that did not return at once
 };
 extern Counts counts;

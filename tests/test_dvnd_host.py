@@ -24,7 +24,7 @@ def check(tmp_path_factory):
     return str(exe)
 
 
-@pytest.mark.parametrize("what", ["graphs", "failed_rows", "evaluations", "timed", "fused_grid"])
+@pytest.mark.parametrize("what", ["graphs", "failed_rows", "evaluations", "timed", "fused_grid", "wide_merges"])
 def test_dvnd_host(check, what):
     out = subprocess.run([check, what], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0, out.stdout + out.stderr

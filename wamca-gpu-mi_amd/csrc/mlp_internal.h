@@ -180,6 +180,12 @@ struct FusedPlan {
 #endif
 
 #define MLP_SLOTS_INLINE 128
+// flags of a merge's launch
+enum {
+  MLP_MERGE_ROUND = 1,  // inside a DVND round: inactive slots are skipped, parities committed
+  MLP_MERGE_KEEP = 2,   // block summaries of the new tour are kept
+  MLP_MERGE_WIDE = 4,   // more slots than the GPU holds workgroups of the usual width
+};
 // 64-bit word ranges of a slot block holding row buffers (set to KEY_NONE
 // when the slot is created)
 // Row buffers read by mlp_eval_static's output.

@@ -1939,7 +1939,7 @@ __device__ __forceinline__ void merge_slot(const SlotRegs& s, int nb, int rowmap
   const int N = s.N, tid = threadIdx.x;
   const int R = rows_of(nb, rowmap, N);
   const int pcap = pcap_l, ncap = ncap_l;  // capacities of the launch
-  const bool dvnd = flags != 0;
+  const bool dvnd = (flags & 1) != 0;
   int64_t* keys = lds;
   int32_t* told = (int32_t*)(keys + pcap);
   int32_t* tnew = told + ncap;
@@ -1963,13 +1963,18 @@ __device__ __forceinline__ void merge_slot(const SlotRegs& s, int nb, int rowmap
   // is active is looked at afterwards, so that no load waits for the info
   // words (a merge n = 1000 7.4 -> 6.8 us, n = 100 4.3 -> 3.6).
   const int par = (int)(parity & 1) ^ (dvnd ? 1 : 0);
-  const auto rk = s.rows;
-  const int cap = s.rowcap;
+  auto ra = s.rows, rb = s.rows + s.rowcap;
+  if (flags & MLP_MERGE_WIDE) {
+    // other workgroups hide the wait, and the second buffer would cost
+    // bandwidth (1500 tours n = 600 at their optimum 62 us -> 54)
+    if (dvnd && active == 0) return;
+    ra = rb = par ? rb : ra;
+  }
   merge_rows<TB, PER>(
       s,
       [&](int q, int64_t& a, int64_t& b) {
-        a = rk[q];
-        b = rk[cap + q];
+        a = ra[q];
+        b = rb[q];
       },
       [&](int64_t a, int64_t b) { return par ? b : a; }, R, 0, max(R, N), told, tnew, xyc, ctxL,
       [&](int64_t k) { keys[atomicAdd(&S.m, 1)] = k; });
@@ -4133,10 +4138,16 @@ static_assert(kGmemMergeLds + sizeof(MergeShared<kSelBlock>) <= 160 * 1024, "LDS
 
 // The merge's workgroup for tours of up to n positions: as few positions a
 // thread as 1024 threads allow (its steps over the tour are one batch each).
-#define MLP_MERGE_FOR(n, F)          \
+// A CU holds one workgroup of 1024 (77 registers) but three of 512, so a launch
+// over more slots than CUs (wide) takes 512 threads up to 2048 positions: swap
+// merges of 1500 random tours n = 600 152 us -> 102 (124 with the 256 threads
+// of old), 600 tours n = 1500 120 -> 79; 400 tours n = 2500 106 against 125.
+#define MLP_MERGE_FOR(n, wide, F)    \
   do {                               \
     if ((n) <= 256) F(256, 1);       \
     else if ((n) <= 512) F(512, 1);  \
+    else if ((wide) && (n) <= 1024) F(512, 2); \
+    else if ((wide) && (n) <= 2048) F(512, 4); \
     else if ((n) <= 1024) F(1024, 1); \
     else if ((n) <= 2048) F(1024, 2); \
     else if ((n) <= 4096) F(1024, 4); \
@@ -4148,7 +4159,8 @@ hipError_t mlp_merge_setup(size_t max_dyn_lds) {
 #define MLP_MERGE_ATTR(TB, PER)                                                              \
   e = hipFuncSetAttribute((const void*)k_merge_apply<TB, PER>,                               \
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_dyn_lds)
-  for (int n = 256; n <= 8192 && e == hipSuccess; n *= 2) MLP_MERGE_FOR(n, MLP_MERGE_ATTR);
+  for (int n = 256; n <= 8192 && e == hipSuccess; n *= 2)
+    for (int wide = 0; wide < 2 && e == hipSuccess; ++wide) MLP_MERGE_FOR(n, wide, MLP_MERGE_ATTR);
   if (e == hipSuccess)
     e = hipFuncSetAttribute((const void*)k_mg_select, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)kGmemMergeLds);
@@ -4178,12 +4190,12 @@ hipError_t mlp_launch_fused(hipStream_t st, const SlotDev* table, const FusedPla
 
 hipError_t mlp_launch_merge_apply(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
                                   const int32_t* list_dev, int count, int nb, int rowmap,
-                                  int pcap, int ncap, int skip_inactive, int tail) {
+                                  int pcap, int ncap, int flags, int tail) {
 #define MLP_MERGE_LAUNCH(TB, PER)                                                             \
   hipLaunchKernelGGL((k_merge_apply<TB, PER>), dim3(count), dim3(TB),                          \
                      mlp_merge_lds_bytes(pcap, ncap), st, table, inl, list_dev, nb, rowmap, pcap, \
-                     ncap, skip_inactive, tail)
-  MLP_MERGE_FOR(ncap, MLP_MERGE_LAUNCH);
+                     ncap, flags, tail)
+  MLP_MERGE_FOR(ncap, flags & MLP_MERGE_WIDE, MLP_MERGE_LAUNCH);
   return hipGetLastError();
 }
 

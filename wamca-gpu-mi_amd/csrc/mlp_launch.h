@@ -45,7 +45,7 @@ hipError_t mlp_merge_setup(size_t max_dyn_lds);
 // tail > 0: the last merge of a DVND round also ends the round (max_rounds = tail - 1).
 hipError_t mlp_launch_merge_apply(hipStream_t st, const SlotDev* table, const SlotListInline& inl,
                                   const int32_t* list_dev, int count, int nb, int rowmap,
-                                  int pcap, int ncap, int skip_inactive, int tail);
+                                  int pcap, int ncap, int flags, int tail);
 // The merge of slots whose working arrays exceed LDS over many workgroups
 // per slot (three launches; max_n: the largest N among the slots).
 hipError_t mlp_launch_merge_gmem(hipStream_t st, const SlotDev* table, const SlotListInline& inl,

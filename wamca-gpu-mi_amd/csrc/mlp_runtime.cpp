@@ -1637,8 +1637,12 @@ static int merge_impl(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t
   // room beside the keys for the selections of merges with many improving
   // rows (a position array for swaps, the kept spans), where LDS has it
   if (ncap > 256) {
+    const int need = ncap + std::max(ncap, 512);
     int roomy = pcap;
-    while (roomy < ncap + std::max(ncap, 512)) roomy <<= 1;
+    while (roomy < need) roomy <<= 1;
+    // no more than that in a wide launch, whose workgroups share a CU (tours
+    // n = 1500: three, not two)
+    if ((int)in_lds.size() > ctx->cu_count) roomy = std::max(pcap, need);
     if (mlp_merge_lds_bytes(roomy, ncap) <= ctx->max_merge_lds) pcap = roomy;
   }
   for (int q = 0; q < count; ++q) ctx->slots[slots[q]].merged[nb] = true;
@@ -1659,7 +1663,7 @@ static int merge_impl(mlp_ctx* ctx, const int32_t* slots, int32_t count, int32_t
                                   gmem_n));
       else
         HCK(mlp_launch_merge_apply(ctx->stream, ctx->d_table, inl, dev, c, nb, rowmap, pcap, ncap,
-                                   skip, tail));
+                                   skip | (c > ctx->cu_count ? MLP_MERGE_WIDE : 0), tail));
     }
   }
   return MLP_OK;
