@@ -13,7 +13,10 @@ Counts counts;
 std::function<int(int)> rounds_of_slot = [](int) { return 1 << 20; };
 int fail_sync = 0;
 static const SlotDev* last_table = nullptr;
-bool left_out(int slot) { return last_table[slot].info[MLP_INFO_PARTIAL] == 1; }
+bool left_out(int slot) {
+  const int64_t* info = last_table[slot].info;
+  return info[MLP_INFO_PARTIAL] > 0 && info[MLP_INFO_PARTIAL] == info[MLP_INFO_ROUNDS] + (info[MLP_INFO_ACTIVE] ? 1 : 0);
+}
 
 namespace {
 
@@ -133,14 +136,15 @@ hipError_t mlp_launch_dvnd_start(hipStream_t st, const SlotDev* table, const Slo
   });
   return hipSuccess;
 }
-hipError_t mlp_launch_sweep(hipStream_t st, int, const SlotDev* table, const SweepSegsInline& inl,
-                            const SweepSeg* dev, int nsegs, int, int*, int, int flags) {
-  submit_eval(st, flags & 8 ? &Counts::fills : &Counts::evals, [=] {
+hipError_t mlp_launch_sweep(hipStream_t st, int tile, const SlotDev* table, const SweepSegsInline& inl,
+                            const SweepSeg* dev, int nsegs, int, int*, int, int) {
+  const bool fill = (tile & MLP_TILE_FILL) != 0;
+  submit_eval(st, fill ? &Counts::fills : &Counts::evals, [=] {
     for (const SweepSeg& g : listed(inl.s, dev, nsegs)) {
       int64_t* info = table[g.slot].info;
-      if (flags & 8 ? info[MLP_INFO_PARTIAL] : info[MLP_INFO_ACTIVE]) counts.worked += __builtin_popcount(g.mask);
-      if (flags & 8) info[MLP_INFO_PARTIAL] *= 2;  // (the device's word stays 1: nothing reads it again)
-      else if (info[MLP_INFO_ACTIVE]) info[MLP_INFO_PARTIAL] = 0;
+      if (fill ? info[MLP_INFO_PARTIAL] == info[MLP_INFO_ROUNDS] : info[MLP_INFO_ACTIVE])
+        counts.worked += __builtin_popcount(g.mask);
+      if (fill) info[MLP_INFO_PARTIAL] = 0;  // (the device's word stays: nothing reads it again)
     }
   });
   return hipSuccess;
@@ -150,7 +154,7 @@ hipError_t mlp_launch_psweep(hipStream_t st, const SlotDev* table, const SweepSe
   submit_eval(st, &Counts::pruned, [=] {
     for (const SweepSeg& g : listed(inl.s, dev, nsegs))
       if (table[g.slot].info[MLP_INFO_ACTIVE]) {
-        table[g.slot].info[MLP_INFO_PARTIAL] = 1;
+        table[g.slot].info[MLP_INFO_PARTIAL] = table[g.slot].info[MLP_INFO_ROUNDS] + 1;
         ++counts.worked;
       }
   });

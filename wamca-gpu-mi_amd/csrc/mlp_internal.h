@@ -33,7 +33,7 @@ enum {
   MLP_INFO_KEPT0 = 8,     // kept-move count of nb (8 + nb)
   MLP_INFO_MG_APPLY = 23, // moves the last many-workgroup merge applied (its rebuild runs if > 0)
   MLP_INFO_PARITY0 = 24,  // row buffer (0/1) holding the last eval of nb (24 + nb)
-  MLP_INFO_PARTIAL = 39,  // 1: the last DVND round kept only improving rows (k_psweep)
+  MLP_INFO_PARTIAL = 39,  // the last round (from 1) that kept only improving rows (k_psweep)
   MLP_INFO_WORDS = 40
 };
 
@@ -62,8 +62,8 @@ struct SlotDev {
   int32_t n;      // clients
   int32_t round;  // 0 trunc, 1 nint
   int32_t maxd;   // upper bound of any distance in the instance
-  int32_t small;  // every squared distance is below 2^21 (short distance form)
   int32_t rowcap; // entries per row buffer (rows[nb] holds two buffers)
+  int32_t small;  // every squared distance is below 2^21 (short distance form)
   const int32_t* xs;  // instance coordinates (client indexed)
   const int32_t* ys;
   int32_t* tour;  // [N]
@@ -75,7 +75,6 @@ struct SlotDev {
   int32_t* h32;   // [N] 2-opt j-side constant Z[p] - (N-p-1) w[p+1]  (mod 2^32)
   int64_t* t64;   // [N]
   int64_t* q64;   // [N]
-  BlkSum* blk;    // [ceil(N / MLP_BLK)]
   int64_t* info;  // [MLP_INFO_WORDS]
   // per-row best keys (delta << 20 | ctx), two buffers of rowcap entries.
   // info[PARITY0 + nb] = p names the buffer holding the last result; the
@@ -88,6 +87,7 @@ struct SlotDev {
   int32_t* kept_ij[MLP_NB_MAX];   // (i, j, row) triplets
   int32_t nbs;                    // neighborhoods with buffers (ids 0 .. nbs-1)
   void* mscratch;  // the merge's working arrays when they exceed LDS (layout of its LDS)
+  BlkSum* blk;     // [ceil(N / MLP_BLK)]
 };
 
 // Z[p] = 2 Q[p] - (2p + 1) T[p] turns the 2-opt internal sum into
@@ -137,6 +137,12 @@ struct SweepSeg {
 // each tile it crosses, and all of a tour's tiles fold at once, so the row
 // count of the tile sets the contention on each ODC row).
 #define MLP_TILE_ODC 0x200
+// flag beside a shape: every slot of the launch has short distances
+// (SlotDev.small), now and in every replay of the launch.
+#define MLP_TILE_SMALL 0x400
+// ... the rows that a finished DVND run left out are completed (shapes 4 x 256
+// and 8 x 512, ADS row map).
+#define MLP_TILE_FILL 0x800
 
 #define MLP_SEGS_INLINE 32
 struct EvalSegsInline {

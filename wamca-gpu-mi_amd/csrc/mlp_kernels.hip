@@ -155,6 +155,16 @@ struct FullDist {
   float dr;
   __device__ __forceinline__ int operator()(int s) const { return dist_s(s, dr); }
 };
+// Which of them a tile uses: one for the whole launch (both side by side cost
+// the small tiles registers: 4 x 256 with two spilled to memory, one tour
+// n = 100 17.6 -> 18.5 us, 256 tours n = 1000 in [0, 2000]^2, or-opt-1 alone
+// 257 -> 265), or its slot's (fused rounds).
+constexpr int kFullDist = 0, kSmallDist = 1, kSlotDist = 2;
+template <int DIST>
+__device__ __forceinline__ auto tile_dist(int round, float dr) {
+  if constexpr (DIST == kSmallDist) return fast_dist(round);
+  else return FullDist{dr};
+}
 template <typename Dist>
 __device__ __forceinline__ int dist_by(int a, int b, const Dist& D) {
   const short2v d = __builtin_bit_cast(short2v, a) - __builtin_bit_cast(short2v, b);
@@ -2886,10 +2896,6 @@ __device__ __forceinline__ void reset_other(const SlotDev& s, int nb, int par, i
   }
 }
 
-// Bit of a tile's parity word: it folds into buffers that already hold moves
-// of the same tour and resets nothing.
-constexpr int kNoReset = 1 << 30;
-
 // Value barrier: the compiler sees an opaque value, so a per-column term
 // stays one shared value instead of being distributed into every row's
 // products (which turns two 24-bit multiplies into one quarter-rate 32-bit
@@ -3273,14 +3279,14 @@ __device__ __forceinline__ void tile_oropt(const SlotDev& s, int b0, int q0, int
 
 // int64 fallback of a fixed-i tile (column tile 0 only): one wave per
 // (neighborhood, row) over the whole row.
-template <int R, int RM = 0>
+template <int R, int RM, bool FILL>
 __device__ __forceinline__ void sweep_fixed_wide(const SlotDev& s, int rb, int ct, int mask, int parity) {
   const int N = s.N, wave = wave_id(), lane = threadIdx.x % kWave;
   const int b0 = rb * R;
   if (ct != 0) return;
 #pragma unroll
   for (int nb = 0; nb < MLP_NB_COUNT; ++nb)
-    if (nb != 1 && ((mask >> nb) & 1) && !(parity & kNoReset))
+    if (nb != 1 && ((mask >> nb) & 1) && !FILL)
       reset_other(s, nb, (parity >> nb) & 1, b0, min(b0 + R, rows_of(nb, RM, N)), rb == 0, RM);
   for (int sg = wave; sg < 4 * R; sg += kBlock / kWave) {
     const int g = sg / R, by = b0 + sg % R;
@@ -3296,21 +3302,21 @@ __device__ __forceinline__ void sweep_fixed_wide(const SlotDev& s, int rb, int c
 // but whose tour does not take the in-tile path (64-bit deltas, or
 // T[N-1] >= 2^24): column tile 0 resets them and evaluates each diagonal row
 // with one wave.
-template <int R>
+template <int R, bool FILL>
 __device__ __forceinline__ void two_rows_wide(const SlotDev& s, int rb, int ct, int parity,
                                               bool p32) {
   if (ct != 0) return;
   const int N = s.N, wave = wave_id(), lane = threadIdx.x % kWave;
   const int rows2 = (N + 1) >> 1, b0 = rb * R;
   const int par = (parity >> 1) & 1;
-  if (!(parity & kNoReset)) reset_other(s, 1, par, b0, min(b0 + R, rows2), rb == 0);
+  if (!FILL) reset_other(s, 1, par, b0, min(b0 + R, rows2), rb == 0);
   for (int by = b0 + wave; by < min(b0 + R, rows2); by += kBlock / kWave) {
     if (p32) eval_row<1, true>(s, 1, 0, by, lane, row_buf(s, 1, par) + by);
     else eval_row<1, false>(s, 1, 0, by, lane, row_buf(s, 1, par) + by);
   }
 }
 
-template <int R, int C, int X>
+template <int R, int C, int X, int DIST, bool FILL>
 __device__ __forceinline__ void sweep_fixed(const SlotDev& s, int rb, int ct, int mask, int parity,
                             FixedLds<R, C, X>& F, bool filtered) {
   constexpr bool TWO = X == kTwo;
@@ -3357,12 +3363,12 @@ __device__ __forceinline__ void sweep_fixed(const SlotDev& s, int rb, int ct, in
     if (TWO) rgv = ldg(s.g32 + p);
   }
   if (TWO && (mask & 2) && !two)
-    two_rows_wide<R>(s, rb, ct, parity, (pflags & MLP_P32_2OPT) != 0);
+    two_rows_wide<R, FILL>(s, rb, ct, parity, (pflags & MLP_P32_2OPT) != 0);
   if (!p32) {
-    sweep_fixed_wide<R, RM>(s, rb, ct, mask, parity);
+    sweep_fixed_wide<R, RM, FILL>(s, rb, ct, mask, parity);
     return;
   }
-  if (ct == 0 && !(parity & kNoReset)) {
+  if (ct == 0 && !FILL) {
 #pragma unroll
     for (int nb = 0; nb < MLP_NB_COUNT; ++nb)
       if (nb != 1 && ((mask >> nb) & 1))
@@ -3371,21 +3377,18 @@ __device__ __forceinline__ void sweep_fixed(const SlotDev& s, int rb, int ct, in
   }
   // swap alone covers j >= i + 2 only: a tile left of that diagonal is empty
   if (mask == 1 && q1 <= b0 + 3) return;
-  auto fill = [&](const auto& dist) {
+  const auto dist = tile_dist<DIST>(s.round, dr);
 #pragma unroll
-    for (int it = 0; it < FI; ++it) {
-      const int c = cfill + tid + it * kBlock;
-      if (c < cend) {
+  for (int it = 0; it < FI; ++it) {
+    const int c = cfill + tid + it * kBlock;
+    if (c < cend) {
 #pragma unroll
-        for (int va = 0; va < R + 4; ++va) L.v[va][c - cbase] = (uint16_t)dist_by(xa[va], xc[it], dist);
-        L.w[c - cbase] = (uint16_t)wv[it];
-        L.t[c - cbase] = tv[it];
-        if constexpr (TWO) F.two.h[c - cbase] = hv[it];
-      }
+      for (int va = 0; va < R + 4; ++va) L.v[va][c - cbase] = (uint16_t)dist_by(xa[va], xc[it], dist);
+      L.w[c - cbase] = (uint16_t)wv[it];
+      L.t[c - cbase] = tv[it];
+      if constexpr (TWO) F.two.h[c - cbase] = hv[it];
     }
-  };
-  if (s.small) fill(fast_dist(s.round));
-  else fill(FullDist{dr});
+  }
   if (tid < R + 8) {
     L.rw[tid] = rwv;
     L.rt[tid] = rtv;
@@ -3486,18 +3489,19 @@ __device__ __forceinline__ void sweep_fixed(const SlotDev& s, int rb, int ct, in
   }
 }
 
+template <bool FILL>
 __device__ __forceinline__ void sweep_2opt_wide(const SlotDev& s, int rb, int ct, int parity) {
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int rows = (s.N + 1) >> 1;
   const int par = (parity >> 1) & 1;
   if (ct != 0) return;
-  if (!(parity & kNoReset))
+  if (!FILL)
     reset_other(s, 1, par, rb * MLP_2OPT_ROWS, min(rb * MLP_2OPT_ROWS + MLP_2OPT_ROWS, rows), rb == 0);
   const int by = rb * MLP_2OPT_ROWS + wave;
   if (by < rows) eval_row<1, false>(s, 1, 0, by, lane, row_buf(s, 1, par) + by);
 }
 
-template <int C>
+template <int C, int DIST, bool FILL>
 __device__ __forceinline__ void sweep_2opt(const SlotDev& s, int rb, int ct, int parity, DiagLds<C>& L) {
   constexpr int FE = (C + 1 + kWave - 1) / kWave;  // e entries per lane and part
   constexpr int FT = (C + 2 + kWave - 1) / kWave;  // e entries per lane, both parts
@@ -3566,40 +3570,37 @@ __device__ __forceinline__ void sweep_2opt(const SlotDev& s, int rb, int ct, int
   // arithmetic; the small ones, whose register budget sets their occupancy,
   // take one wave per row over the whole row.
   if (!p32 && C < 1024) {
-    sweep_2opt_wide(s, rb, ct, parity);
+    sweep_2opt_wide<FILL>(s, rb, ct, parity);
     return;
   }
-  if (ct == 0 && !(parity & kNoReset))
+  if (ct == 0 && !FILL)
     reset_other(s, 1, par, rb * MLP_2OPT_ROWS, min(rb * MLP_2OPT_ROWS + MLP_2OPT_ROWS, rows), rb == 0);
-  auto fill = [&](const auto& dist) {
-    if constexpr (FLAT) {
-      if (net > 0) {
+  const auto dist = tile_dist<DIST>(s.round, dr);
+  if constexpr (FLAT) {
+    if (net > 0) {
 #pragma unroll
-        for (int it = 0; it < FI; ++it) {
-          const int x = lane + it * kWave;
-          if (x < net) {
-            const bool p1 = x >= ne0;
-            L.e[wave][p1 ? 1 : 0][p1 ? x - ne0 : x] = (uint16_t)dist_by(pa[0][it], pb[0][it], dist);
-          }
-        }
-      }
-    } else {
-#pragma unroll
-      for (int part = 0; part < FP; ++part) {
-        const int ne = part ? ne1 : ne0;
-        uint16_t* e = L.e[wave][part];
-        if (ne >= 2) {
-#pragma unroll
-          for (int it = 0; it < FI; ++it) {
-            const int x = lane + it * kWave;
-            if (x < ne) e[x] = (uint16_t)dist_by(pa[part][it], pb[part][it], dist);
-          }
+      for (int it = 0; it < FI; ++it) {
+        const int x = lane + it * kWave;
+        if (x < net) {
+          const bool p1 = x >= ne0;
+          L.e[wave][p1 ? 1 : 0][p1 ? x - ne0 : x] = (uint16_t)dist_by(pa[0][it], pb[0][it], dist);
         }
       }
     }
-  };
-  if (s.small) fill(fast_dist(s.round));
-  else fill(FullDist{dr});
+  } else {
+#pragma unroll
+    for (int part = 0; part < FP; ++part) {
+      const int ne = part ? ne1 : ne0;
+      uint16_t* e = L.e[wave][part];
+      if (ne >= 2) {
+#pragma unroll
+        for (int it = 0; it < FI; ++it) {
+          const int x = lane + it * kWave;
+          if (x < ne) e[x] = (uint16_t)dist_by(pa[part][it], pb[part][it], dist);
+        }
+      }
+    }
+  }
   __syncthreads();
   // A tour above the int32 bound can still have rows whose moves all stay
   // below 2^31: reversing positions i..j moves each reversed node's arrival
@@ -3767,33 +3768,38 @@ __device__ __forceinline__ SweepSeg find_sweep_dev(const SweepSeg* segs, int nse
   return segs[2 * g + (item - g * group >= segs[1].blk0 ? 1 : 0)];
 }
 
-template <int R, int C, int X>
+// FILL: the rows of a finished DVND run whose last round kept only the
+// improving ones, completed in place (the tour is the one they were evaluated
+// on: that round applied no move); nothing is reset.
+template <int R, int C, int X, int DIST, bool FILL>
 __device__ __forceinline__ void sweep_item(const SlotDev* __restrict__ table, const SweepSeg& sg, int item,
-                           SweepLds<R, C, X>& L, bool dvnd, bool filtered, bool fill = false) {
+                           SweepLds<R, C, X>& L, bool dvnd, bool filtered) {
   const SlotDev& s = table[sg.slot];
-  // fill: the rows of a finished DVND run whose last round kept only the
-  // improving ones, completed in place (the tour is the one they were
-  // evaluated on: that round applied no move)
-  if (fill ? s.info[MLP_INFO_PARTIAL] == 0 : dvnd && s.info[MLP_INFO_ACTIVE] == 0) return;
+  if (FILL ? s.info[MLP_INFO_PARTIAL] != s.info[MLP_INFO_ROUNDS] : dvnd && s.info[MLP_INFO_ACTIVE] == 0) return;
   // bit nb of par: the buffer this sweep writes (the one not holding the last result)
   int par = sg.parity;
   if (dvnd) {
     par = 0;
 #pragma unroll
     for (int nb = 0; nb < MLP_NB_COUNT; ++nb)
-      if ((sg.mask >> nb) & 1) par |= (int)((s.info[MLP_INFO_PARITY0 + nb] & 1) ^ (fill ? 0 : 1)) << nb;
-    if (fill) par |= kNoReset;
+      if ((sg.mask >> nb) & 1) par |= (int)((s.info[MLP_INFO_PARITY0 + nb] & 1) ^ (FILL ? 0 : 1)) << nb;
   }
   const int b = item - sg.blk0;
-  if (dvnd && !fill && b == 0 && threadIdx.x == 0) s.info[MLP_INFO_PARTIAL] = 0;
   const int rb = b / sg.ncols, ct = b % sg.ncols;
   if (!dvnd && b == 0 && threadIdx.x == 0) {
 #pragma unroll
     for (int nb = 0; nb < MLP_NB_COUNT; ++nb)
       if ((sg.mask >> nb) & 1) s.info[MLP_INFO_PARITY0 + nb] = (par >> nb) & 1;
   }
-  if (sg.kind == 0) sweep_fixed<R, C, X>(s, rb, ct, sg.mask, par, L.f, filtered);
-  else sweep_2opt<C>(s, rb, ct, par, L.d);
+  if constexpr (DIST == kSlotDist) {
+    if (s.small) {
+      if (sg.kind == 0) sweep_fixed<R, C, X, kSmallDist, FILL>(s, rb, ct, sg.mask, par, L.f, filtered);
+      else sweep_2opt<C, kSmallDist, FILL>(s, rb, ct, par, L.d);
+      return;
+    }
+  }
+  if (sg.kind == 0) sweep_fixed<R, C, X, DIST, FILL>(s, rb, ct, sg.mask, par, L.f, filtered);
+  else sweep_2opt<C, DIST, FILL>(s, rb, ct, par, L.d);
 }
 
 }  // namespace
@@ -3803,7 +3809,7 @@ __device__ __forceinline__ void sweep_item(const SlotDev* __restrict__ table, co
 // depends on every tile being resident at once, and many-tour launches,
 // which gain from the occupancy.  The large shapes are held to three
 // workgroups per CU by their LDS tiles anyway.
-template <int R, int C, int X>
+template <int R, int C, int X, int DIST, bool FILL>
 __global__ __launch_bounds__(kBlock, (R * C <= 2048 ? 7 : 1)) void k_sweep(
     const SlotDev* __restrict__ table,
                                                   SweepSegsInline inl, const SweepSeg* segs_dev,
@@ -3812,15 +3818,14 @@ __global__ __launch_bounds__(kBlock, (R * C <= 2048 ? 7 : 1)) void k_sweep(
   // flags bit 0: a DVND launch (inactive slots skipped, parities read from
   // info); bit 1: filtered folds of the diagonal rows (many more tiles than
   // resident workgroups, so most tiles fold after others of their tour);
-  // bits 2, 8..31: equal segments per slot (find_sweep_dev); bit 3: rows that
-  // a finished DVND run left incomplete (with bit 0)
+  // bits 2, 8..31: equal segments per slot (find_sweep_dev)
   __shared__ SweepLds<R, C, X> L;
-  const bool dvnd = (flags & 1) != 0, filtered = (flags & 2) != 0, fill = (flags & 8) != 0;
+  const bool dvnd = (flags & 1) != 0, filtered = (flags & 2) != 0;
   if (!counter) {
     const int item = blockIdx.x;
     const SweepSeg sg = segs_dev ? find_sweep_dev(segs_dev, nsegs, item, flags)
                                   : find_sweep_inline(inl, nsegs, item);
-    sweep_item<R, C, X>(table, sg, item, L, dvnd, filtered, fill);
+    sweep_item<R, C, X, DIST, FILL>(table, sg, item, L, dvnd, filtered);
     return;
   }
   __shared__ int s_item;
@@ -3832,7 +3837,7 @@ __global__ __launch_bounds__(kBlock, (R * C <= 2048 ? 7 : 1)) void k_sweep(
     if (item >= total) break;
     const SweepSeg sg = segs_dev ? find_sweep_dev(segs_dev, nsegs, item, flags)
                                   : find_sweep_inline(inl, nsegs, item);
-    sweep_item<R, C, X>(table, sg, item, L, dvnd, filtered, fill);
+    sweep_item<R, C, X, DIST, FILL>(table, sg, item, L, dvnd, filtered);
     __syncthreads();
   }
 }
@@ -3948,7 +3953,7 @@ __global__ __launch_bounds__(kBlock) void k_dvnd_fused(const SlotDev* __restrict
       const int g = e - pre[q];
       const int t1 = min((g + 1) * P.group, P.tiles[nb * P.count + q]);
       for (int t = g * P.group; t < t1; ++t) {
-        sweep_item<R, C, kPlain>(table, sg, t, L, true, true);
+        sweep_item<R, C, kPlain, kSlotDist, false>(table, sg, t, L, true, true);
         __syncthreads();  // the next tile reuses the LDS
       }
       signal_done(done + q);
@@ -3970,9 +3975,11 @@ __global__ __launch_bounds__(kBlock) void k_dvnd_fused(const SlotDev* __restrict
 
 template __global__ void k_dvnd_fused<MLP_FUSED_R, MLP_FUSED_C>(const SlotDev*, FusedPlan);
 
+#define MLP_SWEEP_INST_OF(R, C, X, DIST, FILL)                                        \
+  template __global__ void k_sweep<R, C, X, DIST, FILL>(const SlotDev*, SweepSegsInline,         \
+                                                        const SweepSeg*, int, int, int*, int);
 #define MLP_SWEEP_INST(R, C, X)                                                       \
-  template __global__ void k_sweep<R, C, X>(const SlotDev*, SweepSegsInline, const SweepSeg*,   \
-                                            int, int, int*, int);
+  MLP_SWEEP_INST_OF(R, C, X, kFullDist, false) MLP_SWEEP_INST_OF(R, C, X, kSmallDist, false)
 MLP_SWEEP_INST(4, 256, kPlain)
 MLP_SWEEP_INST(8, 512, kPlain)
 MLP_SWEEP_INST(16, 1024, kPlain)
@@ -3988,6 +3995,10 @@ MLP_SWEEP_INST(4, 256, kOdc)
 MLP_SWEEP_INST(8, 512, kOdc)
 MLP_SWEEP_INST(16, 128, kOdc)
 MLP_SWEEP_INST(4, 512, kOdc)
+// a finished run's rows completed: once a run, so few shapes and one form
+MLP_SWEEP_INST_OF(4, 256, kPlain, kFullDist, true)
+MLP_SWEEP_INST_OF(8, 512, kPlain, kFullDist, true)
+MLP_SWEEP_INST_OF(8, 512, kTwo, kFullDist, true)
 
 // ===========================================================================
 // host-side launch wrappers (called by the C ABI runtime in mlp_runtime.cpp)
@@ -4055,9 +4066,18 @@ hipError_t mlp_launch_sweep(hipStream_t st, int tile, const SlotDev* table,
   // variants; MLP_TILE_ODC: the ODC row map (16 x 1024 runs as 8 x 512,
   // 8 x 256 as 16 x 128)
 #define MLP_SWEEP_LAUNCH(R, C, X)                                                              \
-  hipLaunchKernelGGL((k_sweep<R, C, X>), dim3(grid), dim3(kBlock), 0, st, table, inl,          \
-                     segs_dev, nsegs, total, counter, flags)
+  MLP_SWEEP_GO((small ? k_sweep<R, C, X, kSmallDist, false> : k_sweep<R, C, X, kFullDist, false>))
+#define MLP_SWEEP_GO(KERNEL)                                                                   \
+  hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(kBlock), 0, st, table, inl, segs_dev, nsegs,     \
+                     total, counter, flags)
   const bool two = (tile & MLP_TILE_TWO) != 0, odc = (tile & MLP_TILE_ODC) != 0;
+  const bool small = (tile & MLP_TILE_SMALL) != 0;
+  if (tile & MLP_TILE_FILL) {
+    if ((tile & 0xff) == MLP_TILE_4x256) MLP_SWEEP_GO((k_sweep<4, 256, kPlain, kFullDist, true>));
+    else if (two) MLP_SWEEP_GO((k_sweep<8, 512, kTwo, kFullDist, true>));
+    else MLP_SWEEP_GO((k_sweep<8, 512, kPlain, kFullDist, true>));
+    return hipGetLastError();
+  }
   switch (tile & 0xff) {
     case MLP_TILE_4x256:
       if (odc) MLP_SWEEP_LAUNCH(4, 256, kOdc);

@@ -494,7 +494,7 @@ __global__ __launch_bounds__(kBlock) void k_psweep(const SlotDev* __restrict__ t
   const int par = 1 - (int)(ldg(s.info + MLP_INFO_PARITY0 + NB) & 1);
   first.arrive();
   if (active == 0) return;
-  if (b == 0 && tid == 0) s.info[MLP_INFO_PARTIAL] = 1;
+  if (b == 0 && tid == 0) s.info[MLP_INFO_PARTIAL] = s.info[MLP_INFO_ROUNDS] + 1;
   if (ct == 0) reset_other(s, NB, par, w0, min(w0 + kPWg, rows), rb == 0);
   if constexpr (NB != 1) {
     if (!(pf & MLP_P32_SWAP_OROPT)) {  // deltas beyond 32 bits: whole rows, one wave each

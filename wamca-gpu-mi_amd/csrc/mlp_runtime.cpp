@@ -1097,7 +1097,8 @@ static int check_mask(mlp_ctx* ctx, const int32_t* slots, int32_t count, uint32_
 }
 
 static int eval_impl(mlp_ctx* ctx, const int32_t* slots, int32_t count, uint32_t nb_mask,
-                     int32_t rowmap, int32_t persistent, int skip, int* round_counter) {
+                     int32_t rowmap, int32_t persistent, int skip, int* round_counter,
+                     bool fill = false) {
   if (ctx->user_capture)
     for (int q = 0; q < count; ++q)
       ctx->capture_ops.push_back({slots[q], 0, nb_mask, rowmap});
@@ -1138,6 +1139,7 @@ static int eval_impl(mlp_ctx* ctx, const int32_t* slots, int32_t count, uint32_t
       if (odc && maxn >= 512 && (nb_mask & 0x1cu)) tile = MLP_TILE_8x256;
     }
     if (odc && tile == MLP_TILE_16x1024) tile = MLP_TILE_8x512;
+    if (fill) tile = tile == MLP_TILE_4x256 || tile == MLP_TILE_4x512 ? MLP_TILE_4x256 : MLP_TILE_8x512;
     int TR, TC;
     mlp_tile_shape(tile | (odc ? MLP_TILE_ODC : 0), &TR, &TC);
     // with swap in the launch, tiles of eight or more rows evaluate 2-opt
@@ -1205,6 +1207,11 @@ static int eval_impl(mlp_ctx* ctx, const int32_t* slots, int32_t count, uint32_t
     a.grid = total;
     if (two) a.rowmap |= MLP_TILE_TWO;
     if (odc) a.rowmap |= MLP_TILE_ODC;
+    // a replay of a caller's graph may meet another instance in a slot
+    bool small = !ctx->user_capture;
+    for (int q = 0; q < count && small; ++q) small = ctx->slots[slots[q]].dev.small != 0;
+    if (small) a.rowmap |= MLP_TILE_SMALL;
+    if (fill) a.rowmap |= MLP_TILE_FILL;
     // tiles of a tour run mostly one after another: filtered diagonal folds
     if (total > 2 * ctx->cu_count * kTileWgPerCu[tile]) a.skip |= 2;
     if (ctx->user_capture)  // replays fold into the same buffers: clear them in the graph
@@ -2062,8 +2069,8 @@ int run_chunk(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max
   if (!ctx->dvnd_graph || ctx->user_capture)
     return enqueue_rounds(ctx, slots, count, rowmap, max_rounds, plan);
   int tile = ctx->tile_override;  // (the per-neighborhood shapes follow from the slots)
-  // the captured launches embed the slot table address, every slot's id and
-  // size (segment tables, merge capacities) and the settings
+  // the captured launches embed the slot table address, every slot's id, size
+  // (segment tables, merge capacities) and distance form, and the settings
   const int32_t hdr[12] = {rowmap, max_rounds, plan.rounds, ctx->dvnd_persistent, tile, count,
                            ctx->dvnd_nbs, ctx->merge_force_global ? 1 : 0, ctx->dvnd_fused,
                            plan.from, plan.to, plan.keep};
@@ -2071,7 +2078,8 @@ int run_chunk(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap, int max
   key.append((const char*)&ctx->d_table, sizeof ctx->d_table);
   key.append((const char*)slots, 4 * (size_t)count);
   for (int q = 0; q < count; ++q) {
-    const int32_t Nn[2] = {ctx->slots[slots[q]].N, ctx->slots[slots[q]].nbs};
+    const Slot& s = ctx->slots[slots[q]];
+    const int32_t Nn[3] = {s.N, s.nbs, s.dev.small};
     key.append((const char*)Nn, sizeof Nn);
   }
   mlp_ctx::ChunkGraph* c = &ctx->graphs[gc][0];
@@ -2241,7 +2249,7 @@ int complete_rows(mlp_ctx* ctx, const int32_t* slots, int count, int rowmap) {
   const int nbs = std::min(ctx->dvnd_nbs, MLP_NB_COUNT);
   const bool timing = ctx->timing;
   ctx->timing = false;
-  const int st = eval_impl(ctx, slots, count, (1u << nbs) - 1u, rowmap, 0, 1 | 8, nullptr);
+  const int st = eval_impl(ctx, slots, count, (1u << nbs) - 1u, rowmap, 0, 1, nullptr, true);
   ctx->timing = timing;
   for (int q = 0; q < count; ++q)
     for (int nb = 0; nb < nbs; ++nb) ctx->slots[slots[q]].merged[nb] = true;
@@ -2682,6 +2690,7 @@ int mlp_eval_static(mlp_ctx* ctx, int32_t inst, const int32_t* tour, uint32_t nb
     }
     if (two) tile |= MLP_TILE_TWO;
     if (odc) tile |= MLP_TILE_ODC;
+    if (d.small && !ctx->user_capture) tile |= MLP_TILE_SMALL;
     if ((nb_mask & 2u) && !two && rows_of(1, 0, N) > 0 && N >= 4) {
       const int ncols = (N - 3 + TC - 1) / TC;
       segs.s[nsegs++] = SweepSeg{0, 1, 2, total, ncols, 0x1f};
