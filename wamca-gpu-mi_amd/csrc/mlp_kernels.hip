@@ -160,6 +160,9 @@ struct FullDist {
 // n = 100 17.6 -> 18.5 us, 256 tours n = 1000 in [0, 2000]^2, or-opt-1 alone
 // 257 -> 265), or its slot's (fused rounds).
 constexpr int kFullDist = 0, kSmallDist = 1, kSlotDist = 2;
+// The short form starts behind a scheduling barrier: mixed with the address
+// arithmetic before it, 200 tours n = 784 take 442 us instead of 439, 64 tours
+// n = 400 63.0 instead of 62.5.
 template <int DIST>
 __device__ __forceinline__ auto tile_dist(int round, float dr) {
   if constexpr (DIST == kSmallDist) return fast_dist(round);
@@ -3378,6 +3381,7 @@ __device__ __forceinline__ void sweep_fixed(const SlotDev& s, int rb, int ct, in
   // swap alone covers j >= i + 2 only: a tile left of that diagonal is empty
   if (mask == 1 && q1 <= b0 + 3) return;
   const auto dist = tile_dist<DIST>(s.round, dr);
+  if constexpr (DIST == kSmallDist) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int it = 0; it < FI; ++it) {
     const int c = cfill + tid + it * kBlock;
@@ -3576,6 +3580,7 @@ __device__ __forceinline__ void sweep_2opt(const SlotDev& s, int rb, int ct, int
   if (ct == 0 && !FILL)
     reset_other(s, 1, par, rb * MLP_2OPT_ROWS, min(rb * MLP_2OPT_ROWS + MLP_2OPT_ROWS, rows), rb == 0);
   const auto dist = tile_dist<DIST>(s.round, dr);
+  if constexpr (DIST == kSmallDist) __builtin_amdgcn_sched_barrier(0);
   if constexpr (FLAT) {
     if (net > 0) {
 #pragma unroll
