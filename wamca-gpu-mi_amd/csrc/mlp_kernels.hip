@@ -10,9 +10,12 @@
 //   k_sweep         the same rows over LDS-tiled distance blocks: fixed-row
 //                   tiles (swap, or-opt-1/2/3, optionally 2-opt) folding into
 //                   either row map, 2-opt diagonal tiles
-//   k_merge_apply   stable sort of the improving rows, greedy non-overlapping
-//                   subset, parallel application, ADS rebuild, one workgroup
-//                   per slot with its working arrays in LDS
+//   k_psweep        (mlp_prune.h) a DVND round's rows that improve, blocks of
+//                   moves that cannot improve left out
+//   k_merge_apply   greedy non-overlapping subset of the improving rows in
+//                   (cost, row) order, selected or after a sort, parallel
+//                   application, ADS rebuild, one workgroup per slot with its
+//                   working arrays in LDS
 //                   [MLKernel::mergeGPU mlkernel.cu:254-384 + testSwap/test2Opt/
 //                   testOrOpt :73-170 + applyMove mlkswap.cu:1066, mlk2opt.cu:725,
 //                   mlkoropt.cu:886]
@@ -114,7 +117,6 @@ __device__ __forceinline__ SlotRegs slot_regs(const SlotDev* table, int id, int 
                "+s"(r.N), "+s"(r.n), "+s"(r.round), "+s"(r.maxd), "+s"(r.rowcap));
   return r;
 }
-__device__ __forceinline__ gptr<int64_t> slot_rows(const SlotRegs& s, int) { return s.rows; }
 __device__ __forceinline__ gptr<int64_t> kept_cost(const SlotRegs& s, int) { return s.kcost; }
 __device__ __forceinline__ gptr<int32_t> kept_ij(const SlotRegs& s, int) { return s.kij; }
 
@@ -449,13 +451,13 @@ __device__ __forceinline__ int list_at(const SlotListInline& inl, const int32_t*
 }
 
 // ---------------------------------------------------------------------------
-// ADS prefix build for one slot by one workgroup (tour may live in LDS).
-// Segments of kBlock * kPrepPer positions: thread t owns kPrepPer
-// consecutive positions, gathers their coordinates (all loads issued before
-// the first wait), forms w, T and Q prefixes in registers, and one
-// block-wide exclusive scan of the per-thread totals places them.
+// ADS prefix build for one slot by one workgroup (prep_tour; tour may live in
+// LDS).  Segments of TB x PER positions: thread t owns PER consecutive
+// positions, gathers their coordinates (all loads issued before the first
+// wait), forms w, T and Q prefixes in registers, and scans of the waves' and
+// the workgroup's totals place them.
 // ---------------------------------------------------------------------------
-constexpr int kPrepPer = 8;
+constexpr int kPrepPer = 8;  // positions a thread of k_dvnd_start summarises
 
 // 64-bit value of lane (lane - shift within a row of 16, or a row
 // broadcast) through DPP on both halves; lanes without a source get 0.
@@ -2038,7 +2040,7 @@ __global__ __launch_bounds__(TB) void k_merge_apply(const SlotDev* __restrict__ 
 //   k_mg_compact  the improving rows as (cost, row) keys (gathered per
 //                 workgroup in LDS, then appended with one atomic), the tour
 //                 copied to told / tnew, the coordinates by client;
-//   k_mg_select   one workgroup per slot: sort, greedy, the kept moves'
+//   k_mg_select   one workgroup per slot: the greedy subset, the kept moves'
 //                 spans written into tnew, the merge's and round's counters;
 //   k_mg_rebuild  per segment of 1024 positions of the new tour: the prefixes
 //                 before it, summed from the edges, then the prefix arrays
