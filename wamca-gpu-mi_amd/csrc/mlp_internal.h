@@ -52,6 +52,11 @@ enum { MLP_P32_2OPT = 1, MLP_P32_SWAP_OROPT = 2, MLP_PK_SWAP_OROPT = 4, MLP_T24 
 struct BlkSum {
   int32_t lo, hi, wmax, wpair;
 };
+// The summaries of a slot's tour end where its info words begin (blk_of), so
+// that the table entry holds no pointer to them (one cache line less to
+// wait for in every merge and pruned evaluation: 88 served jobs 10.6 to 11.3 ms
+// with a pointer at its end, 10.5 to 10.8 without).
+#define MLP_BLK_BYTES(N) (((size_t)(((N) + MLP_BLK - 1) / MLP_BLK) * sizeof(BlkSum) + 255) & ~(size_t)255)
 
 // maxd - 1 bounds the real distances (mlp_runtime.cpp check_instance): up to
 // this maxd every dx^2 + dy^2 <= 1448^2 < 2^21.
@@ -87,7 +92,6 @@ struct SlotDev {
   int32_t* kept_ij[MLP_NB_MAX];   // (i, j, row) triplets
   int32_t nbs;                    // neighborhoods with buffers (ids 0 .. nbs-1)
   void* mscratch;  // the merge's working arrays when they exceed LDS (layout of its LDS)
-  BlkSum* blk;     // [ceil(N / MLP_BLK)]
 };
 
 // Z[p] = 2 Q[p] - (2p + 1) T[p] turns the 2-opt internal sum into

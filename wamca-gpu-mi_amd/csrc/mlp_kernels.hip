@@ -90,7 +90,6 @@ struct SlotRegs {
   gptr<const int32_t> xs, ys;
   gptr<int32_t> tour, xy, w, t32, q32, g32, h32;
   gptr<int64_t> t64, q64;
-  gptr<BlkSum> blk;
   gptr<int64_t> info, rows, kcost;  // rows and kept moves of one neighborhood
   gptr<int32_t> kij;
 };
@@ -104,7 +103,7 @@ __device__ __forceinline__ SlotRegs slot_regs(const SlotDev* table, int id, int 
   r.rowcap = p->rowcap;
 #define MLP_FIELD(F) r.F = (decltype(r.F))p->F
   MLP_FIELD(xs); MLP_FIELD(ys); MLP_FIELD(tour); MLP_FIELD(xy); MLP_FIELD(w); MLP_FIELD(t32);
-  MLP_FIELD(q32); MLP_FIELD(g32); MLP_FIELD(h32); MLP_FIELD(t64); MLP_FIELD(q64); MLP_FIELD(blk);
+  MLP_FIELD(q32); MLP_FIELD(g32); MLP_FIELD(h32); MLP_FIELD(t64); MLP_FIELD(q64);
   MLP_FIELD(info);
 #undef MLP_FIELD
   r.rows = (gptr<int64_t>)p->rows[nb];
@@ -113,9 +112,13 @@ __device__ __forceinline__ SlotRegs slot_regs(const SlotDev* table, int id, int 
   // all of them are there before the first use of any
   asm volatile("" : "+s"(r.xs), "+s"(r.ys), "+s"(r.tour), "+s"(r.xy), "+s"(r.w), "+s"(r.t32),
                "+s"(r.q32), "+s"(r.g32), "+s"(r.h32), "+s"(r.t64), "+s"(r.q64));
-  asm volatile("" : "+s"(r.blk), "+s"(r.info), "+s"(r.rows), "+s"(r.kcost), "+s"(r.kij),
+  asm volatile("" : "+s"(r.info), "+s"(r.rows), "+s"(r.kcost), "+s"(r.kij),
                "+s"(r.N), "+s"(r.n), "+s"(r.round), "+s"(r.maxd), "+s"(r.rowcap));
   return r;
+}
+template <typename Slot>
+__device__ __forceinline__ gptr<BlkSum> blk_of(const Slot& s) {
+  return (gptr<BlkSum>)((gptr<char>)s.info - MLP_BLK_BYTES(s.N));
 }
 __device__ __forceinline__ gptr<int64_t> kept_cost(const SlotRegs& s, int) { return s.kcost; }
 __device__ __forceinline__ gptr<int32_t> kept_ij(const SlotRegs& s, int) { return s.kij; }
@@ -588,7 +591,7 @@ __device__ __forceinline__ void put_summary(const Slot& s, int p0, const int (&x
   const int b = group_pk<G, false>(__builtin_bit_cast(int, hi));
   wm = group_max<G>(wm);
   wp = group_max<G>(wp);
-  if (threadIdx.x % G == 0 && p0 < s.N) *(gptr<int4v>)(s.blk + p0 / MLP_BLK) = int4v{a, b, wm, wp};
+  if (threadIdx.x % G == 0 && p0 < s.N) *(gptr<int4v>)(blk_of(s) + p0 / MLP_BLK) = int4v{a, b, wm, wp};
 }
 
 // PER consecutive words of a thread as the widest stores they allow.
@@ -801,7 +804,7 @@ __global__ __launch_bounds__(TB) void k_static_begin(SlotDev* table, SlotDev d) 
   s.N = d.N; s.n = d.n; s.round = d.round; s.maxd = d.maxd; s.small = d.small; s.rowcap = d.rowcap;
 #define MLP_FIELD(F) s.F = (decltype(s.F))d.F
   MLP_FIELD(xs); MLP_FIELD(ys); MLP_FIELD(tour); MLP_FIELD(xy); MLP_FIELD(w); MLP_FIELD(t32);
-  MLP_FIELD(q32); MLP_FIELD(g32); MLP_FIELD(h32); MLP_FIELD(t64); MLP_FIELD(q64); MLP_FIELD(blk);
+  MLP_FIELD(q32); MLP_FIELD(g32); MLP_FIELD(h32); MLP_FIELD(t64); MLP_FIELD(q64);
   MLP_FIELD(info);
 #undef MLP_FIELD
   s.rows = s.kcost = nullptr;

@@ -61,7 +61,7 @@ struct PruneFirst {
     rxy = ldg(s.xy + rp);
     rw = ldg(s.w + rp);
     rt = ldg(s.t32 + rp);
-    sm = *(gptr<const int4v>)(s.blk + B);
+    sm = *(gptr<const int4v>)(blk_of(s) + B);
     tp = ldg(s.t32 + max(B * MLP_BLK - 1, 0));
   }
   __device__ __forceinline__ void arrive() {
@@ -240,7 +240,7 @@ __device__ __forceinline__ void prune_wave(const SlotDev& s, int b0, int ct, int
     int4v sm = first.sm;
     int tp = first.tp;
     if (q0 > wb0) {
-      sm = *(gptr<const int4v>)(s.blk + Bc);
+      sm = *(gptr<const int4v>)(blk_of(s) + Bc);
       tp = ldg(s.t32 + max(c0 - 1, 0));
     }
     bool keep;

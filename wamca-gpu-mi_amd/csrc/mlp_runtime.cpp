@@ -105,7 +105,7 @@ size_t merge_gmem_bytes(int N) { return merge_bytes(N); }
 
 // Byte layout of one slot's device block.
 struct SlotLayout {
-  size_t tour, xy, w, t32, q32, g32, h32, t64, q64, blk, info, rows[MLP_NB_MAX], kc[MLP_NB_MAX],
+  size_t tour, xy, w, t32, q32, g32, h32, t64, q64, info, rows[MLP_NB_MAX], kc[MLP_NB_MAX],
       kij[MLP_NB_MAX], ms, total;
 };
 
@@ -126,7 +126,7 @@ SlotLayout slot_layout(int N, int nbs) {
   L.h32 = take(4 * (size_t)N);
   L.t64 = take(8 * (size_t)N);
   L.q64 = take(8 * (size_t)N);
-  L.blk = take(sizeof(BlkSum) * (size_t)((N + MLP_BLK - 1) / MLP_BLK));
+  take(MLP_BLK_BYTES(N));  // block summaries, just before the info words
   L.info = take(8 * MLP_INFO_WORDS);
   for (int nb = 0; nb < nbs; ++nb) {
     const size_t r = (size_t)row_cap(N);
@@ -812,7 +812,6 @@ int mlp_slot_create(mlp_ctx* ctx, int32_t inst, int32_t* slot) {
   d.h32 = (int32_t*)(b + L.h32);
   d.t64 = (int64_t*)(b + L.t64);
   d.q64 = (int64_t*)(b + L.q64);
-  d.blk = (BlkSum*)(b + L.blk);
   d.info = (int64_t*)(b + L.info);
   d.nbs = ctx->nbs;
   for (int nb = 0; nb < d.nbs; ++nb) {
@@ -2647,7 +2646,6 @@ int mlp_eval_static(mlp_ctx* ctx, int32_t inst, const int32_t* tour, uint32_t nb
   d.h32 = (int32_t*)(b + L.h32);
   d.t64 = (int64_t*)(b + L.t64);
   d.q64 = (int64_t*)(b + L.q64);
-  d.blk = (BlkSum*)(b + L.blk);
   d.info = (int64_t*)(b + L.info);
   d.nbs = MLP_NB_COUNT;
   RowsOut rows{};
